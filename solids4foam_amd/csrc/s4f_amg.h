@@ -201,7 +201,8 @@ __global__ __launch_bounds__(kBlock) void k_mg0_down(const DevMesh m, const Bloc
                                                      T* __restrict__ r, double omega,
                                                      const Ctl* __restrict__ ctl) {
     const int lb = logicalBlock(bm.nBlocks);
-    const int inst = bm.inst[lb];
+    const Tile tl = bm.at(lb);
+    const int inst = tl.inst;
     const Ctl* c = ctl + inst;
     if (mgSkip(c)) return;
     const int C = m.nCells;
@@ -212,13 +213,11 @@ __global__ __launch_bounds__(kBlock) void k_mg0_down(const DevMesh m, const Bloc
     const bool all = act[0] && act[1] && act[2];
     const T w = (T)omega;
     const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
-    const int s1 = bm.s1[lb];
-    const int cEnd = bm.iCell0[inst] + bm.iNCell[inst];
-    for (int s = bm.s0[lb] + wave; s < s1; s += kBlock / 64) {
+    for (int s = tl.s0 + wave; s < tl.s1; s += kBlock / 64) {
         const int P = s * kSlice + lane;
-        if (P >= cEnd) continue;
-        const int e0 = m.sliceStart[s];
-        const int width = m.sliceWidth[s];
+        if (P >= tl.cEnd) continue;
+        const int width = m.width(s);
+        const int e0 = m.entry0(s);
         if (all && width == 6) {
             mg0DownRowAll<T, 6>(m, P, e0, lane, C, b, r, w);
             continue;
@@ -270,7 +269,8 @@ __global__ __launch_bounds__(kBlock) void k_mg0_up(const DevMesh m, const BlockM
                                                    double alpha, const Ctl* __restrict__ ctl,
                                                    double* __restrict__ part) {
     const int lb = logicalBlock(bm.nBlocks);
-    const int inst = bm.inst[lb];
+    const Tile tl = bm.at(lb);
+    const int inst = tl.inst;
     const Ctl* c = ctl + inst;
     if (mgSkip(c)) return;
     const int C = m.nCells;
@@ -280,13 +280,11 @@ __global__ __launch_bounds__(kBlock) void k_mg0_up(const DevMesh m, const BlockM
     const T w = (T)omega, w1 = (T)(1.0 - omega), al = (T)alpha;
     double acc[3] = {0, 0, 0};
     const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
-    const int s1 = bm.s1[lb];
-    const int cEnd = bm.iCell0[inst] + bm.iNCell[inst];
-    for (int s = bm.s0[lb] + wave; s < s1; s += kBlock / 64) {
+    for (int s = tl.s0 + wave; s < tl.s1; s += kBlock / 64) {
         const int P = s * kSlice + lane;
-        if (P >= cEnd) continue;
-        const int e0 = m.sliceStart[s];
-        const int width = m.sliceWidth[s];
+        if (P >= tl.cEnd) continue;
+        const int width = m.width(s);
+        const int e0 = m.entry0(s);
         if (all && width == 6) {
             mg0UpRowAll<T, 6>(m, qCol, q, P, e0, lane, C, b, r0, agg, e, z, w, w1, al, acc);
             continue;
@@ -321,7 +319,7 @@ __global__ __launch_bounds__(kBlock) void k_mg0_up(const DevMesh m, const BlockM
             acc[j] += (double)zv * (double)bv;
         }
     }
-    storeBlockPartials<3>(acc, 0u, part, lb, bm.nBlocks);
+    storeBlockPartials<3, 0>(acc, part, kOffRho, lb, bm.nBlocks);
 }
 
 // Prolongation + post-smoothing on level 0 of a smoothed hierarchy (the first
@@ -339,7 +337,8 @@ __global__ __launch_bounds__(kBlock) void k_mg0_up_g(const DevMesh m, const Bloc
                                                      T* __restrict__ z, double omega, double alpha,
                                                      const Ctl* __restrict__ ctl, double* __restrict__ part) {
     const int lb = logicalBlock(bm.nBlocks);
-    const int inst = bm.inst[lb];
+    const Tile tl = bm.at(lb);
+    const int inst = tl.inst;
     const Ctl* c = ctl + inst;
     if (mgSkip(c)) return;
     const int C = m.nCells;
@@ -348,11 +347,9 @@ __global__ __launch_bounds__(kBlock) void k_mg0_up_g(const DevMesh m, const Bloc
     const T w = (T)omega, al = (T)alpha;
     double acc[3] = {0, 0, 0};
     const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
-    const int s1 = bm.s1[lb];
-    const int cEnd = bm.iCell0[inst] + bm.iNCell[inst];
-    for (int s = bm.s0[lb] + wave; s < s1; s += kBlock / 64) {
+    for (int s = tl.s0 + wave; s < tl.s1; s += kBlock / 64) {
         const int P = s * kSlice + lane;
-        if (P >= cEnd) continue;
+        if (P >= tl.cEnd) continue;
         const int e0 = gStart[s];
         const int width = gWidth[s];
         T sum[3] = {(T)0, (T)0, (T)0};
@@ -384,7 +381,7 @@ __global__ __launch_bounds__(kBlock) void k_mg0_up_g(const DevMesh m, const Bloc
             acc[j] += (double)zv * (double)bv;
         }
     }
-    storeBlockPartials<3>(acc, 0u, part, lb, bm.nBlocks);
+    storeBlockPartials<3, 0>(acc, part, kOffRho, lb, bm.nBlocks);
 }
 
 // ---------------------------------------------------------------------------
@@ -632,24 +629,6 @@ __global__ __launch_bounds__(kBlock) void k_mg_dense(const MgLevel L, const T* _
 #pragma unroll
     for (int j = 0; j < 3; ++j) acc[j] = waveReduce<false>(acc[j]);
     if (lane == 0) x[row] = row4((T)acc[0], (T)acc[1], (T)acc[2]);
-}
-
-// rho' = z.r finalize for a V-cycle-preconditioned PCG: beta = rho'/rho
-// (first iteration: no beta), rho = rho'
-__global__ __launch_bounds__(kFinBlock) void k_fin_rho(const BlockMap bm, Ctl* __restrict__ ctlAll,
-                                                       const double* __restrict__ part) {
-    const int inst = bm.finInst ? bm.finInst[blockIdx.x] : (int)blockIdx.x;
-    Ctl* ctl = ctlAll + inst;
-    if (ctl->outerDone || ctl->innerDone) return;
-    __shared__ double tot[3];
-    finReduce<3>(part, bm.nBlocks, bm.iBlk0[inst], bm.iNBlk[inst], 0u, tot);
-    if (threadIdx.x == 0) {
-        for (int j = 0; j < 3; ++j) {
-            if (!ctl->active[j]) continue;
-            ctl->beta[j] = ctl->firstInner ? 0.0 : tot[j] / ctl->rho[j];
-            ctl->rho[j] = tot[j];
-        }
-    }
 }
 
 // ---------------------------------------------------------------------------

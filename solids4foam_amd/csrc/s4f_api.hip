@@ -28,7 +28,7 @@
 #include "s4f_device.h"
 #include "s4f_internal.h"
 #include "s4f_kernels.h"
-#include "s4f_amg.h"
+#include "s4f_merged.h"
 
 namespace s4f {
 
@@ -107,13 +107,14 @@ struct s4f_ctx {
 // hipGetSymbolAddress (at context creation on that device) and only that
 // address is ever passed to kernels.
 // ---------------------------------------------------------------------------
+constexpr int kChain = 5;  // control blocks of a launch sequence (Chain)
 constexpr int kNoAllocMaxCells = 262144;  // 64^3, the largest batched-box instance
-constexpr size_t kNoAllocCtlBytes = 1024;
-constexpr size_t kNoAllocPartBytes = (size_t)8192 * kMaxPartials * sizeof(double);
+constexpr size_t kNoAllocCtlBytes = 4096;  // the launch sequence's control blocks
+constexpr size_t kNoAllocPartBytes = (size_t)8192 * kPcgPartials * sizeof(double);
 // r, p, p2, q as FP64 (FP32 sweeps need r, p, p2, q, x: 60 of these 96 bytes per cell)
 constexpr size_t kNoAllocVecBytes = (size_t)4 * 3 * kNoAllocMaxCells * sizeof(double);
 constexpr size_t kNoAllocScratchBytes = kNoAllocCtlBytes + kNoAllocPartBytes + kNoAllocVecBytes;
-static_assert(sizeof(Ctl) <= kNoAllocCtlBytes, "control block exceeds its scratch slot");
+static_assert(kChain * sizeof(Ctl) <= kNoAllocCtlBytes, "control block exceeds its scratch slot");
 
 static __device__ __align__(256) unsigned char scratch[kNoAllocScratchBytes];
 
@@ -205,6 +206,12 @@ struct HostMesh {
     std::vector<int> eIf;                 // per ELL entry: interface side, -1 (empty: no interfaces)
     std::vector<unsigned char> sliceIf;   // per slice: holds interface entries
     std::vector<double> minv0;            // whole-mesh LS inverses, kept once zones replace some
+    // slot count of every slice, 0 when they differ
+    int uniformWidth() const {
+        for (int w : sliceWidth)
+            if (w != sliceWidth[0]) return 0;
+        return sliceWidth.empty() ? 0 : sliceWidth[0];
+    }
 };
 
 struct SolveState {
@@ -301,10 +308,13 @@ struct s4f_mesh {
     DArr<double> ifN, ifDc, ifLs;
     DArr<unsigned char> sliceIf;
     // block map (single instance)
-    DArr<int> bmInst, bmS0, bmS1, iBlk0, iNBlk, iCell0, iNCell, iB0, iNB;
+    DArr<Tile> bmTile;
+    DArr<int> iBlk0, iNBlk, iNCell, iB0, iNB;
     int nBlocks = 0, slicesPerBlock = 0, maxInstNB = 0;
-    std::vector<int> tInst, tS0, tS1, tBlk0, tNBlk;  // host copy of the workgroup tiles
-    DArr<int> aInst, aS0, aS1, aBlk0, aNBlk, aFin;   // tiles of the instances still iterating (batches)
+    std::vector<Tile> tTile;          // host copy of the workgroup tiles
+    std::vector<int> tBlk0, tNBlk;
+    DArr<Tile> aTile;                 // tiles of the instances still iterating (batches)
+    DArr<int> aBlk0, aNBlk, aFin;
     bool materialSet = false;
     unsigned generation = 0;  // bumped when material data changes (serving cache key)
     unsigned tileGen = 0;     // bumped when the workgroup-tile rule changes
@@ -327,6 +337,8 @@ DevMesh s4f_mesh::dm() const {
     m.nSlices = h.nSlices;
     m.slicesPerBlock = slicesPerBlock;
     m.nBlocks = nBlocks;
+    m.uniW = h.uniformWidth();
+    m.contig = m.uniW > 0 && (size_t)h.nSlices * m.uniW * kSlice == h.col.size() ? 1 : 0;
     m.nEntries = h.col.size();
     m.sliceStart = sliceStart.p;
     m.sliceWidth = sliceWidth.p;
@@ -379,12 +391,13 @@ DevMesh s4f_mesh::dm() const {
 
 BlockMap s4f_mesh::bmap() const {
     BlockMap b{};
-    b.inst = bmInst.p;
-    b.s0 = bmS0.p;
-    b.s1 = bmS1.p;
+    b.tile = bmTile.p;
+    // (a batch of one has padding cells after its own)
+    b.spb = h.instCell0.size() == 1 && h.instNCell[0] == h.C ? slicesPerBlock : 0;
+    b.nSlices = h.nSlices;
+    b.nCells = h.C;
     b.iBlk0 = iBlk0.p;
     b.iNBlk = iNBlk.p;
-    b.iCell0 = iCell0.p;
     b.iNCell = iNCell.p;
     b.iB0 = iB0.p;
     b.iNB = iNB.p;
@@ -769,6 +782,15 @@ void uploadGeometry(s4f_mesh* M) {
     uploadTiles(M);
 }
 
+// appends the tiles of an instance: spb slices each from slice a, nS slices
+// (an empty instance keeps one idle tile, so its reductions are defined)
+void addTiles(std::vector<Tile>& tile, int inst, int a, int nS, int spb, int cEnd, int nCell) {
+    const int blk0 = (int)tile.size();
+    for (int x = a; x < a + nS; x += spb) tile.push_back(Tile{inst, x, std::min(x + spb, a + nS), cEnd, blk0, 0, nCell, 0});
+    if ((int)tile.size() == blk0) tile.push_back(Tile{inst, a, a, cEnd, blk0, 0, nCell, 0});
+    for (size_t k = blk0; k < tile.size(); ++k) tile[k].nBlk = (int)tile.size() - blk0;
+}
+
 // Workgroups: each instance is cut into workgroup tiles by a rule that
 // depends on that instance alone (tileSlices: at least one slice per wave,
 // at most its tile cap), so its reductions -- and therefore its result -- are
@@ -777,36 +799,24 @@ void uploadTiles(s4f_mesh* M) {
     HostMesh& h = M->h;
     hipStream_t s = M->ctx->stream;
     const int nInst = (int)h.instCell0.size();
-    std::vector<int> inst, s0, s1, blk0(nInst), nblk(nInst);
+    std::vector<Tile> tile;
+    std::vector<int> blk0(nInst), nblk(nInst);
     int spb = 0;
     for (int i = 0; i < nInst; ++i) {
         const int a = h.instCell0[i] / kSlice;
         const int nS = (h.instNCell[i] + kSlice - 1) / kSlice;
-        const int e = a + nS;
         const int spbI = tileSlices(h, i, nS);
         spb = std::max(spb, spbI);
-        blk0[i] = (int)inst.size();
-        for (int x = a; x < e; x += spbI) {
-            inst.push_back(i);
-            s0.push_back(x);
-            s1.push_back(std::min(x + spbI, e));
-        }
-        if ((int)inst.size() == blk0[i]) {  // empty instance: one idle workgroup keeps the reductions defined
-            inst.push_back(i);
-            s0.push_back(a);
-            s1.push_back(a);
-        }
-        nblk[i] = (int)inst.size() - blk0[i];
+        blk0[i] = (int)tile.size();
+        addTiles(tile, i, a, nS, spbI, h.instCell0[i] + h.instNCell[i], h.instNCell[i]);
+        nblk[i] = (int)tile.size() - blk0[i];
     }
     M->slicesPerBlock = spb;
-    M->nBlocks = (int)inst.size();
-    M->tInst = inst; M->tS0 = s0; M->tS1 = s1; M->tBlk0 = blk0; M->tNBlk = nblk;
-    M->bmInst.upload(inst, s);
-    M->bmS0.upload(s0, s);
-    M->bmS1.upload(s1, s);
+    M->nBlocks = (int)tile.size();
+    M->tTile = tile; M->tBlk0 = blk0; M->tNBlk = nblk;
+    M->bmTile.upload(tile, s);
     M->iBlk0.upload(blk0, s);
     M->iNBlk.upload(nblk, s);
-    M->iCell0.upload(h.instCell0, s);
     M->iNCell.upload(h.instNCell, s);
     M->iB0.upload(h.instB0, s);
     M->iNB.upload(h.instNB, s);
@@ -905,27 +915,87 @@ void allocState(s4f_mesh* M) {
     st.G.alloc(9 * (size_t)C);
     st.Db.alloc(3 * (size_t)B); st.g.alloc(3 * (size_t)B); st.snb.alloc(3 * (size_t)B);
     st.Gb.alloc(9 * (size_t)B); st.sigb.alloc(6 * (size_t)B);
-    st.ctl.alloc(nInst);
+    st.ctl.alloc((size_t)kChain * nInst);
     st.part.alloc((size_t)M->nBlocks * kMaxPartials);
     st.histCap = nInst == 1 ? kHistCap : 4096;
     st.hist.alloc(3 * (size_t)st.histCap * nInst);
 }
 
-// `n` inner PCG iterations: fused direction update + SpMV, alpha, solution /
-// residual update, convergence + beta.  v.p / v.p2 swap roles every iteration.
-template <typename T>
-void launchPcgChunk(const DevMesh& dm, const BlockMap& bm, int nInst, PcgVecs<T>& v, Ctl* ctl, double* part, int n,
-                    hipStream_t s) {
-    for (int i = 0; i < n; ++i) {
-        hipLaunchKernelGGL((k_spmvp<T, false>), dim3(bm.nBlocks), dim3(kBlock), 0, s, dm, bm, (const T*)v.r, (const T*)v.p,
-                           v.p2, v.q, ctl, part, 1, (const T*)nullptr);
-        hipLaunchKernelGGL(k_fin_spmv, dim3(nInst), dim3(kFinBlock), 0, s, bm, ctl, (const double*)part);
-        hipLaunchKernelGGL((k_update<T>), dim3(bm.nBlocks), dim3(kBlock), 0, s, dm, bm, v.x, (const T*)v.p2, v.r,
-                           (const T*)v.q, (const Ctl*)ctl, part);
-        hipLaunchKernelGGL(k_fin_update, dim3(nInst), dim3(kFinBlock), 0, s, bm, ctl, (const double*)part);
-        std::swap(v.p, v.p2);
+// Control blocks of a launch sequence (kChain arrays, one after the other) and
+// whether its kernels resolve the scalars themselves (merged: each kernel
+// reads its predecessor's array and writes its own) or finalize kernels do, in
+// place in x.  x holds the state between sequences, the one the host reads.
+struct Chain {
+    Ctl *x = nullptr, *y = nullptr, *z = nullptr, *w = nullptr, *v = nullptr;
+    bool merged = false;
+    double* hist = nullptr;
+    Chain() = default;
+    Chain(Ctl* base, size_t n, bool m, double* h) : merged(m), hist(h) {
+        x = base;
+        y = m ? x + n : x;
+        z = m ? x + 2 * n : x;
+        w = m ? x + 3 * n : x;
+        v = m ? x + 4 * n : x;
     }
+    Stage at(const Ctl* in, Ctl* out) const { return Stage{in, out, hist}; }
+};
+
+// Most tiles of an instance whose partials every workgroup reduces itself: the
+// reductions grow with the square of the tiles, a finalize launch costs its
+// 4-5 us at any size.  Measured, us per outer iteration (cube of n^3 cells,
+// tiles of 256; mixed and FP64, smoothed multigrid), finalize kernels -> merged:
+//   n=8 73 -> 58, 75 -> 59; 25 251 -> 204, 284 -> 233; 40 334 -> 268, 386 -> 322;
+//   50 518 -> 438, 649 -> 572; 64 (1,024 tiles) 675 -> 637, 849 -> 827;
+//   72 756 -> 787, 982 -> 1024; 80 862 -> 1033, 1136 -> 1301.
+// With the diagonal preconditioner the lines cross at the same size (64: mixed
+// 889 -> 838, FP64 1130 -> 1174).
+constexpr int kMergeTiles = 1024;
+// the merged kernels read every slot of a row at once, for these slot counts
+inline bool canMerge(const DevMesh& dm, int maxTiles) {
+    return maxTiles <= kMergeTiles && (dm.uniW == 6 || dm.uniW == 4);
+}
+
+template <int POINT>
+void launchFin(const BlockMap& bm, int nFin, const Chain& c, const Ctl* in, Ctl* out, const double* part, hipStream_t s) {
+    hipLaunchKernelGGL((k_fin<POINT>), dim3(nFin), dim3(kFinBlock), 0, s, bm, c.at(in, out), part);
+}
+
+// search direction + SpMV, alpha, solution / residual update of one PCG
+// iteration; `in`: the control blocks to start from, `again`: they may hold a
+// previous iteration of the same pass
+template <typename T, bool MG, bool AGAIN>
+void launchPcgBody(const DevMesh& dm, const BlockMap& bm, int nFin, const PcgVecs<T>& v, const Chain& c, const Ctl* in,
+                   double* part, hipStream_t s) {
+    const dim3 g(bm.nBlocks), b(kBlock);
+    if (c.merged) {
+        hipLaunchKernelGGL((dm.uniW == 6 ? k_spmvp_m<T, MG, AGAIN, 6> : k_spmvp_m<T, MG, AGAIN, 4>), g, b, 0, s, dm, bm, (const T*)v.r, v.p, v.p2, v.q, c.at(in, c.v),
+                           part, (const T*)v.z);
+        hipLaunchKernelGGL((k_update_m<T>), g, b, 0, s, dm, bm, v.x, (const T*)v.p, (const T*)v.p2, v.r, (const T*)v.q,
+                           c.at(c.v, c.x), part);
+        return;
+    }
+    launchFin<MG ? kPtSpmv : AGAIN ? kPtAgain : kPtInner>(bm, nFin, c, c.x, c.x, part, s);
+    hipLaunchKernelGGL((k_spmvp<T, MG>), g, b, 0, s, dm, bm, (const T*)v.r, v.p, v.p2, v.q, (const Ctl*)c.x, part, 1,
+                       (const T*)v.z);
+    launchFin<kPtUpdate>(bm, nFin, c, c.x, c.x, part, s);
+    hipLaunchKernelGGL((k_update<T>), g, b, 0, s, dm, bm, v.x, (const T*)v.p, (const T*)v.p2, v.r, (const T*)v.q,
+                       (const Ctl*)c.x, part);
+}
+
+// `n` diagonal PCG iterations from the state in c.x (a pending start already
+// resolved); the last iteration's convergence is still pending afterwards
+// (launchSettle)
+template <typename T>
+void launchPcgChunk(const DevMesh& dm, const BlockMap& bm, int nFin, const PcgVecs<T>& v, const Chain& c, double* part,
+                    int n, hipStream_t s) {
+    for (int i = 0; i < n; ++i) launchPcgBody<T, false, true>(dm, bm, nFin, v, c, c.x, part, s);
     HIP_CHECK(hipGetLastError());
+}
+
+// resolves the PCG convergence still pending in c.x (before the host reads it
+// or the tile map changes)
+void launchSettle(const BlockMap& bm, int nFin, const Chain& c, const double* part, hipStream_t s) {
+    launchFin<kPtSettle>(bm, nFin, c, c.x, c.x, part, s);
 }
 
 // ---------------------------------------------------------------------------
@@ -1725,7 +1795,7 @@ MgRun meshRun(s4f_mesh* M, bool smoothed) {
 // level-0 prolongation + post-smoothing: the aggregation form (q) or, on a
 // smoothed hierarchy, the G form
 template <typename T>
-void launchMg0Up(std::vector<std::unique_ptr<AmgDevLevel>>& d, const DevMesh& dm, const BlockMap& bm, PcgVecs<T>& v,
+void launchMg0Up(std::vector<std::unique_ptr<AmgDevLevel>>& d, const DevMesh& dm, const BlockMap& bm, const PcgVecs<T>& v,
                  double omega, double alpha, Ctl* ctl, double* part, hipStream_t s) {
     AmgDevLevel& D0 = *d[0];
     const Row4<T>* e1 = d.size() > 1 ? (const Row4<T>*)MgVec<T>::xs(*d[1]) : nullptr;
@@ -1739,10 +1809,11 @@ void launchMg0Up(std::vector<std::unique_ptr<AmgDevLevel>>& d, const DevMesh& dm
                            e1, v.z, omega, alpha, (const Ctl*)ctl, part);
 }
 
-// z = V(r): one V(1,1) cycle on the 3-RHS residual, then k_fin_rho
-template <typename T>
-void launchVcycle(const MgRun& R, const DevMesh& dm, const BlockMap& bm, PcgVecs<T>& v, Ctl* ctl, double* part,
-                  hipStream_t s) {
+// z = V(r): one V(1,1) cycle on the 3-RHS residual
+template <typename T, bool AGAIN>
+void launchVcycle(const MgRun& R, const DevMesh& dm, const BlockMap& bm, const PcgVecs<T>& v, const Chain& ch,
+                  const Ctl* in, double* part, hipStream_t s) {
+    Ctl* ctl = ch.w;
     std::vector<std::unique_ptr<AmgDevLevel>>& Ad = *R.levels;
     struct {
         std::vector<std::unique_ptr<AmgDevLevel>>& d;
@@ -1752,8 +1823,14 @@ void launchVcycle(const MgRun& R, const DevMesh& dm, const BlockMap& bm, PcgVecs
     const double w = R.omega;
     AmgDevLevel& D0 = *A.d[0];
     T* r0 = MgVec<T>::r0(D0);
-    hipLaunchKernelGGL((k_mg0_down<T>), dim3(bm.nBlocks), dim3(kBlock), 0, s, dm, bm, (const T*)v.r, r0, w,
-                       (const Ctl*)ctl);
+    if (ch.merged) {
+        hipLaunchKernelGGL((dm.uniW == 6 ? k_mg0_down_m<T, AGAIN, 6> : k_mg0_down_m<T, AGAIN, 4>), dim3(bm.nBlocks), dim3(kBlock), 0, s, dm, bm, (const T*)v.r, r0, w,
+                           ch.at(in, ch.w), (const double*)part);
+    } else {
+        launchFin<AGAIN ? kPtAgain : kPtInner>(bm, R.nFin, ch, ch.x, ch.x, part, s);
+        hipLaunchKernelGGL((k_mg0_down<T>), dim3(bm.nBlocks), dim3(kBlock), 0, s, dm, bm, (const T*)v.r, r0, w,
+                           (const Ctl*)ch.x);
+    }
     if (nl > 1) {
         // down: restrict the finer level's residual (with the coarse
         // pre-smoothing), then the coarse residual
@@ -1796,27 +1873,19 @@ void launchVcycle(const MgRun& R, const DevMesh& dm, const BlockMap& bm, PcgVecs
         }
     }
     launchMg0Up<T>(A.d, dm, bm, v, w, A.alpha, ctl, part, s);
-    hipLaunchKernelGGL(k_fin_rho, dim3(R.nFin), dim3(kFinBlock), 0, s, bm, ctl, (const double*)part);
     HIP_CHECK(hipGetLastError());
 }
 
-// PCG iterations with the V-cycle: spmv(p = z + beta p), alpha, update,
-// convergence, z = V(r), beta
-template <typename T>
-void launchPcgChunkMg(const MgRun& R, const DevMesh& dm, const BlockMap& bm, PcgVecs<T>& v, Ctl* ctl, double* part,
-                      int n, hipStream_t s) {
-    for (int i = 0; i < n; ++i) {
-        hipLaunchKernelGGL((k_spmvp<T, true>), dim3(bm.nBlocks), dim3(kBlock), 0, s, dm, bm, (const T*)v.r, (const T*)v.p,
-                           v.p2, v.q, ctl, part, 1, (const T*)v.z);
-        const dim3 nI(R.nFin);
-        hipLaunchKernelGGL(k_fin_spmv, nI, dim3(kFinBlock), 0, s, bm, ctl, (const double*)part);
-        hipLaunchKernelGGL((k_update<T>), dim3(bm.nBlocks), dim3(kBlock), 0, s, dm, bm, v.x, (const T*)v.p2, v.r,
-                           (const T*)v.q, (const Ctl*)ctl, part);
-        hipLaunchKernelGGL(k_fin_update, nI, dim3(kFinBlock), 0, s, bm, ctl, (const double*)part);
-        launchVcycle<T>(R, dm, bm, v, ctl, part, s);
-        std::swap(v.p, v.p2);
+// one PCG iteration: (V-cycle,) search direction, product, update
+template <typename T, bool AGAIN>
+void launchInner(bool mg, const MgRun& R, const DevMesh& dm, const BlockMap& bm, const PcgVecs<T>& v, const Chain& c,
+                 const Ctl* in, double* part, hipStream_t s) {
+    if (mg) {
+        launchVcycle<T, AGAIN>(R, dm, bm, v, c, in, part, s);
+        launchPcgBody<T, true, AGAIN>(dm, bm, R.nFin, v, c, c.w, part, s);
+    } else {
+        launchPcgBody<T, false, AGAIN>(dm, bm, R.nFin, v, c, in, part, s);
     }
-    HIP_CHECK(hipGetLastError());
 }
 
 // device copies of the (effective) diagonal and its inverse, FP64 and FP32
@@ -1952,19 +2021,19 @@ GradBufs meshGradBufs(s4f_mesh* M) {
 }
 
 // boundary values, cell gradients, boundary gradients and stress (modes as
-// k_grad); nInst instances (bm.finInst, or 0..nInst-1), at most maxNB
-// boundary faces each
+// k_grad) as separate launches reading `ctl`; nInst instances (bm.finInst, or
+// 0..nInst-1), at most maxNB boundary faces each
 template <typename T>
 void launchGradStep(const DevMesh& dm, const BlockMap& bm, int nInst, int maxNB, const GradBufs& f, const T* x,
-                    const double* Dold, Ctl* ctl, double* part, int mode, hipStream_t s) {
+                    const double* Dold, const Ctl* ctl, double* part, int mode, hipStream_t s) {
     const dim3 fg(std::max(1, std::min(1024, (maxNB + kBlock - 1) / kBlock)), std::max(1, nInst));
     if (mode == 0 && f.aAlpha)
         hipLaunchKernelGGL((k_aitken<T>), dim3(bm.nBlocks), dim3(kBlock), 0, s, dm, bm, f.D0, x, f.D1, f.aAlpha,
-                           f.aRes, (const Ctl*)ctl);
+                           f.aRes, ctl);
     if (mode != 2)
         hipLaunchKernelGGL((k_grad_bnd_pre<T>), fg, dim3(kBlock), 0, s, dm, bm, (const double*)f.D0, x,
-                           (const double*)f.D1, (const double*)f.G, f.Db, (const double*)f.g, f.snb,
-                           (const Ctl*)ctl, f.aAlphaB, f.aResB, mode);
+                           (const double*)f.D1, (const double*)f.G, f.Db, (const double*)f.g, f.snb, ctl, f.aAlphaB,
+                           f.aResB, mode);
     // sub-meshes: the interface displacement before the gradient, the
     // sub-meshes' interface stress after it (a mode-2 gradient uses the
     // interface state as it is)
@@ -1972,14 +2041,67 @@ void launchGradStep(const DevMesh& dm, const BlockMap& bm, int nInst, int maxNB,
     const dim3 ig(std::max(1, std::min(1024, (dm.nIf + kBlock - 1) / kBlock)));
     if (sub)
         hipLaunchKernelGGL((k_iface_pre<T>), ig, dim3(kBlock), 0, s, dm, (const double*)f.D0, x, (const double*)f.D1,
-                           f.DI, (const double*)f.sigI, (const Ctl*)ctl, mode);
+                           f.DI, (const double*)f.sigI, ctl, mode);
     hipLaunchKernelGGL((k_grad<T>), dim3(bm.nBlocks), dim3(kBlock), 0, s, dm, bm, f.D0, x, f.D1, f.G,
                        (const double*)f.Db, (const double*)f.DI, Dold, ctl, part, mode);
     if (sub)
         hipLaunchKernelGGL(k_iface_post, ig, dim3(kBlock), 0, s, dm, (const double*)f.D0, (const double*)f.D1,
-                           (const double*)f.G, (const double*)f.DI, f.sigI, (const Ctl*)ctl, mode);
+                           (const double*)f.G, (const double*)f.DI, f.sigI, ctl, mode);
     hipLaunchKernelGGL(k_grad_bnd_post, fg, dim3(kBlock), 0, s, dm, bm, (const double*)f.G, (const double*)f.snb,
-                       f.Gb, f.sigb, f.g, (const Ctl*)ctl, mode);
+                       f.Gb, f.sigb, f.g, ctl, mode);
+}
+
+// the merged residual for a launch's slot count and moduli
+template <typename T>
+auto residualMerged(const DevMesh& dm, const BlockMap& bm) {
+    if (dm.uniW == 6) return dm.mu ? k_residual_m<T, 6, true> : k_residual_m<T, 6, false>;
+    return dm.mu ? k_residual_m<T, 4, true> : k_residual_m<T, 4, false>;
+}
+
+// The outer step of the momentum loop for the instances whose PCG has
+// finished: gradient step, convergence test, residual (the others skip it).
+template <typename T>
+void launchOuter(const DevMesh& dm, const BlockMap& bm, int nFin, int maxNB, const GradBufs& f, const PcgVecs<T>& v,
+                 const double* Dold, const Chain& c, double* part, hipStream_t s) {
+    if (c.merged && !f.aAlpha && dm.nIf == 0) {
+        hipLaunchKernelGGL((dm.uniW == 6 ? k_grad_m<T, 6> : k_grad_m<T, 4>), dim3(bm.nBlocks), dim3(kBlock), 0, s, dm,
+                           bm, f.D0, (const T*)v.x, f.D1, f.G, f.Db, Dold, c.at(c.x, c.y), part,
+                           BndBufs{f.g, f.snb, f.Gb, f.sigb});
+    } else {
+        launchFin<kPtGrad>(bm, nFin, c, c.x, c.y, part, s);
+        launchGradStep<T>(dm, bm, nFin, maxNB, f, (const T*)v.x, Dold, c.y, part, 0, s);
+    }
+    if (c.merged) {
+        hipLaunchKernelGGL(residualMerged<T>(dm, bm), dim3(bm.nBlocks), dim3(kBlock), 0, s, dm, bm, (const double*)f.D0,
+                           (const double*)f.D1, (const double*)f.G, (const double*)f.sigb, v.r, c.at(c.y, c.z), part);
+    } else {
+        launchFin<kPtRes>(bm, nFin, c, c.x, c.x, part, s);
+        hipLaunchKernelGGL((k_residual<T>), dim3(bm.nBlocks), dim3(kBlock), 0, s, dm, bm, (const double*)f.D0,
+                           (const double*)f.D1, (const double*)f.G, (const double*)f.sigb, v.r, (const Ctl*)c.x, part);
+    }
+}
+
+// One pass of the momentum loop's launch sequence: the outer step of every
+// instance that is ready for it, then `inner` PCG iterations of every instance
+// that is not done with its PCG.
+template <typename T>
+void launchPass(bool mg, const MgRun& R, const DevMesh& dm, const BlockMap& bm, int maxNB, const GradBufs& f,
+                const PcgVecs<T>& v, const double* Dold, const Chain& c, double* part, int inner, hipStream_t s) {
+    launchOuter<T>(dm, bm, R.nFin, maxNB, f, v, Dold, c, part, s);
+    launchInner<T, false>(mg, R, dm, bm, v, c, c.z, part, s);
+    for (int i = 1; i < inner; ++i) launchInner<T, true>(mg, R, dm, bm, v, c, c.x, part, s);
+    HIP_CHECK(hipGetLastError());
+}
+
+// PCG iterations per pass.  A pass launches the outer step's kernels also for
+// an instance still in its PCG (they exit at once), and PCG iterations also
+// for one that has just finished; with `used` iterations per outer one the
+// empty launches are fewest near sqrt(ratio used), ratio the outer step's
+// launches over an iteration's times two.  One V-cycle iteration has more
+// launches than the outer step, a diagonal one has two.
+int innerPerPass(bool mg, int used) {
+    const double k = std::sqrt((mg ? 0.5 : 2.0) * used);
+    return k >= 12.0 ? 16 : k >= 6.0 ? 8 : k >= 3.0 ? 4 : k >= 1.5 ? 2 : 1;
 }
 
 // An instantiated HIP graph of a captured launch sequence.
@@ -2033,7 +2155,6 @@ struct InstanceIO {
 struct Fallback {
     bool stalled = false;            // the FP32 run stopped for the fallback
     std::vector<char> live;          // instances still iterating at the switch
-    std::vector<long long> instPcg;  // 3-RHS PCG sweeps so far, per instance
 };
 
 // Default window of mixed precision's stall test: outer iterations within
@@ -2078,8 +2199,10 @@ void solveT(s4f_mesh* M, const s4f_solve_opts& o, std::vector<InstanceIO>& io, F
     const DevMesh dm = M->dm();
     const BlockMap bmFull = M->bmap();
     BlockMap bm = bmFull;  // narrowed to the iterating instances as a batch's instances finish
-    int nFin = nInst;
     MgRun mgRun = meshRun(M, mgSmoothed);
+    // mixed precision's stall test runs on the device (innerEnd)
+    const int stallWindow = !std::is_same<T, float>::value || !fb ? 0
+                            : o.mixedStallWindow == 0 ? kMixedStallWindow : std::max(0, o.mixedStallWindow);
     // initial and old-time fields (a resumed run keeps the device state)
     std::vector<double> D0(resume ? 0 : 3 * (size_t)C, 0.0);
     bool warm = false;
@@ -2112,13 +2235,16 @@ void solveT(s4f_mesh* M, const s4f_solve_opts& o, std::vector<InstanceIO>& io, F
             c0[i].warm = ((o.warmStart && io[i].D_inout) || transient) ? 1 : 0;  // a time step continues
             c0[i].sigma0 = c0[i].warm ? 0 : 1;  // a cold start's stress field is zero until the first update
             c0[i].pcMode = mg ? 1 : 0;
+            c0[i].pending = kPendStart;
+            c0[i].stallWindow = stallWindow;
+            c0[i].bestRes = HUGE_VAL;
             c0[i].solveMask = M->h.instMask.empty() ? 7 : M->h.instMask[i];
         }
         HIP_CHECK(hipMemcpyAsync(st.ctl.p, c0.data(), nInst * sizeof(Ctl), hipMemcpyHostToDevice, s));
         HIP_CHECK(hipMemsetAsync(st.hist.p, 0, st.hist.bytes(), s));
     }
-    Ctl* hctl = nullptr;
-    HIP_CHECK(hipHostMalloc((void**)&hctl, nInst * sizeof(Ctl), hipHostMallocDefault));
+    Ctl* hctl = nullptr;  // two host copies of the control blocks: one being read, one in flight
+    HIP_CHECK(hipHostMalloc((void**)&hctl, 2 * nInst * sizeof(Ctl), hipHostMallocDefault));
     std::unique_ptr<Ctl, void (*)(Ctl*)> hctlGuard(hctl, [](Ctl* p) { (void)hipHostFree(p); });
     const double* Dold = warm ? st.Dold.p : nullptr;
     if (!resume) HIP_CHECK(hipEventRecord(ctx->ev0, s));  // a resumed run's time counts from the FP32 start
@@ -2131,174 +2257,164 @@ void solveT(s4f_mesh* M, const s4f_solve_opts& o, std::vector<InstanceIO>& io, F
     }
     if (!resume) {
         launchGradStep<T>(dm, bm, nInst, M->maxInstNB, gbuf, nullptr, Dold, st.ctl.p, st.part.p, 1, s);
-        hipLaunchKernelGGL(k_fin_grad, dim3(nInst), dim3(kFinBlock), 0, s, bm, st.ctl.p, (const double*)st.part.p,
-                           st.hist.p, 1);
+        hipLaunchKernelGGL(k_fin_init, dim3(nInst), dim3(kFinBlock), 0, s, bm, st.ctl.p, (const double*)st.part.p);
+        HIP_CHECK(hipGetLastError());
+    } else {  // the FP32 run's last PCG solution in FP64; its instances wait at the end of their PCG
+        hipLaunchKernelGGL(k_widen, dim3(gridRows(3 * C)), dim3(kBlock), 0, s, (const float*)st.x32.p, (double*)v.x,
+                           3 * (size_t)C);
+        hipLaunchKernelGGL(k_ctl_hold, dim3(1), dim3(kBlock), 0, s, st.ctl.p, nInst, 0);
         HIP_CHECK(hipGetLastError());
     }
+    auto maxTiles = [&](const std::vector<int>& live) {
+        int t = 0;
+        for (int i : live) t = std::max(t, M->tNBlk[i]);
+        return t;
+    };
+    std::vector<int> all(nInst);
+    for (int i = 0; i < nInst; ++i) all[i] = i;
+    Chain chain(st.ctl.p, nInst, canMerge(dm, maxTiles(all)), st.hist.p);
     // Batches: when instances finish, launch only the tiles of those still
     // iterating.  Each instance keeps its own tiles (and the order of its
     // partials), so its result does not change.
     auto narrow = [&](const std::vector<int>& live) {
-        std::vector<int> inst, s0, s1, blk0(nInst, 0), nblk(nInst, 0);
+        std::vector<Tile> tile;
+        std::vector<int> blk0(nInst, 0), nblk(nInst, 0);
         for (int i : live) {
-            blk0[i] = (int)inst.size();
+            blk0[i] = (int)tile.size();
+            nblk[i] = M->tNBlk[i];
             for (int b = M->tBlk0[i]; b < M->tBlk0[i] + M->tNBlk[i]; ++b) {
-                inst.push_back(M->tInst[b]);
-                s0.push_back(M->tS0[b]);
-                s1.push_back(M->tS1[b]);
+                tile.push_back(M->tTile[b]);
+                tile.back().blk0 = blk0[i];
             }
-            nblk[i] = (int)inst.size() - blk0[i];
         }
-        M->aInst.upload(inst, s); M->aS0.upload(s0, s); M->aS1.upload(s1, s);
+        M->aTile.upload(tile, s);
         M->aBlk0.upload(blk0, s); M->aNBlk.upload(nblk, s); M->aFin.upload(live, s);
         bm = bmFull;
-        bm.inst = M->aInst.p; bm.s0 = M->aS0.p; bm.s1 = M->aS1.p; bm.iBlk0 = M->aBlk0.p; bm.iNBlk = M->aNBlk.p;
+        bm.tile = M->aTile.p; bm.iBlk0 = M->aBlk0.p; bm.iNBlk = M->aNBlk.p;
         bm.finInst = M->aFin.p;
-        bm.nBlocks = (int)inst.size();
-        nFin = (int)live.size();
-        mgRun.nFin = nFin;
+        bm.nBlocks = (int)tile.size();
+        mgRun.nFin = (int)live.size();
+        chain = Chain(st.ctl.p, nInst, canMerge(dm, maxTiles(live)), st.hist.p);
     };
-    // launch sequences: the explicit terms of an outer iteration (after the
-    // previous one's gradient), and PCG iterations.  After the first outer
-    // iteration (which allocates every buffer) they are captured into HIP
-    // graphs and replayed; PCG iterations go in pairs so the two search-
-    // direction buffers are where the captured launches expect them.
-    auto launchGradResidual = [&](hipStream_t q) {
-        launchGradStep<T>(dm, bm, nFin, M->maxInstNB, gbuf, (const T*)v.x, Dold, st.ctl.p, st.part.p, 0, q);
-        hipLaunchKernelGGL(k_fin_grad, dim3(nFin), dim3(kFinBlock), 0, q, bm, st.ctl.p, (const double*)st.part.p,
-                           st.hist.p, 0);
-    };
-    auto launchResidual = [&](hipStream_t q) {
-        hipLaunchKernelGGL((k_residual<T>), dim3(bm.nBlocks), dim3(kBlock), 0, q, dm, bm, (const double*)st.D0.p,
-                           (const double*)st.D1.p, st.G.p, st.sigb.p, v.r, st.ctl.p, st.part.p);
-        hipLaunchKernelGGL(k_fin_residual, dim3(nFin), dim3(kFinBlock), 0, q, bm, st.ctl.p, (const double*)st.part.p);
-        if (mg) launchVcycle<T>(mgRun, dm, bm, v, st.ctl.p, st.part.p, q);  // z0 = V(r0), rho0
-    };
-    auto launchPcg = [&](int n, hipStream_t q) {
-        if (mg) launchPcgChunkMg<T>(mgRun, dm, bm, v, st.ctl.p, st.part.p, n, q);
-        else launchPcgChunk<T>(dm, bm, nFin, v, st.ctl.p, st.part.p, n, q);
-    };
+    // A pass advances every instance from where it stands, so the host launches
+    // passes without knowing where that is and looks at the control blocks of
+    // an earlier burst while the next one runs.  After the first pass (which
+    // allocates every buffer) passes are replayed from HIP graphs, one per
+    // number of PCG iterations in a pass.
     bool graphs = o.eagerLaunch == 0;
-    GraphExec gOuter, gPair;
-    bool captured = false;
-    int chunk = 4;
-    std::vector<long long> instPcg(nInst, 0);
-    if (resume) {
-        // the FP32 run's last PCG solution in FP64, then the outer iteration it stopped before
-        instPcg = fb->instPcg;
-        hipLaunchKernelGGL(k_widen, dim3(gridRows(3 * C)), dim3(kBlock), 0, s, (const float*)st.x32.p, (double*)v.x,
-                           3 * (size_t)C);
-        launchGradResidual(s);
+    std::map<int, GraphExec> graph;
+    int inner = mg ? 1 : 4;
+    long long passes = 0;
+    auto pass = [&]() {
+        auto launch = [&](hipStream_t q) {
+            launchPass<T>(mg, mgRun, dm, bm, M->maxInstNB, gbuf, v, Dold, chain, st.part.p, inner, q);
+        };
+        if (graphs && passes > 0) {
+            GraphExec& g = graph[inner];
+            if (!g.e) {
+                try {
+                    g.capture(ctx->capture, launch);
+                } catch (const HipError&) {  // a runtime without capture: the same launches, one by one
+                    (void)hipGetLastError();
+                    graph.clear();
+                    graphs = false;
+                }
+            }
+        }
+        if (graphs && passes > 0) graph[inner].launch(s);
+        else launch(s);
+        ++passes;
+    };
+    struct Flight {  // a burst of passes and the control blocks after it
+        hipEvent_t ev = nullptr;
+        Ctl* h = nullptr;
+        ~Flight() { if (ev) (void)hipEventDestroy(ev); }
+    } flight[2];
+    for (int k = 0; k < 2; ++k) {
+        flight[k].h = hctl + (size_t)k * nInst;
+        HIP_CHECK(hipEventCreateWithFlags(&flight[k].ev, hipEventDisableTiming));
     }
-    launchResidual(s);
-    HIP_CHECK(hipGetLastError());
-    const int stallWindow = o.mixedStallWindow == 0 ? kMixedStallWindow : o.mixedStallWindow;
+    // bursts grow with the passes already made: a short solve wastes little at its end
+    auto burst = [&](Flight& f) {
+        const int n = (int)std::min<long long>(8, 1 + passes / 16);
+        for (int k = 0; k < n; ++k) pass();
+        HIP_CHECK(hipMemcpyAsync(f.h, st.ctl.p, nInst * sizeof(Ctl), hipMemcpyDeviceToHost, s));
+        HIP_CHECK(hipEventRecord(f.ev, s));
+    };
     const auto tStart = std::chrono::steady_clock::now();
     double tShown = 0.0;
-    std::vector<double> bestRes(nInst, HUGE_VAL);
-    std::vector<int> bestIt(nInst, 0);
-    for (int it = 0;; ++it) {
-        bool allDone = false;
-        int total = 0;
-        for (;;) {
-            if (captured) {
-                const int pairs = (chunk + 1) / 2;
-                for (int k = 0; k < pairs; ++k) gPair.launch(s);
-                total += 2 * pairs;
-            } else {
-                launchPcg(chunk, s);
-                total += chunk;
-            }
-            chunk = std::max(2, chunk / 4);  // top-up chunks after an under-estimate
-            HIP_CHECK(hipMemcpyAsync(hctl, st.ctl.p, nInst * sizeof(Ctl), hipMemcpyDeviceToHost, s));
-            HIP_CHECK(hipStreamSynchronize(s));
-            allDone = true;
-            bool anyInner = false;
-            for (int i = 0; i < nInst; ++i) {
-                if (!hctl[i].outerDone) allDone = false;
-                if (!hctl[i].outerDone && !hctl[i].innerDone) anyInner = true;
-            }
-            if (allDone || !anyInner) break;
-            if (total > o.pcgMaxIter + 2) break;  // maxIter deactivates every component before this
+    long long liveTiles = M->nBlocks;
+    burst(flight[0]);
+    for (int cur = 0;; cur ^= 1) {
+        burst(flight[cur ^ 1]);
+        HIP_CHECK(hipEventSynchronize(flight[cur].ev));
+        const Ctl* hc = flight[cur].h;
+        int nLive = 0, used = 1;
+        bool stalled = false;
+        for (int i = 0; i < nInst; ++i) {
+            if (hc[i].outerDone) continue;
+            ++nLive;
+            stalled |= hc[i].stalled != 0;
+            used = std::max({used, hc[i].nIter[0], hc[i].nIter[1], hc[i].nIter[2]});
         }
-        if (allDone) break;
+        if (nLive == 0) break;
         if (o.progressSeconds > 0) {  // the per-iteration log, rate-limited
             const double now = std::chrono::duration<double>(std::chrono::steady_clock::now() - tStart).count();
             if (now - tShown >= o.progressSeconds) {
                 tShown = now;
-                int live = 0, iMax = 0;
+                int iMax = 0;
                 double rMax = 0.0;
                 for (int i = 0; i < nInst; ++i) {
-                    if (hctl[i].outerDone) continue;
-                    ++live;
-                    iMax = std::max(iMax, hctl[i].iCorr);
-                    rMax = std::max(rMax, hctl[i].initResMag);
+                    if (hc[i].outerDone) continue;
+                    iMax = std::max(iMax, hc[i].iCorr);
+                    rMax = std::max(rMax, hc[i].initResMag);
                 }
                 fprintf(stderr, "[s4f] %.0f s: outer iteration %d, %d of %d instances iterating, |initRes| %.3e, "
-                        "residualvf %.3e\n", now, iMax, live, nInst, rMax, hctl[0].rvf);
+                        "residualvf %.3e\n", now, iMax, nLive, nInst, rMax, hc[0].rvf);
                 fflush(stderr);
             }
         }
-        int used = 1;
-        for (int i = 0; i < nInst; ++i)
-            if (!hctl[i].outerDone) used = std::max({used, hctl[i].nIter[0], hctl[i].nIter[1], hctl[i].nIter[2]});
-        for (int i = 0; i < nInst; ++i)
-            if (!hctl[i].outerDone) instPcg[i] += std::max({hctl[i].nIter[0], hctl[i].nIter[1], hctl[i].nIter[2]});
-        // mixed precision's stall test: an iterating instance whose |initRes|
-        // found no new minimum 1 % below the last one within the window
-        if (std::is_same<T, float>::value && fb && stallWindow > 0) {
-            bool stall = false;
-            for (int i = 0; i < nInst; ++i) {
-                if (hctl[i].outerDone || hctl[i].iCorr < 2) continue;
-                const double r = hctl[i].initResMag;
-                if (r < 0.99 * bestRes[i]) {
-                    bestRes[i] = r;
-                    bestIt[i] = it;
-                } else if (it - bestIt[i] >= stallWindow) {
-                    stall = true;
+        inner = innerPerPass(mg, used);
+        if (stalled) {
+            // every instance finishes its PCG and waits before its gradient step
+            hipLaunchKernelGGL(k_ctl_hold, dim3(1), dim3(kBlock), 0, s, st.ctl.p, nInst, 1);
+            fb->live.assign(nInst, 0);
+            for (bool waiting = false; !waiting;) {
+                pass();
+                launchSettle(bm, mgRun.nFin, chain, st.part.p, s);
+                HIP_CHECK(hipMemcpyAsync(hctl, st.ctl.p, nInst * sizeof(Ctl), hipMemcpyDeviceToHost, s));
+                HIP_CHECK(hipStreamSynchronize(s));
+                waiting = true;
+                for (int i = 0; i < nInst; ++i) {
+                    fb->live[i] = hctl[i].outerDone ? 0 : 1;
+                    if (!hctl[i].outerDone && !hctl[i].innerDone) waiting = false;
                 }
             }
-            if (stall) {
-                HIP_CHECK(hipStreamSynchronize(s));
-                fb->stalled = true;
-                fb->live.assign(nInst, 0);
-                for (int i = 0; i < nInst; ++i) fb->live[i] = hctl[i].outerDone ? 0 : 1;
-                fb->instPcg = instPcg;
-                return;
-            }
+            // an instance that finished meanwhile leaves nothing to continue when it was the last
+            fb->stalled = std::any_of(fb->live.begin(), fb->live.end(), [](char x) { return x != 0; });
+            if (fb->stalled) return;
+            break;
         }
-        // next outer iteration: launch just under the last count, then top up
-        chunk = std::max(1, used - 1);
-        if (nInst > 1) {  // instances that finished at the previous outer iteration leave the launch
+        if (nInst > 1) {
+            // finished instances leave the launch once they hold a quarter of its tiles
+            // (their workgroups exit at once; a new map costs a capture)
             std::vector<int> live;
+            long long tiles = 0;
             for (int i = 0; i < nInst; ++i)
-                if (!hctl[i].outerDone) live.push_back(i);
-            if ((int)live.size() < nFin && !live.empty()) {
-                HIP_CHECK(hipStreamSynchronize(s));  // queued kernels still read the current tile arrays
+                if (!hc[i].outerDone) {
+                    live.push_back(i);
+                    tiles += M->tNBlk[i];
+                }
+            if (4 * tiles <= 3 * liveTiles) {
+                // pending partials are laid out by the present map: resolve them, then
+                // wait: queued kernels still read the current tile arrays
+                launchSettle(bm, mgRun.nFin, chain, st.part.p, s);
+                HIP_CHECK(hipStreamSynchronize(s));
                 narrow(live);
-                captured = false;
+                liveTiles = tiles;
+                graph.clear();
             }
         }
-        if (graphs && !captured) {
-            try {
-                gOuter.capture(ctx->capture, [&](hipStream_t q) { launchGradResidual(q); launchResidual(q); });
-                gPair.capture(ctx->capture, [&](hipStream_t q) { launchPcg(2, q); });
-                captured = true;
-            } catch (const HipError&) {  // a runtime without capture: the same launches, one by one
-                gOuter.reset();
-                gPair.reset();
-                (void)hipGetLastError();
-                graphs = false;
-            }
-        }
-        if (captured) {
-            gOuter.launch(s);
-        } else {
-            launchGradResidual(s);
-            launchResidual(s);
-        }
-        HIP_CHECK(hipGetLastError());
-        if (it > o.nCorrectors + 2) break;  // the device loop ends at nCorrectors
     }
     if (h.nIf > 0)  // sub-meshes: the interface update of the point interpolation after the loop
         hipLaunchKernelGGL((k_iface_pre<T>), dim3(std::max(1, std::min(1024, (h.nIf + kBlock - 1) / kBlock))),
@@ -2349,7 +2465,7 @@ void solveT(s4f_mesh* M, const s4f_solve_opts& o, std::vector<InstanceIO>& io, F
             rep->seconds = ms * 1e-3;
             rep->mixedFallback = (resume && fb->live[i]) ? 1 : 0;
             rep->warmStarted = cf.warm;
-            rep->pcgIterations = instPcg[i];
+            rep->pcgIterations = cf.pcgTotal;
         }
         io[i].status = cf.diverged ? S4F_ERR_DIVERGED : (cf.converged ? S4F_OK : S4F_WARN_MAXITER);
     }
@@ -3036,11 +3152,12 @@ s4f_status s4f_residual(s4f_mesh* M, const double* D, const double* gradD, const
         }
         Ctl c0;
         std::memset(&c0, 0, sizeof(c0));
+        c0.pending = kPendRes;
         HIP_CHECK(hipMemcpyAsync(st.ctl.p, &c0, sizeof(Ctl), hipMemcpyHostToDevice, s));
         const DevMesh dm = M->dm();
         const BlockMap bm = M->bmap();
         hipLaunchKernelGGL((k_residual<double>), dim3(bm.nBlocks), dim3(kBlock), 0, s, dm, bm, (const double*)st.D0.p,
-                           (const double*)st.D1.p, st.G.p, st.sigb.p, v.r, st.ctl.p, st.part.p);
+                           (const double*)st.D1.p, (const double*)st.G.p, (const double*)st.sigb.p, v.r, (const Ctl*)st.ctl.p, st.part.p);
         HIP_CHECK(hipGetLastError());
         soaToAos(download(st.r64, 3 * (size_t)C, s), C, 3, R);
         return S4F_OK;
@@ -3064,8 +3181,9 @@ s4f_status s4f_spmv3(s4f_mesh* M, const double* x, double* y, int32_t precision)
             PcgVecs<float> v = pcgVecs<float>(st, C);
             std::vector<float> tf(t.begin(), t.end());
             HIP_CHECK(hipMemcpyAsync(v.p, tf.data(), tf.size() * 4, hipMemcpyHostToDevice, s));
-            hipLaunchKernelGGL((k_spmvp<float, false>), dim3(bm.nBlocks), dim3(kBlock), 0, s, dm, bm, (const float*)nullptr,
-                               (const float*)v.p, (float*)nullptr, v.q, st.ctl.p, st.part.p, 0, (const float*)nullptr);
+            hipLaunchKernelGGL((k_spmvp<float, false>), dim3(bm.nBlocks), dim3(kBlock), 0, s, dm, bm,
+                               (const float*)nullptr, v.p, (float*)nullptr, v.q, (const Ctl*)st.ctl.p,
+                               st.part.p, 0, (const float*)nullptr);
             HIP_CHECK(hipGetLastError());
             std::vector<float> yf(3 * (size_t)C);
             HIP_CHECK(hipMemcpyAsync(yf.data(), v.q, yf.size() * 4, hipMemcpyDeviceToHost, s));
@@ -3075,8 +3193,9 @@ s4f_status s4f_spmv3(s4f_mesh* M, const double* x, double* y, int32_t precision)
         } else {
             PcgVecs<double> v = pcgVecs<double>(st, C);
             HIP_CHECK(hipMemcpyAsync(v.p, t.data(), t.size() * 8, hipMemcpyHostToDevice, s));
-            hipLaunchKernelGGL((k_spmvp<double, false>), dim3(bm.nBlocks), dim3(kBlock), 0, s, dm, bm, (const double*)nullptr,
-                               (const double*)v.p, (double*)nullptr, v.q, st.ctl.p, st.part.p, 0, (const double*)nullptr);
+            hipLaunchKernelGGL((k_spmvp<double, false>), dim3(bm.nBlocks), dim3(kBlock), 0, s, dm, bm,
+                               (const double*)nullptr, v.p, (double*)nullptr, v.q, (const Ctl*)st.ctl.p,
+                               st.part.p, 0, (const double*)nullptr);
             HIP_CHECK(hipGetLastError());
             soaToAos(download(st.q64, 3 * (size_t)C, s), C, 3, y);
         }
@@ -3106,6 +3225,7 @@ s4f_status s4f_pcg3(s4f_mesh* M, const s4f_solve_opts* o, const double* b, const
         for (int j = 0; j < 3; ++j) c0.normFactor[j] = normFactor[j];
         HIP_CHECK(hipMemcpyAsync(st.ctl.p, &c0, sizeof(Ctl), hipMemcpyHostToDevice, s));
         Ctl hc;
+        const Chain chain(st.ctl.p, M->h.instCell0.size(), canMerge(dm, bm.nBlocks), nullptr);
         auto run = [&](auto v, auto tag) {
             using T = decltype(tag);
             hipLaunchKernelGGL((k_pcg_start<T>), dim3(bm.nBlocks), dim3(kBlock), 0, s, dm, bm, bd.p, v.r, v.p, st.ctl.p,
@@ -3116,7 +3236,8 @@ s4f_status s4f_pcg3(s4f_mesh* M, const s4f_solve_opts* o, const double* b, const
             HIP_CHECK(hipMemsetAsync(v.x, 0, 3 * (size_t)C * sizeof(T), s));
             int total = 0;
             for (;;) {
-                launchPcgChunk<T>(dm, bm, 1, v, st.ctl.p, st.part.p, 8, s);
+                launchPcgChunk<T>(dm, bm, 1, v, chain, st.part.p, 8, s);
+                launchSettle(bm, 1, chain, st.part.p, s);
                 total += 8;
                 HIP_CHECK(hipMemcpyAsync(&hc, st.ctl.p, sizeof(Ctl), hipMemcpyDeviceToHost, s));
                 HIP_CHECK(hipStreamSynchronize(s));
@@ -3151,7 +3272,7 @@ s4f_status s4f_pcg3_noalloc(s4f_mesh* M, const s4f_solve_opts* o, const double* 
         if (C > kNoAllocMaxCells)
             throw InvalidError("s4f_pcg3_noalloc: " + std::to_string(C) + " cells exceed its scratch limit of " +
                                std::to_string(kNoAllocMaxCells) + " cells (use s4f_pcg3)");
-        if ((size_t)M->nBlocks * kMaxPartials * sizeof(double) > kNoAllocPartBytes)
+        if ((size_t)M->nBlocks * kPcgPartials * sizeof(double) > kNoAllocPartBytes)
             throw InvalidError("s4f_pcg3_noalloc: too many workgroup tiles for its scratch");
         if (M->h.instCell0.size() != 1) throw InvalidError("s4f_pcg3_noalloc: single meshes only");
         HIP_CHECK(hipSetDevice(M->ctx->device));
@@ -3167,6 +3288,7 @@ s4f_status s4f_pcg3_noalloc(s4f_mesh* M, const s4f_solve_opts* o, const double* 
         hipLaunchKernelGGL(k_ctl_set, dim3(1), dim3(64), 0, s, ctl, c0);
         const size_t n3 = 3 * (size_t)C;
         Ctl hc;
+        const Chain chain(ctl, 1, canMerge(dm, bm.nBlocks), nullptr);
         auto run = [&](auto tag, auto* xv) {
             using T = decltype(tag);
             PcgVecs<T> v;
@@ -3183,7 +3305,8 @@ s4f_status s4f_pcg3_noalloc(s4f_mesh* M, const s4f_solve_opts* o, const double* 
             HIP_CHECK(hipGetLastError());
             int total = 0;
             for (;;) {
-                launchPcgChunk<T>(dm, bm, 1, v, ctl, part, 8, s);
+                launchPcgChunk<T>(dm, bm, 1, v, chain, part, 8, s);
+                launchSettle(bm, 1, chain, part, s);
                 total += 8;
                 HIP_CHECK(hipMemcpyAsync(&hc, ctl, sizeof(Ctl), hipMemcpyDeviceToHost, s));
                 HIP_CHECK(hipStreamSynchronize(s));
@@ -3255,8 +3378,15 @@ double replayT(s4f_mesh* M, int kernel, int launches) {
     Ctl c;
     std::memset(&c, 0, sizeof(c));
     for (int j = 0; j < 3; ++j) { c.active[j] = 1; c.alpha[j] = 0.5; c.beta[j] = 0.5; c.rho[j] = 1.0; c.normFactor[j] = 1.0; }
+    c.pcgMaxIter = 1;
+    // the point of the solve at which the kernel runs; the kernels leave the
+    // control block as it is, the finalize kernels' results go to a second one
+    c.pending = kernel == S4F_KERNEL_RESIDUAL ? kPendRes
+                : kernel == S4F_KERNEL_GRAD ? kPendGrad
+                : kernel == S4F_KERNEL_PCG_UPDATE ? kPendUpd : kPendSpmv;
     DArr<Ctl> rc;
-    rc.alloc(1);
+    rc.alloc(2);
+    Chain chain(rc.p, 1, false, nullptr);
     HIP_CHECK(hipMemcpyAsync(rc.p, &c, sizeof(Ctl), hipMemcpyHostToDevice, s));
     // the multigrid kernels replay the hierarchy of the mesh's last multigrid solve
     const bool smoothedK = M->amgLast == &M->amgSm;
@@ -3264,25 +3394,26 @@ double replayT(s4f_mesh* M, int kernel, int launches) {
     auto launch = [&]() {
         switch (kernel) {
             case S4F_KERNEL_RESIDUAL:
-                hipLaunchKernelGGL((k_residual<T>), dim3(bm.nBlocks), dim3(kBlock), 0, s, dm, bm, (const double*)st.D0.p,
-                                   (const double*)st.D1.p, st.G.p, st.sigb.p, v.r, rc.p, st.part.p);
+                hipLaunchKernelGGL((k_residual<T>), dim3(bm.nBlocks), dim3(kBlock), 0, s, dm, bm,
+                                   (const double*)st.D0.p, (const double*)st.D1.p, (const double*)st.G.p,
+                                   (const double*)st.sigb.p, v.r, (const Ctl*)rc.p, st.part.p);
                 break;
             case S4F_KERNEL_SPMV:
                 hipLaunchKernelGGL((k_spmvp<T, false>), dim3(bm.nBlocks), dim3(kBlock), 0, s, dm, bm, (const T*)v.r,
-                                   (const T*)v.p, v.p2, v.q, rc.p, st.part.p, 1, (const T*)nullptr);
+                                   v.p, v.p2, v.q, (const Ctl*)rc.p, st.part.p, 1, (const T*)nullptr);
                 std::swap(v.p, v.p2);
                 break;
             case S4F_KERNEL_SPMV_MG:
                 hipLaunchKernelGGL((k_spmvp<T, true>), dim3(bm.nBlocks), dim3(kBlock), 0, s, dm, bm, (const T*)v.r,
-                                   (const T*)v.p, v.p2, v.q, rc.p, st.part.p, 1, (const T*)v.z);
+                                   v.p, v.p2, v.q, (const Ctl*)rc.p, st.part.p, 1, (const T*)v.z);
                 std::swap(v.p, v.p2);
                 break;
             case S4F_KERNEL_PCG_UPDATE:
-                hipLaunchKernelGGL((k_update<T>), dim3(bm.nBlocks), dim3(kBlock), 0, s, dm, bm, v.x, (const T*)v.p, v.r,
-                                   (const T*)v.q, (const Ctl*)rc.p, st.part.p);
+                hipLaunchKernelGGL((k_update<T>), dim3(bm.nBlocks), dim3(kBlock), 0, s, dm, bm, v.x, (const T*)v.p,
+                                   (const T*)v.p2, v.r, (const T*)v.q, (const Ctl*)rc.p, st.part.p);
                 break;
             case S4F_KERNEL_FINALIZE:
-                hipLaunchKernelGGL(k_fin_spmv, dim3(1), dim3(kFinBlock), 0, s, bm, rc.p, (const double*)st.part.p);
+                launchFin<kPtUpdate>(bm, 1, chain, rc.p, rc.p + 1, st.part.p, s);
                 break;
             case S4F_KERNEL_GRAD:
                 launchGradStep<T>(dm, bm, 1, M->maxInstNB,
@@ -3299,7 +3430,7 @@ double replayT(s4f_mesh* M, int kernel, int launches) {
                 launchMg0Up<T>(AK.d, dm, bm, v, AK.omega, AK.alpha, rc.p, st.part.p, s);
                 break;
             case S4F_KERNEL_VCYCLE:
-                launchVcycle<T>(meshRun(M, smoothedK), dm, bm, v, rc.p, st.part.p, s);
+                launchVcycle<T, false>(meshRun(M, smoothedK), dm, bm, v, chain, rc.p, st.part.p, s);
                 break;
             default:
                 throw InvalidError("unknown kernel id");
@@ -3649,14 +3780,17 @@ struct s4f_server {
     DArr<SegInt> segI;
     DArr<SegWords> segW;
     DArr<double> part;
-    DArr<int> bmInst, bmS0, bmS1, iBlk0, iNBlk, iCell0, iNCell, iB0, iNB, finList;
-    DArr<int> nbmInst, nbmS0, nbmS1, nfinList;  // init map of newly admitted instances
+    DArr<Tile> bmTile, nbmTile;  // map of the in-flight instances, init map of newly admitted ones
+    DArr<int> iBlk0, iNBlk, iNCell, iB0, iNB, finList, nfinList;
     std::vector<int> hiBlk0, hiNBlk, hiCell0, hiNCell, hiB0, hiNB;
-    int nTiles = 0, nActive = 0, chunk = 4;
-    // launch sequences of a step replayed from HIP graphs while the packed
-    // map they were captured on stands (mapGen counts rebuilds)
-    GraphExec gStart, gPair, gEnd;
-    unsigned mapGen = 0, capGen = ~0u, ranGen = ~0u;
+    int nTiles = 0, nActive = 0, inner = 1;
+    int maxTiles = 0;       // most tiles of an instance on the map
+    int uniW = 0;           // slot count of all slices on the map, 0 when they differ
+    long long liveTiles = 0;  // tiles of the map's unfinished instances
+    // passes replayed from HIP graphs (per PCG iterations in a pass) while the
+    // packed map they were captured on stands (mapGen counts rebuilds)
+    std::map<int, GraphExec> graph;
+    unsigned mapGen = 0, ranGen = ~0u;
     Ctl* hctl = nullptr;
     // bookkeeping (server thread only)
     std::vector<Placement> places;
@@ -3733,8 +3867,8 @@ void serverAllocate(s4f_server* S) {
         S->r64.alloc(3 * Cc); S->p64.alloc(3 * Cc); S->pb64.alloc(3 * Cc); S->q64.alloc(3 * Cc); S->x64.alloc(3 * Cc);
         if (S->mgOn) S->z64.alloc(3 * Cc);
     }
-    S->ctl.alloc(S->maxSlots);
-    std::vector<Ctl> zero(S->maxSlots);
+    S->ctl.alloc((size_t)kChain * S->maxSlots);
+    std::vector<Ctl> zero(S->ctl.n);
     std::memset(zero.data(), 0, zero.size() * sizeof(Ctl));
     for (Ctl& c : zero) c.outerDone = 1;
     hcopy(S->ctx->stream, S->ctl.p, zero.data(), zero.size());
@@ -3742,7 +3876,7 @@ void serverAllocate(s4f_server* S) {
     S->hiBlk0.assign(S->maxSlots, 0); S->hiNBlk.assign(S->maxSlots, 0);
     S->hiCell0.assign(S->maxSlots, 0); S->hiNCell.assign(S->maxSlots, 0);
     S->hiB0.assign(S->maxSlots, 0); S->hiNB.assign(S->maxSlots, 0);
-    S->iBlk0.alloc(S->maxSlots); S->iNBlk.alloc(S->maxSlots); S->iCell0.alloc(S->maxSlots); S->iNCell.alloc(S->maxSlots);
+    S->iBlk0.alloc(S->maxSlots); S->iNBlk.alloc(S->maxSlots); S->iNCell.alloc(S->maxSlots);
     S->iB0.alloc(S->maxSlots); S->iNB.alloc(S->maxSlots);
     S->slotReq.assign(S->maxSlots, -1);
 }
@@ -3899,21 +4033,16 @@ int acquirePlacement(s4f_server* S, const Request& rq) {
 }
 
 // tile list of the given slots (the same per-instance rule as a plain solve)
-void buildTiles(const s4f_server* S, const std::vector<int>& slots, std::vector<int>& inst, std::vector<int>& s0,
-                std::vector<int>& s1, std::vector<int>& blk0, std::vector<int>& nblk) {
-    inst.clear(); s0.clear(); s1.clear();
+void buildTiles(const s4f_server* S, const std::vector<int>& slots, std::vector<Tile>& tile, std::vector<int>& blk0,
+                std::vector<int>& nblk) {
+    tile.clear();
     for (int slot : slots) {
         const Request& rq = S->live[S->slotReq[slot]];
         const Placement& pl = S->places[rq.place];
-        const int a = pl.slice0, nS = pl.nSlices, e = a + nS;
-        const int spbI = tileSlices(rq.mesh->h, 0, nS);
-        blk0[slot] = (int)inst.size();
-        for (int x = a; x < e; x += spbI) {
-            inst.push_back(slot);
-            s0.push_back(x);
-            s1.push_back(std::min(x + spbI, e));
-        }
-        nblk[slot] = (int)inst.size() - blk0[slot];
+        blk0[slot] = (int)tile.size();
+        addTiles(tile, slot, pl.slice0, pl.nSlices, tileSlices(rq.mesh->h, 0, pl.nSlices), (int)pl.c0 + pl.nCells,
+                 pl.nCells);
+        nblk[slot] = (int)tile.size() - blk0[slot];
     }
 }
 
@@ -3936,10 +4065,10 @@ GradBufs serverGradBufs(s4f_server* S) {
 
 int serverMaxNB(const s4f_server* S) { return *std::max_element(S->hiNB.begin(), S->hiNB.end()); }
 
-BlockMap makeMap(const s4f_server* S, const int* inst, const int* s0, const int* s1, const int* fin, int nBlocks) {
+BlockMap makeMap(const s4f_server* S, const Tile* tile, const int* fin, int nBlocks) {
     BlockMap b{};
-    b.inst = inst; b.s0 = s0; b.s1 = s1;
-    b.iBlk0 = S->iBlk0.p; b.iNBlk = S->iNBlk.p; b.iCell0 = S->iCell0.p; b.iNCell = S->iNCell.p;
+    b.tile = tile;
+    b.iBlk0 = S->iBlk0.p; b.iNBlk = S->iNBlk.p; b.iNCell = S->iNCell.p;
     b.iB0 = S->iB0.p; b.iNB = S->iNB.p;
     b.finInst = fin;
     b.nBlocks = nBlocks;
@@ -3978,6 +4107,7 @@ void serverAdmit(s4f_server* S) {
         c.dpar = warm ? pl.dpar : 0;
         c.solveMask = rq.mesh->h.instMask.empty() ? 7 : rq.mesh->h.instMask[0];
         c.pcMode = S->mgOn ? 1 : 0;
+        c.pending = kPendStart;
         c.warm = warm;
         c.sigma0 = warm ? 0 : 1;
         HIP_CHECK(hipStreamSynchronize(S->ctx->stream));
@@ -3998,21 +4128,21 @@ void serverAdmit(s4f_server* S) {
     }
     if (newSlots.empty()) return;
     // initialisation (constructor grad) of the new instances only
-    std::vector<int> inst, s0, s1;
-    buildTiles(S, newSlots, inst, s0, s1, S->hiBlk0, S->hiNBlk);
+    std::vector<Tile> tile;
+    buildTiles(S, newSlots, tile, S->hiBlk0, S->hiNBlk);
     hipStream_t s = S->ctx->stream;
-    S->nbmInst.upload(inst, s); S->nbmS0.upload(s0, s); S->nbmS1.upload(s1, s); S->nfinList.upload(newSlots, s);
+    S->nbmTile.upload(tile, s); S->nfinList.upload(newSlots, s);
     S->iBlk0.upload(S->hiBlk0, s); S->iNBlk.upload(S->hiNBlk, s);
-    S->iCell0.upload(S->hiCell0, s); S->iNCell.upload(S->hiNCell, s);
+    S->iNCell.upload(S->hiNCell, s);
     S->iB0.upload(S->hiB0, s); S->iNB.upload(S->hiNB, s);
-    S->part.alloc(std::max<size_t>(S->part.n, inst.size() * kMaxPartials));
-    const BlockMap bm = makeMap(S, S->nbmInst.p, S->nbmS0.p, S->nbmS1.p, S->nfinList.p, (int)inst.size());
+    S->part.alloc(std::max<size_t>(S->part.n, tile.size() * kMaxPartials));
+    const BlockMap bm = makeMap(S, S->nbmTile.p, S->nfinList.p, (int)tile.size());
     const DevMesh dm = serverDm(S);
     launchGradStep<T>(dm, bm, (int)newSlots.size(), serverMaxNB(S),
                       serverGradBufs(S), nullptr,
                       (const double*)S->Dold.p, S->ctl.p, S->part.p, 1, s);
-    hipLaunchKernelGGL(k_fin_grad, dim3((int)newSlots.size()), dim3(kFinBlock), 0, s, bm, S->ctl.p,
-                       (const double*)S->part.p, (double*)nullptr, 1);
+    hipLaunchKernelGGL(k_fin_init, dim3((int)newSlots.size()), dim3(kFinBlock), 0, s, bm, S->ctl.p,
+                       (const double*)S->part.p);
     HIP_CHECK(hipGetLastError());
     S->nTiles = -1;  // active map must be rebuilt
 }
@@ -4208,103 +4338,82 @@ MgRun serverRun(s4f_server* S) {
 
 void serverRebuildMap(s4f_server* S) {
     S->mapGen++;  // tiles, multigrid packing and slot set change: captured graphs are stale
+    S->graph.clear();
     std::vector<int> slots;
     for (int i = 0; i < S->maxSlots; ++i)
         if (S->slotReq[i] >= 0) slots.push_back(i);
     if (S->mgOn && !slots.empty()) serverPackMg(S, slots);
-    std::vector<int> inst, s0, s1;
-    buildTiles(S, slots, inst, s0, s1, S->hiBlk0, S->hiNBlk);
+    std::vector<Tile> tile;
+    buildTiles(S, slots, tile, S->hiBlk0, S->hiNBlk);
     hipStream_t s = S->ctx->stream;
-    S->bmInst.upload(inst, s); S->bmS0.upload(s0, s); S->bmS1.upload(s1, s); S->finList.upload(slots, s);
+    S->bmTile.upload(tile, s); S->finList.upload(slots, s);
     S->iBlk0.upload(S->hiBlk0, s); S->iNBlk.upload(S->hiNBlk, s);
-    S->part.alloc(std::max<size_t>(S->part.n, inst.size() * kMaxPartials));
-    S->nTiles = (int)inst.size();
+    S->part.alloc(std::max<size_t>(S->part.n, tile.size() * kMaxPartials));
+    S->nTiles = (int)tile.size();
     S->nActive = (int)slots.size();
+    S->liveTiles = S->nTiles;
+    S->maxTiles = 0;
+    S->uniW = 0;
+    for (size_t k = 0; k < slots.size(); ++k) {
+        S->maxTiles = std::max(S->maxTiles, S->hiNBlk[slots[k]]);
+        const int w = S->live[S->slotReq[slots[k]]].mesh->h.uniformWidth();
+        S->uniW = k == 0 || w == S->uniW ? w : 0;
+    }
 }
 
-// one outer iteration of every in-flight solve, then retire the converged
+// passes of the launch sequence over every in-flight solve between two looks
+// at their control blocks (a finished solve waits this long at most)
+constexpr int kServerPasses = 8;
+
+// a few passes over every in-flight solve, then retire the converged
 template <typename T>
 void serverStep(s4f_server* S) {
     hipStream_t s = S->ctx->stream;
     if (S->nTiles < 0) serverRebuildMap(S);
     if (S->nActive == 0) return;
-    const DevMesh dm = serverDm(S);
-    const BlockMap bm = makeMap(S, S->bmInst.p, S->bmS0.p, S->bmS1.p, S->finList.p, S->nTiles);
+    DevMesh dm = serverDm(S);
+    dm.uniW = S->uniW;  // entry ranges are placed one by one: their starts are loaded
+    const BlockMap bm = makeMap(S, S->bmTile.p, S->finList.p, S->nTiles);
     PcgVecs<T> v = serverVecs<T>(S);
-    const int nA = S->nActive;
+    const Chain chain(S->ctl.p, S->maxSlots, canMerge(dm, S->maxTiles), nullptr);
+    MgRun run{nullptr, 0.0, 0.0, S->nActive};
+    if (S->mgOn) run = serverRun(S);
     std::vector<int> slots;
     for (int i = 0; i < S->maxSlots; ++i)
         if (S->slotReq[i] >= 0) slots.push_back(i);
-    // one outer iteration of every active request: explicit terms and the
-    // first V-cycle, PCG iterations (in pairs, so the search-direction
-    // buffers return to their places), the gradient step
-    auto launchStart = [&](hipStream_t q) {
-        hipLaunchKernelGGL((k_residual<T>), dim3(bm.nBlocks), dim3(kBlock), 0, q, dm, bm, (const double*)S->D0.p,
-                           (const double*)S->D1.p, S->G.p, S->sigb.p, v.r, S->ctl.p, S->part.p);
-        hipLaunchKernelGGL(k_fin_residual, dim3(nA), dim3(kFinBlock), 0, q, bm, S->ctl.p, (const double*)S->part.p);
-        if (S->mgOn) launchVcycle<T>(serverRun(S), dm, bm, v, S->ctl.p, S->part.p, q);  // z0 = V(r0), rho0
+    auto launch = [&](hipStream_t q) {
+        launchPass<T>(S->mgOn, run, dm, bm, serverMaxNB(S), serverGradBufs(S), v, (const double*)S->Dold.p, chain,
+                      S->part.p, S->inner, q);
     };
-    auto launchPcg = [&](int n, hipStream_t q) {
-        if (S->mgOn) launchPcgChunkMg<T>(serverRun(S), dm, bm, v, S->ctl.p, S->part.p, n, q);
-        else launchPcgChunk<T>(dm, bm, nA, v, S->ctl.p, S->part.p, n, q);
-    };
-    auto launchEnd = [&](hipStream_t q) {
-        launchGradStep<T>(dm, bm, nA, serverMaxNB(S), serverGradBufs(S), (const T*)v.x, (const double*)S->Dold.p,
-                          S->ctl.p, S->part.p, 0, q);
-        hipLaunchKernelGGL(k_fin_grad, dim3(nA), dim3(kFinBlock), 0, q, bm, S->ctl.p, (const double*)S->part.p,
-                           (double*)nullptr, 0);
-    };
-    // the first step on a new map runs eagerly (it allocates the multigrid
-    // vectors of the packing); the next one captures
-    bool graphs = false;
-    if (S->opts.eagerLaunch == 0 && S->ranGen == S->mapGen) {
-        graphs = true;
-        if (S->capGen != S->mapGen) {
-            try {
-                S->gStart.capture(S->ctx->capture, launchStart);
-                S->gPair.capture(S->ctx->capture, [&](hipStream_t q) { launchPcg(2, q); });
-                S->gEnd.capture(S->ctx->capture, launchEnd);
-                S->capGen = S->mapGen;
-            } catch (const HipError&) {  // a runtime without capture: the same launches, one by one
-                S->gStart.reset();
-                S->gPair.reset();
-                S->gEnd.reset();
-                (void)hipGetLastError();
-                S->opts.eagerLaunch = 1;
-                graphs = false;
+    for (int k = 0; k < kServerPasses; ++k) {
+        // the first pass on a new map runs eagerly (it allocates the
+        // multigrid vectors of the packing); later ones are replayed
+        const bool eager = S->opts.eagerLaunch != 0 || S->ranGen != S->mapGen;
+        if (!eager) {
+            GraphExec& g = S->graph[S->inner];
+            if (!g.e) {
+                try {
+                    g.capture(S->ctx->capture, launch);
+                } catch (const HipError&) {  // a runtime without capture: the same launches, one by one
+                    (void)hipGetLastError();
+                    S->graph.clear();
+                    S->opts.eagerLaunch = 1;
+                }
             }
         }
+        if (!eager && S->opts.eagerLaunch == 0) S->graph[S->inner].launch(s);
+        else launch(s);
+        S->ranGen = S->mapGen;
     }
-    if (graphs) S->gStart.launch(s);
-    else launchStart(s);
-    int total = 0, chunk = S->chunk;
-    for (;;) {
-        if (graphs) {
-            const int pairs = (chunk + 1) / 2;
-            for (int k = 0; k < pairs; ++k) S->gPair.launch(s);
-            chunk = 2 * pairs;
-        } else {
-            launchPcg(chunk, s);
-        }
-        total += chunk;
-        chunk = std::max(2, chunk / 4);
-        HIP_CHECK(hipMemcpyAsync(S->hctl, S->ctl.p, S->maxSlots * sizeof(Ctl), hipMemcpyDeviceToHost, s));
-        HIP_CHECK(hipStreamSynchronize(s));
-        bool any = false;
-        for (int sl : slots)
-            if (!S->hctl[sl].outerDone && !S->hctl[sl].innerDone) any = true;
-        if (!any || total > S->opts.pcgMaxIter + 2) break;
-    }
+    // pending partials are laid out by this map: nothing stays pending over a change
+    launchSettle(bm, S->nActive, chain, S->part.p, s);
+    HIP_CHECK(hipGetLastError());
+    HIP_CHECK(hipMemcpyAsync(S->hctl, S->ctl.p, S->maxSlots * sizeof(Ctl), hipMemcpyDeviceToHost, s));
+    HIP_CHECK(hipStreamSynchronize(s));
     int used = 1;
     for (int sl : slots)
         if (!S->hctl[sl].outerDone) used = std::max({used, S->hctl[sl].nIter[0], S->hctl[sl].nIter[1], S->hctl[sl].nIter[2]});
-    S->chunk = std::max(1, used - 1);
-    if (graphs) S->gEnd.launch(s);
-    else launchEnd(s);
-    HIP_CHECK(hipGetLastError());
-    S->ranGen = S->mapGen;
-    HIP_CHECK(hipMemcpyAsync(S->hctl, S->ctl.p, S->maxSlots * sizeof(Ctl), hipMemcpyDeviceToHost, s));
-    HIP_CHECK(hipStreamSynchronize(s));
+    S->inner = innerPerPass(S->mgOn, used);
     // retire
     bool changed = false;
     for (int sl : slots) {
@@ -4350,6 +4459,7 @@ void serverStep(s4f_server* S) {
         const long long id = rq.id;
         rq.place = -1;
         S->slotReq[sl] = -1;
+        S->liveTiles -= S->hiNBlk[sl];
         changed = true;
         {
             std::lock_guard<std::mutex> lk(S->mu_);
@@ -4368,7 +4478,9 @@ void serverStep(s4f_server* S) {
                 S->slotReq[i] = (int)keep.size() - 1;
             }
         S->live.swap(keep);
-        S->nTiles = -1;
+        // the map drops its finished instances once they hold a quarter of its
+        // tiles (their workgroups exit at once; a new map costs a packing and a capture)
+        if (4 * S->liveTiles <= 3 * (long long)S->nTiles) S->nTiles = -1;
     }
 }
 
@@ -4642,25 +4754,28 @@ s4f_status s4f_ldu_solve(s4f_ldu* L, const double* diag, const double* upper, co
         o.precision = precision;
         checkOpts(o);
         Ctl c0 = makeCtl(o, 0);
+        c0.pending = kPendRes;
         HIP_CHECK(hipMemcpyAsync(st.ctl.p, &c0, sizeof(Ctl), hipMemcpyHostToDevice, s));
         const DevMesh dm = M->dm();
         const BlockMap bm = M->bmap();
+        const Chain chain(st.ctl.p, 1, canMerge(dm, bm.nBlocks), nullptr);
         Ctl hc;
         std::vector<double> x(C, 0.0);
         auto run = [&](auto v, auto tag) {
             using T = decltype(tag);
             hipLaunchKernelGGL((k_ldu_start<T>), dim3(bm.nBlocks), dim3(kBlock), 0, s, dm, bm, (const double*)dpsi.p,
                                (const double*)dsrc.p, avg, v.r, st.part.p);
-            hipLaunchKernelGGL(k_fin_residual, dim3(1), dim3(kFinBlock), 0, s, bm, st.ctl.p, (const double*)st.part.p);
+            launchFin<kPtInner>(bm, 1, chain, st.ctl.p, st.ctl.p, st.part.p, s);
             HIP_CHECK(hipMemsetAsync(v.x, 0, 3 * (size_t)C * sizeof(T), s));
             HIP_CHECK(hipGetLastError());
             int total = 0, chunk = 8;
             for (;;) {
+                launchPcgChunk<T>(dm, bm, 1, v, chain, st.part.p, chunk, s);
+                launchSettle(bm, 1, chain, st.part.p, s);
+                total += chunk;
                 HIP_CHECK(hipMemcpyAsync(&hc, st.ctl.p, sizeof(Ctl), hipMemcpyDeviceToHost, s));
                 HIP_CHECK(hipStreamSynchronize(s));
                 if (hc.innerDone || total > maxIter + 8) break;
-                launchPcgChunk<T>(dm, bm, 1, v, st.ctl.p, st.part.p, chunk, s);
-                total += chunk;
             }
             std::vector<T> xs(C);
             HIP_CHECK(hipMemcpyAsync(xs.data(), v.x, C * sizeof(T), hipMemcpyDeviceToHost, s));

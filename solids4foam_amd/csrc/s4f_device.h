@@ -9,7 +9,15 @@ namespace s4f {
 constexpr int kBlock = 256;          // threads per workgroup (4 wave64)
 constexpr int kSlice = 64;           // rows per sliced-ELL slice (one wavefront)
 constexpr int kPad = INT32_MIN;      // padding entry in the ELL column array
-constexpr int kMaxPartials = 16;     // reduction values per block
+// block partials: each reducing kernel has its own value range, so a kernel
+// can reduce its predecessor's partials while it writes its own
+constexpr int kOffSpmv = 0;    // p.q (3)
+constexpr int kOffUpd = 3;     // z.r, sum|r| (6)
+constexpr int kOffRho = 9;     // z.r of the V-cycle (3); the PCG start's sums (6)
+constexpr int kOffRes = 12;    // sum|R|, normFactor sums, z.r (12)
+constexpr int kOffGrad = 24;   // outer convergence maxima, sum D' (6)
+constexpr int kMaxPartials = 30;  // reduction values per block
+constexpr int kPcgPartials = 16;  // of them used by a PCG without an outer loop
 constexpr double kSmall = 1e-15;     // OpenFOAM SMALL (double)
 constexpr double kVSmall = 1e-300;   // OpenFOAM VSMALL (double)
 
@@ -18,6 +26,28 @@ constexpr double kVSmall = 1e-300;   // OpenFOAM VSMALL (double)
 // so the L2 keeps the neighbour rows that the gathers reuse.
 template <typename T> __device__ __forceinline__ T ldS(const T* p) { return __builtin_nontemporal_load(p); }
 template <typename T> __device__ __forceinline__ void stS(T* p, T v) { __builtin_nontemporal_store(v, p); }
+
+// Element of an array at a 32-bit byte offset.  With a base that is uniform over
+// the wavefront (scalar registers) this is one load with a scalar base and a
+// vector offset: a cell's offset serves every component array, where a 64-bit
+// address per array cost two vector registers and two additions each (the
+// merged residual went from 256 registers with spills to 160 without).  Cell
+// arrays fit: 2^29 cells (8-byte elements) need more than the 288 GB of a card.
+// The empty asm keeps the base in scalar registers: the compiler would
+// otherwise add the component's distance to the per-lane address.
+#define S4F_GLOBAL __attribute__((address_space(1)))
+template <typename T> __device__ __forceinline__ T at32(const T* base, unsigned off) {
+    const S4F_GLOBAL char* b = (const S4F_GLOBAL char*)base;
+    asm("" : "+s"(b));
+    return *(const S4F_GLOBAL T*)(b + off);
+}
+template <typename T> __device__ __forceinline__ void put32(T* base, unsigned off, T v) {
+    S4F_GLOBAL char* b = (S4F_GLOBAL char*)base;
+    asm("" : "+s"(b));
+    *(S4F_GLOBAL T*)(b + off) = v;
+}
+// wavefront of the workgroup, known uniform
+__device__ __forceinline__ int waveOf() { return __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6); }
 
 // Device view of one solver mesh (or of a packed batch of meshes).
 // Cell-indexed arrays are structure-of-arrays: component k of cell c at
@@ -29,6 +59,8 @@ template <typename T> __device__ __forceinline__ void stS(T* p, T v) { __builtin
 // face order (= ascending other-cell label), then boundary faces.
 struct DevMesh {
     int nCells, nBoundary, nSlices, slicesPerBlock, nBlocks;
+    int uniW;               // > 0: every slice has this many slots
+    int contig;             // and the slices' entries follow one another: slice s from s * uniW * 64
     size_t nEntries;
     const int* sliceStart;  // first ELL entry of each slice
     const int* sliceWidth;  // slots of each slice
@@ -75,11 +107,33 @@ struct DevMesh {
     const int* eIf;               // per ELL entry: interface side 2 i + (0 a, 1 b), or -1
     const unsigned char* sliceIf; // per slice: 1 if it holds interface entries
     const int* zone;              // material zone of each cell (nullptr: one material)
+    __device__ __forceinline__ int width(int s) const { return uniW ? uniW : sliceWidth[s]; }
+    __device__ __forceinline__ int entry0(int s) const { return contig ? s * uniW * kSlice : sliceStart[s]; }
 };
 
-// Solve control block, written by the last workgroup of each reducing kernel
-// and read by every later kernel in the stream.
+// Reduced scalars an instance still owes its control block: the block partials
+// of the named step are written, and the next kernel of the launch sequence
+// (or a finalize kernel in front of it) reduces them and moves the instance on.
+// A kernel runs for an instance only when the instance has reached it, so one
+// launch sequence serves instances at different points of their solves.
+enum Pending {
+    kPendNone = 0,   // between steps: innerDone says whether the PCG or the outer step comes next
+    kPendStart = 1,  // fields initialised, residual next
+    kPendGrad = 2,   // gradient step of an outer iteration
+    kPendRes = 3,    // residual
+    kPendRho = 4,    // V-cycle of a PCG iteration
+    kPendSpmv = 5,   // search direction and matrix product
+    kPendUpd = 6     // solution and residual update
+};
+
+// Solve control block of one instance.
 struct Ctl {
+    int pending;     // Pending
+    int pIt;         // PCG iterations of this outer iteration (its parity names the direction buffer)
+    int hold;        // no further outer step starts (mixed precision's fallback)
+    int stallWindow, bestIt, stalled;  // mixed precision's stall test (0: off)
+    double bestRes;
+    long long pcgTotal;  // 3-RHS PCG iterations over the outer iterations
     int outerDone, innerDone, converged, diverged;
     int iCorr, nOuter, firstInner, warm;
     int dpar;        // which displacement buffer holds the current field
@@ -91,10 +145,9 @@ struct Ctl {
     double xbar[4];
     double initResMag, rvf;
     long long innerTotal;
-    unsigned counter[8];
     // settings
     double pcgTol, pcgRelTol, solTol, altTol;
-    int pcgMaxIter, nCorr, histCap, pcMode;  // pcMode 1: z comes from the V-cycle (k_fin_rho sets beta)
+    int pcgMaxIter, nCorr, histCap, pcMode;  // pcMode 1: z comes from the V-cycle (finRho sets beta)
     double relaxD;                           // fixed field under-relaxation factor (1: none)
     int solveMask;                           // solved components (bit j); 2-D leaves the empty axis out
     int relaxAitken;                         // relaxationMethod Aitken (relaxD: its first factor)

@@ -5,10 +5,11 @@
 // slice is one coalesced load per array.  Face contributions are gathered
 // per cell in OpenFOAM's face order, so no atomics touch field data and the
 // summation order is fixed (run-to-run bitwise deterministic).  Reductions
-// are per workgroup (wave shuffles + LDS) into a partial array; a one-block-
-// per-instance finalize kernel then reduces the instance's partials in fixed
-// order and updates the control block (kernel boundaries order the writes of
-// every XCD before the finalize reads them).
+// are per workgroup (wave shuffles + LDS) into a partial array; the next kernel
+// of a merged launch sequence (Chain), or else a one-block-per-instance finalize
+// kernel, then reduces the instance's partials in fixed order and updates the
+// control block (kernel boundaries order the writes of every XCD before they
+// are read).
 //
 // Kernel <-> reference map (paths relative to the solids4foam tree):
 //   k_residual   linGeomTotalDispSolid.C:141-149: fvc::div(sigma) [Gauss linear]
@@ -17,7 +18,7 @@
 //   k_spmvp      OpenFOAM PCG search-direction update p = z + beta p fused with
 //                lduMatrix::Amul (3 right-hand sides sharing M)
 //   k_update     OpenFOAM PCG solution/residual update + diagonal preconditioner
-//   k_fin_*      the scalar parts of PCG::solve / normFactor / solidModel::converged
+//   fin* / k_fin  the scalar parts of PCG::solve / normFactor / solidModel::converged
 //   k_grad       solidTractionFvPatchVectorField.C:398-463 / fixedDisplacement
 //                boundary values, leastSquares grad(D) (mechanicalModel.C:571-582),
 //                gaussGrad boundary correction, linearElastic::correct on
@@ -30,18 +31,30 @@
 
 namespace s4f {
 
+// One workgroup tile: its instance, slices [s0, s1), the end of the
+// instance's cells, and the instance's tiles and cell count (32 bytes, one
+// scalar load)
+struct alignas(32) Tile {
+    int inst, s0, s1, cEnd, blk0, nBlk, nCell, pad;
+};
+
 struct BlockMap {
-    const int* inst;   // instance of each logical block
-    const int* s0;     // first slice
-    const int* s1;     // one past last slice
+    const Tile* tile;  // each logical block's tile
+    // one instance (spb > 0): tiles of spb slices from slice 0, computed
+    // instead of loaded (a load less in front of every kernel's own loads)
+    int spb, nSlices, nCells;
     const int* iBlk0;  // per instance: first logical block
     const int* iNBlk;  // per instance: number of blocks
-    const int* iCell0; // per instance: first cell
     const int* iNCell; // per instance: number of cells
     const int* finInst;// instance finalized by finalize-kernel workgroup i (nullptr: i itself)
     const int* iB0;    // per instance: first boundary face
     const int* iNB;    // per instance: number of boundary faces
     int nBlocks;
+    __device__ __forceinline__ Tile at(int lb) const {
+        if (spb == 0) return tile[lb];
+        const int s0 = lb * spb;
+        return Tile{0, s0, s0 + spb < nSlices ? s0 + spb : nSlices, nCells, 0, nBlocks, nCells, 0};
+    }
 };
 
 // Workgroups are dispatched round-robin over the 8 XCDs (hardware block b runs
@@ -56,14 +69,86 @@ __device__ __forceinline__ int logicalBlock(int nb) {
 // NaN-propagating maximum (fmax would drop a NaN and hide a diverged solve)
 __device__ __forceinline__ double nanMax(double a, double b) { return (b > a || b != b) ? b : a; }
 
+// v of the lane a row rotation away (a row: 16 lanes)
+template <int ROR>
+__device__ __forceinline__ double rowRor(double v) {
+    const int lo = __builtin_amdgcn_update_dpp(0, __double2loint(v), 0x120 + ROR, 0xf, 0xf, false);
+    const int hi = __builtin_amdgcn_update_dpp(0, __double2hiint(v), 0x120 + ROR, 0xf, 0xf, false);
+    return __hiloint2double(hi, lo);
+}
+
+// x + y (or their maximum) of the two halves (32) or the two rows of each half
+// (16): with values a and b, lanes of the lower half (even row) get a's result,
+// those of the upper half (odd row) b's
+template <bool MAX>
+__device__ __forceinline__ double redOp(double x, double y) { return MAX ? nanMax(x, y) : x + y; }
+template <bool MAX>
+__device__ __forceinline__ double halves(double a, double b) {
+    const auto l = __builtin_amdgcn_permlane32_swap(__double2loint(a), __double2loint(b), false, false);
+    const auto h = __builtin_amdgcn_permlane32_swap(__double2hiint(a), __double2hiint(b), false, false);
+    return redOp<MAX>(__hiloint2double(h[0], l[0]), __hiloint2double(h[1], l[1]));
+}
+template <bool MAX>
+__device__ __forceinline__ double rows(double a, double b) {
+    const auto l = __builtin_amdgcn_permlane16_swap(__double2loint(a), __double2loint(b), false, false);
+    const auto h = __builtin_amdgcn_permlane16_swap(__double2hiint(a), __double2hiint(b), false, false);
+    return redOp<MAX>(__hiloint2double(h[0], l[0]), __hiloint2double(h[1], l[1]));
+}
+template <bool MAX>
+__device__ __forceinline__ double inRow(double v) {
+    v = redOp<MAX>(v, rowRor<8>(v));
+    v = redOp<MAX>(v, rowRor<4>(v));
+    v = redOp<MAX>(v, rowRor<2>(v));
+    return redOp<MAX>(v, rowRor<1>(v));
+}
+
+// Butterfly over the wavefront (distances 32, 16, 8, 4, 2, 1): every lane gets
+// the result.  The first two steps swap half-wavefronts and rows in registers,
+// the others rotate within a row: once lanes at the larger distances hold
+// equal values, a rotation by d gives the value of the lane at distance d.
 template <bool MAX>
 __device__ __forceinline__ double waveReduce(double v) {
+    v = halves<MAX>(v, v);
+    return inRow<MAX>(rows<MAX>(v, v));
+}
+
+// The same tree for N values at once, each step halving the values a lane
+// carries (21 additions for 12 values instead of 72): value i of the
+// wavefront goes to out[4 i + w].  The reductions were 8 of 20 KB of the
+// merged residual's code, and a kernel of a few workgroups mostly waits for
+// its instructions.
+template <int N, bool MAX>
+__device__ __forceinline__ void waveReduceTo(const double* v, double* out, int w) {
+    constexpr int M = (N + 1) / 2, K = (M + 1) / 2;
+    double r[M], q[K];
 #pragma unroll
-    for (int off = 32; off > 0; off >>= 1) {
-        const double o = __shfl_xor(v, off, 64);
-        v = MAX ? nanMax(v, o) : v + o;
+    for (int i = 0; i < M; ++i) r[i] = halves<MAX>(v[i], v[i + M < N ? i + M : i]);
+#pragma unroll
+    for (int i = 0; i < K; ++i) q[i] = inRow<MAX>(rows<MAX>(r[i], r[i + K < M ? i + K : i]));
+    const int lane = threadIdx.x & 63;
+    if ((lane & 15) == 0) {
+        const int upper = lane >> 5, odd = (lane >> 4) & 1;
+#pragma unroll
+        for (int i = 0; i < K; ++i) {
+            const int ir = odd && i + K < M ? i + K : i;
+            const int iv = upper && ir + M < N ? ir + M : ir;
+            out[4 * iv + w] = q[i];
+        }
     }
-    return v;
+}
+// values [0, NMAX) by maximum, the rest by sum
+template <int N, int NMAX>
+__device__ __forceinline__ void waveReduceAll(const double* v, double* out, int w) {
+    if constexpr (NMAX > 0) waveReduceTo<NMAX, true>(v, out, w);
+    waveReduceTo<N - NMAX, false>(v + NMAX, out + 4 * NMAX, w);
+}
+// value i over the workgroup's wavefronts, from out[4 i + w]
+template <int NMAX>
+__device__ __forceinline__ double overWaves(const double* out, int i) {
+    double r = out[4 * i];
+#pragma unroll
+    for (int w = 1; w < kBlock / 64; ++w) r = i < NMAX ? nanMax(r, out[4 * i + w]) : r + out[4 * i + w];
+    return r;
 }
 
 constexpr int kFinBlock = 256;
@@ -74,57 +159,293 @@ constexpr int kFinBlock = 256;
 // row per block.
 //
 // Fixed-order reduction of the instance's partials (one workgroup per
-// instance); bit i of maxMask selects a maximum instead of a sum.  Result in
+// instance); the first NMAX values by maximum, the others by sum.  Result in
 // out[0..NV) (shared), valid for every thread after the call.
-template <int NV>
-__device__ void finReduce(const double* __restrict__ part, int nb, int blk0, int nblk, unsigned maxMask, double* out) {
+template <int NV, int NMAX>
+__device__ void finReduce(const double* __restrict__ part, int nb, int blk0, int nblk, double* out) {
     double v[NV];
 #pragma unroll
     for (int i = 0; i < NV; ++i) v[i] = 0.0;
     for (int b = threadIdx.x; b < nblk; b += kFinBlock) {
         const double* col = part + blk0 + b;
 #pragma unroll
-        for (int i = 0; i < NV; ++i) {
-            const double x = col[(size_t)i * nb];
-            v[i] = ((maxMask >> i) & 1u) ? nanMax(v[i], x) : v[i] + x;
-        }
+        for (int i = 0; i < NV; ++i) v[i] = i < NMAX ? nanMax(v[i], col[(size_t)i * nb]) : v[i] + col[(size_t)i * nb];
     }
-    __shared__ double sh[NV][kFinBlock / 64];
-    const int w = threadIdx.x >> 6, l = threadIdx.x & 63;
-#pragma unroll
-    for (int i = 0; i < NV; ++i) {
-        v[i] = ((maxMask >> i) & 1u) ? waveReduce<true>(v[i]) : waveReduce<false>(v[i]);
-        if (l == 0) sh[i][w] = v[i];
-    }
+    __shared__ double sh[4 * NV];
+    waveReduceAll<NV, NMAX>(v, sh, threadIdx.x >> 6);
     __syncthreads();
-    if (threadIdx.x < NV) {
-        const int i = threadIdx.x;
-        double r = sh[i][0];
-        for (int k = 1; k < kFinBlock / 64; ++k) r = ((maxMask >> i) & 1u) ? nanMax(r, sh[i][k]) : r + sh[i][k];
-        out[i] = r;
-    }
+    if (threadIdx.x < NV) out[threadIdx.x] = overWaves<NMAX>(sh, threadIdx.x);
     __syncthreads();
 }
 
-// block-level reduction of NV per-thread values; threads 0..NV-1 store them
-// at part[i * nb + lb]
-template <int NV>
-__device__ __forceinline__ void storeBlockPartials(const double* acc, unsigned maxMask, double* part, int lb, int nb) {
-    __shared__ double sh[NV][kBlock / 64];
-    const int w = threadIdx.x >> 6, l = threadIdx.x & 63;
-#pragma unroll
-    for (int i = 0; i < NV; ++i) {
-        const double v = ((maxMask >> i) & 1u) ? waveReduce<true>(acc[i]) : waveReduce<false>(acc[i]);
-        if (l == 0) sh[i][w] = v;
-    }
+// block-level reduction of NV per-thread values (the first NMAX by maximum);
+// threads 0..NV-1 store them at part[(off + i) * nb + lb]
+template <int NV, int NMAX>
+__device__ __forceinline__ void storeBlockPartials(const double* acc, double* part, int off, int lb, int nb) {
+    __shared__ double sh[4 * NV];
+    waveReduceAll<NV, NMAX>(acc, sh, threadIdx.x >> 6);
     __syncthreads();
-    if (threadIdx.x < NV) {
-        const int i = threadIdx.x;
-        double r = sh[i][0];
-        for (int k = 1; k < kBlock / 64; ++k) r = ((maxMask >> i) & 1u) ? nanMax(r, sh[i][k]) : r + sh[i][k];
-        part[(size_t)i * nb + lb] = r;
+    if (threadIdx.x < NV) part[(size_t)(off + threadIdx.x) * nb + lb] = overWaves<NMAX>(sh, threadIdx.x);
+}
+
+// ---------------------------------------------------------------------------
+// The control block's path through the launch sequence.
+//
+// Every reducing kernel leaves block partials; the scalars they give (alpha,
+// beta, residual norms, convergence) are needed by the next kernel only.  Up
+// to kMergeTiles tiles per instance that kernel's workgroups each reduce the
+// partials themselves (same order, same bits in every workgroup), apply the
+// scalar step to a copy of the control block in LDS, and the instance's first
+// workgroup writes it to the next control block of the chain: no launch
+// between two kernels of the PCG.  Above that a one-workgroup finalize kernel
+// (k_fin) does it in place.  Measured at 5,000 cells (20 tiles), FP64 diagonal
+// PCG: 20.2 us per iteration with finalize kernels, 11.3 us merged.
+// ---------------------------------------------------------------------------
+struct Stage {
+    const Ctl* in;  // control blocks left by the previous kernel of the chain
+    Ctl* out;       // where the resolved ones go
+    double* hist;   // per-outer-iteration history (may be null)
+};
+
+// points of the launch sequence at which scalars are resolved
+enum Point {
+    kPtGrad = 0,    // before the gradient step: PCG convergence; may the outer step run?
+    kPtRes = 1,     // before the residual: solidModel::converged, next outer iteration
+    kPtInner = 2,   // before the first PCG iteration of a pass: PCG start (normFactor, initial residual)
+    kPtAgain = 3,   // before a further one: the previous iteration's convergence
+    kPtSpmv = 4,    // before the matrix product of a multigrid PCG: beta
+    kPtUpdate = 5,  // before the solution update: alpha
+    kPtSettle = 6   // PCG convergence only (the tile map is about to change, or the host reads the state)
+};
+
+static_assert(sizeof(Ctl) % 8 == 0 && sizeof(Ctl) / 8 <= 64, "control block copied by one wavefront");
+
+// The scalar steps run on lanes 0..2 of a workgroup's first wavefront, one per
+// component (j), on the LDS copy of the control block; what concerns the
+// instance as a whole follows on lane 0.
+
+// PCG::solve start: normFactor (lduMatrix::solver::normFactor), normalised
+// initial residual, convergence check before the first iteration, z.r
+__device__ __forceinline__ void finResidual(Ctl* c, const double* tot, int j) {
+    const double nf = tot[3 + j] + tot[6 + j] + 1e-20;
+    const bool solved = (c->solveMask >> j) & 1;  // fvMatrix::solveSegregated valid components
+    const double ir = solved ? tot[j] / nf : 0.0;
+    c->normFactor[j] = nf;
+    c->initRes[j] = ir;
+    c->finalRes[j] = ir;
+    c->rho[j] = tot[9 + j];
+    c->nIter[j] = 0;
+    c->alpha[j] = 0.0;
+    c->beta[j] = 0.0;
+    // iterate unless already converged (finalRes = initRes < tolerance)
+    const int act = solved && (c->pcgMaxIter > 0) && !(ir < c->pcgTol);
+    c->active[j] = act;
+    const bool any = __ballot(act) != 0;
+    const double ir1 = __shfl(ir, 1), ir2 = __shfl(ir, 2);
+    if (j == 0) {
+        c->initResMag = sqrt(ir * ir + ir1 * ir1 + ir2 * ir2);
+        c->innerDone = !any;
+        c->firstInner = 1;
+        c->pIt = 0;
+        c->pending = kPendNone;
     }
 }
+
+// PCG convergence per component (tolerance, relTol, maxIter) and beta
+__device__ __forceinline__ void finUpdate(Ctl* c, const double* tot, int j) {
+    int act = c->active[j];
+    const int did = act;
+    if (act) {
+        const int n = c->nIter[j] + 1;
+        const double fr = tot[3 + j] / c->normFactor[j];
+        c->nIter[j] = n;
+        c->finalRes[j] = fr;
+        const bool conv = fr < c->pcgTol || (c->pcgRelTol > 1e-20 && fr < c->pcgRelTol * c->initRes[j]);
+        act = !conv && n < c->pcgMaxIter;
+        if (c->pcMode == 0) {  // diagonal preconditioner: z.r came with the update
+            c->beta[j] = tot[j] / c->rho[j];
+            c->rho[j] = tot[j];
+        }
+        c->active[j] = act;
+    }
+    const bool any = __ballot(act) != 0;
+    const int count = __popcll(__ballot(did));
+    if (j == 0) {
+        c->innerTotal += count;
+        c->innerDone = !any;
+        c->firstInner = 0;
+        c->pIt += 1;
+        c->pending = kPendNone;
+    }
+}
+
+// alpha = rho / p.q, with PCG's singularity test |p.q|/normFactor < VSMALL
+__device__ __forceinline__ void finSpmv(Ctl* c, const double* tot, int j) {
+    int act = c->active[j];
+    double al = 0.0;
+    if (act) {
+        if (fabs(tot[j]) / c->normFactor[j] < kVSmall) {
+            act = 0;
+            c->active[j] = 0;
+        } else {
+            al = c->rho[j] / tot[j];
+        }
+    }
+    c->alpha[j] = al;
+    const bool any = __ballot(act) != 0;
+    if (j == 0) {
+        if (!any) c->innerDone = 1;
+        c->pending = any ? kPendUpd : kPendNone;
+    }
+}
+
+// rho' = z.r of a V-cycle-preconditioned PCG: beta = rho'/rho (first
+// iteration: no beta), rho = rho'
+__device__ __forceinline__ void finRho(Ctl* c, const double* tot, int j) {
+    if (c->active[j]) {
+        c->beta[j] = c->firstInner ? 0.0 : tot[j] / c->rho[j];
+        c->rho[j] = tot[j];
+    }
+    if (j == 0) c->pending = kPendSpmv;
+}
+
+// solidModel::converged (total-displacement form) and the mean field for the
+// next normFactor
+__device__ __forceinline__ void finGrad(Ctl* c, const double* tot, double nc, int inst, double* hist, int j) {
+    c->xbar[j] = tot[3 + j] / nc;
+    if (j != 0) return;
+    c->dpar ^= 1;  // k_grad wrote D' into the other buffer
+    const double dmax = sqrt(tot[2]);  // the partials are squares: sqrt is monotonic
+    double denom = sqrt(tot[1]);
+    if (denom < kSmall) denom = dmax < kSmall ? kSmall : dmax;
+    const double rvf = sqrt(tot[0]) / denom;
+    const double ir = c->initResMag;
+    const int i = c->iCorr;
+    c->rvf = rvf;
+    const int n0 = c->nIter[0], n1 = c->nIter[1], n2 = c->nIter[2];
+    const int n01 = n0 > n1 ? n0 : n1;
+    c->pcgTotal += n01 > n2 ? n01 : n2;
+    const bool conv = i > 1 && ((ir < c->solTol && rvf < c->solTol) || rvf < c->altTol || ir < c->altTol);
+    if (hist && i < c->histCap) {
+        double* h = hist + (size_t)inst * 3 * c->histCap;
+        h[i] = ir;
+        h[c->histCap + i] = rvf;
+        h[2 * c->histCap + i] = (double)(n0 + n1 + n2);
+    }
+    int done = 1;
+    if (!isfinite(ir) || !isfinite(rvf)) c->diverged = 1;
+    else if (conv) c->converged = 1;
+    else if (i + 1 < c->nCorr) done = 0;
+    if (done) {
+        c->outerDone = 1;
+        c->nOuter = i + 1;
+    } else {
+        c->iCorr = i + 1;
+    }
+    c->pending = done ? kPendNone : kPendRes;
+}
+
+// the PCG has finished: mixed precision's stall test (an |initRes| with no new
+// minimum 1 % below the last one within the window stops the instance here),
+// then the outer step may run
+__device__ __forceinline__ void innerEnd(Ctl* c) {
+    if (c->outerDone || !c->innerDone || c->pending != kPendNone || c->hold) return;
+    if (c->stallWindow > 0 && c->iCorr >= 2) {
+        if (c->initResMag < 0.99 * c->bestRes) {
+            c->bestRes = c->initResMag;
+            c->bestIt = c->iCorr;
+        } else if (c->iCorr - c->bestIt >= c->stallWindow) {
+            c->stalled = 1;
+            c->hold = 1;
+            return;
+        }
+    }
+    c->pending = kPendGrad;
+}
+
+// what a point of the launch sequence reduces: the pending step, its partials
+template <int POINT> struct PointOf;
+template <> struct PointOf<kPtGrad> { enum { pend = kPendUpd, off = kOffUpd, nv = 6, nmax = 0 }; };
+template <> struct PointOf<kPtRes> { enum { pend = kPendGrad, off = kOffGrad, nv = 6, nmax = 3 }; };
+template <> struct PointOf<kPtInner> { enum { pend = kPendRes, off = kOffRes, nv = 12, nmax = 0 }; };
+template <> struct PointOf<kPtAgain> { enum { pend = kPendUpd, off = kOffUpd, nv = 6, nmax = 0 }; };
+template <> struct PointOf<kPtSpmv> { enum { pend = kPendRho, off = kOffRho, nv = 3, nmax = 0 }; };
+template <> struct PointOf<kPtUpdate> { enum { pend = kPendSpmv, off = kOffSpmv, nv = 3, nmax = 0 }; };
+template <> struct PointOf<kPtSettle> { enum { pend = kPendUpd, off = kOffUpd, nv = 6, nmax = 0 }; };
+
+// A kernel's passage through its point, in three parts so that its own loads
+// can be in flight meanwhile:
+//   load()    the control block's words and this thread's first partial row
+//   reduce()  the control block in LDS and the reduced partials (one barrier)
+//   finish()  the scalar step, the instance's first workgroup stores the
+//             result (one barrier)
+template <int POINT>
+struct StageRun {
+    typedef PointOf<POINT> Pt;
+    long long word;
+    double v[Pt::nv];
+    __device__ __forceinline__ void load(const Ctl* in, const double* __restrict__ part, int nb, int blk0, int nblk) {
+        constexpr int n = (int)(sizeof(Ctl) / 8);
+        word = (int)threadIdx.x < n ? reinterpret_cast<const long long*>(in)[threadIdx.x] : 0;
+        const double* col = part + (size_t)Pt::off * nb + blk0 + threadIdx.x;
+#pragma unroll
+        for (int i = 0; i < Pt::nv; ++i) v[i] = (int)threadIdx.x < nblk ? col[(size_t)i * nb] : 0.0;
+    }
+    __device__ __forceinline__ void reduce(Ctl* sh, double* tot, const double* __restrict__ part, int nb, int blk0,
+                                           int nblk) {
+        constexpr int n = (int)(sizeof(Ctl) / 8);
+        if ((int)threadIdx.x < n) reinterpret_cast<long long*>(sh)[threadIdx.x] = word;
+        const double* col = part + (size_t)Pt::off * nb + blk0;
+        for (int b = threadIdx.x + kFinBlock; b < nblk; b += kFinBlock)
+#pragma unroll
+            for (int i = 0; i < Pt::nv; ++i) {
+                const double x = col[(size_t)i * nb + b];
+                v[i] = i < Pt::nmax ? nanMax(v[i], x) : v[i] + x;
+            }
+        const int w = waveOf();
+        if (w == 0 || nblk > 64) waveReduceAll<Pt::nv, Pt::nmax>(v, tot, w);
+        else if ((int)(threadIdx.x & 63) < Pt::nv) tot[4 * (threadIdx.x & 63) + w] = 0.0;  // no rows here
+        __syncthreads();
+    }
+    // tot[4 i + w]: wavefront w's share of value i
+    __device__ __forceinline__ void finish(Ctl* sh, const double* tot, const Tile& tl, double* hist, bool first,
+                                           Ctl* out) {
+        if (threadIdx.x < 3) {
+            const int j = threadIdx.x;
+            const int pend = sh->pending;
+            if (pend == Pt::pend) {
+                double t[Pt::nv];
+#pragma unroll
+                for (int i = 0; i < Pt::nv; ++i) t[i] = overWaves<Pt::nmax>(tot, i);
+                step(sh, t, tl, hist, first, j);
+            } else if (POINT == kPtRes && pend == kPendStart) {
+                if (j == 0) sh->pending = kPendRes;
+            }
+            if (j == 0) {
+                if (POINT == kPtGrad) innerEnd(sh);
+                if ((POINT == kPtInner || POINT == kPtAgain) && !sh->outerDone && !sh->innerDone &&
+                    sh->pending == kPendNone)
+                    sh->pending = sh->pcMode ? kPendRho : kPendSpmv;
+            }
+        }
+        __syncthreads();
+        if (out && first) {
+            constexpr int n = (int)(sizeof(Ctl) / 8);
+            if ((int)threadIdx.x < n)
+                reinterpret_cast<long long*>(out)[threadIdx.x] = reinterpret_cast<const long long*>(sh)[threadIdx.x];
+        }
+    }
+    __device__ __forceinline__ static void step(Ctl* sh, const double* t, const Tile& tl, double* hist, bool first,
+                                                int j) {
+        if constexpr (POINT == kPtRes) finGrad(sh, t, (double)tl.nCell, tl.inst, first ? hist : nullptr, j);
+        else if constexpr (POINT == kPtInner) finResidual(sh, t, j);
+        else if constexpr (POINT == kPtSpmv) finRho(sh, t, j);
+        else if constexpr (POINT == kPtUpdate) finSpmv(sh, t, j);
+        else finUpdate(sh, t, j);
+    }
+};
+
+__device__ __forceinline__ int pendingOf(const Ctl* c) { return __builtin_amdgcn_readfirstlane(c->pending); }
 
 // linearElastic: sigma = 2 mu dev(symm G) + K tr(symm G) I   (xx xy xz yy yz zz)
 __device__ __forceinline__ void hooke(const double* G, double mu, double K, double* s) {
@@ -207,17 +528,18 @@ __device__ __forceinline__ void residualInternal(const DevMesh& m, int P, int e0
 
 // ---------------------------------------------------------------------------
 // k_residual: R = div(sigma) + RhieChow (integrated), r = R, and per-workgroup
-// partials of sum|R|, the two normFactor sums and z.r (k_fin_residual).
+// partials of sum|R|, the two normFactor sums and z.r (finResidual).
 // ---------------------------------------------------------------------------
 template <typename T>
 __global__ __launch_bounds__(kBlock) void k_residual(const DevMesh m, const BlockMap bm, const double* __restrict__ D0,
                                                      const double* __restrict__ D1, const double* __restrict__ G, const double* __restrict__ sigb,
-                                                     T* __restrict__ r, Ctl* __restrict__ ctlAll,
+                                                     T* __restrict__ r, const Ctl* __restrict__ ctlAll,
                                                      double* __restrict__ part) {
     const int lb = logicalBlock(bm.nBlocks);
-    const int inst = bm.inst[lb];
-    Ctl* ctl = ctlAll + inst;
-    if (ctl->outerDone) return;
+    const Tile tl = bm.at(lb);
+    const int inst = tl.inst;
+    const Ctl* ctl = ctlAll + inst;
+    if (ctl->pending != kPendRes) return;
     const double* __restrict__ D = ctl->dpar ? D1 : D0;
     const int C = m.nCells;
     const double xb0 = ctl->xbar[0], xb1 = ctl->xbar[1], xb2 = ctl->xbar[2];
@@ -229,13 +551,11 @@ __global__ __launch_bounds__(kBlock) void k_residual(const DevMesh m, const Bloc
     for (int i = 0; i < 12; ++i) acc[i] = 0.0;
     const T* __restrict__ invD = MatSel<T>::invDiag(m);
     const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
-    const int s1 = bm.s1[lb];
-    const int cEnd = bm.iCell0[inst] + bm.iNCell[inst];
-    for (int s = bm.s0[lb] + wave; s < s1; s += kBlock / 64) {
+    for (int s = tl.s0 + wave; s < tl.s1; s += kBlock / 64) {
         const int P = s * kSlice + lane;
-        const int e0 = m.sliceStart[s];
-        const int width = m.sliceWidth[s];
-        if (P >= cEnd) continue;
+        const int width = m.width(s);
+        const int e0 = m.entry0(s);
+        if (P >= tl.cEnd) continue;
         double DP[3], GP[9], CP[3], sP[6];
 #pragma unroll
         for (int k = 0; k < 3; ++k) { DP[k] = D[(size_t)k * C + P]; CP[k] = m.cC[(size_t)k * C + P]; }
@@ -284,7 +604,7 @@ __global__ __launch_bounds__(kBlock) void k_residual(const DevMesh m, const Bloc
             acc[9 + j] += (double)z * (double)rT;
         }
     }
-    storeBlockPartials<12>(acc, 0u, part, lb, bm.nBlocks);
+    storeBlockPartials<12, 0>(acc, part, kOffRes, lb, bm.nBlocks);
 }
 
 // Row of the fused direction update + SpMV with all three components active
@@ -345,13 +665,18 @@ __device__ __forceinline__ void spmvpRowAll(const DevMesh& m, int P, int e0, int
 // ---------------------------------------------------------------------------
 template <typename T, bool MG>
 __global__ __launch_bounds__(kBlock) void k_spmvp(const DevMesh m, const BlockMap bm, const T* __restrict__ r,
-                                                  const T* __restrict__ pOld, T* __restrict__ pNew, T* __restrict__ q,
-                                                  Ctl* __restrict__ ctlAll, double* __restrict__ part, int reduce,
+                                                  T* pA, T* pB, T* __restrict__ q, const Ctl* __restrict__ ctlAll,
+                                                  double* __restrict__ part, int reduce,
                                                   const T* __restrict__ zArr) {
     const int lb = logicalBlock(bm.nBlocks);
-    const int inst = bm.inst[lb];
+    const Tile tl = bm.at(lb);
+    const int inst = tl.inst;
     const Ctl* ctl = ctlAll + inst;
-    if (reduce && (ctl->outerDone || ctl->innerDone)) return;
+    if (reduce && ctl->pending != kPendSpmv) return;
+    // the two direction buffers alternate with the PCG iteration
+    const bool odd = reduce && (ctl->pIt & 1);
+    const T* __restrict__ pOld = odd ? pB : pA;
+    T* __restrict__ pNew = odd ? pA : pB;
     const int C = m.nCells;
     const T* __restrict__ A = MatSel<T>::a(m);
     const T* __restrict__ dg = MatSel<T>::diag(m);
@@ -370,13 +695,11 @@ __global__ __launch_bounds__(kBlock) void k_spmvp(const DevMesh m, const BlockMa
     };
     double acc[3] = {0, 0, 0};
     const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
-    const int s1 = bm.s1[lb];
-    const int cEnd = bm.iCell0[inst] + bm.iNCell[inst];
-    for (int s = bm.s0[lb] + wave; s < s1; s += kBlock / 64) {
+    for (int s = tl.s0 + wave; s < tl.s1; s += kBlock / 64) {
         const int P = s * kSlice + lane;
-        const int e0 = m.sliceStart[s];
-        const int width = m.sliceWidth[s];
-        if (P >= cEnd) continue;
+        const int width = m.width(s);
+        const int e0 = m.entry0(s);
+        if (P >= tl.cEnd) continue;
         if (all && width == 6) {
             spmvpRowAll<T, 6, MG>(m, P, e0, lane, C, r, pOld, zArr, pNew, q, first, be, acc);
             continue;
@@ -412,7 +735,7 @@ __global__ __launch_bounds__(kBlock) void k_spmvp(const DevMesh m, const BlockMa
         }
     }
     if (!reduce) return;
-    storeBlockPartials<3>(acc, 0u, part, lb, bm.nBlocks);
+    storeBlockPartials<3, 0>(acc, part, kOffSpmv, lb, bm.nBlocks);
 }
 
 // ---------------------------------------------------------------------------
@@ -420,12 +743,16 @@ __global__ __launch_bounds__(kBlock) void k_spmvp(const DevMesh m, const BlockMa
 // ---------------------------------------------------------------------------
 template <typename T>
 __global__ __launch_bounds__(kBlock) void k_update(const DevMesh m, const BlockMap bm, T* __restrict__ x,
-                                                   const T* __restrict__ p, T* __restrict__ r, const T* __restrict__ q,
+                                                   const T* __restrict__ pA, const T* __restrict__ pB,
+                                                   T* __restrict__ r, const T* __restrict__ q,
                                                    const Ctl* __restrict__ ctlAll, double* __restrict__ part) {
     const int lb = logicalBlock(bm.nBlocks);
-    const int inst = bm.inst[lb];
+    const Tile tl = bm.at(lb);
+    const int inst = tl.inst;
     const Ctl* ctl = ctlAll + inst;
-    if (ctl->outerDone || ctl->innerDone) return;
+    if (ctl->pending != kPendUpd) return;
+    // the direction k_spmvp wrote
+    const T* __restrict__ p = (ctl->pIt & 1) ? pA : pB;
     const int C = m.nCells;
     const T* __restrict__ invD = MatSel<T>::invDiag(m);
     const T al[3] = {(T)ctl->alpha[0], (T)ctl->alpha[1], (T)ctl->alpha[2]};
@@ -433,11 +760,9 @@ __global__ __launch_bounds__(kBlock) void k_update(const DevMesh m, const BlockM
     const int first = ctl->firstInner;
     double acc[6] = {0, 0, 0, 0, 0, 0};
     const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
-    const int s1 = bm.s1[lb];
-    const int cEnd = bm.iCell0[inst] + bm.iNCell[inst];
-    for (int s = bm.s0[lb] + wave; s < s1; s += kBlock / 64) {
+    for (int s = tl.s0 + wave; s < tl.s1; s += kBlock / 64) {
         const int P = s * kSlice + lane;
-        if (P >= cEnd) continue;
+        if (P >= tl.cEnd) continue;
         const T iD = invD[P];
 #pragma unroll
         for (int j = 0; j < 3; ++j) {
@@ -455,7 +780,7 @@ __global__ __launch_bounds__(kBlock) void k_update(const DevMesh m, const BlockM
             acc[3 + j] += fabs((double)rv);
         }
     }
-    storeBlockPartials<6>(acc, 0u, part, lb, bm.nBlocks);
+    storeBlockPartials<6, 0>(acc, part, kOffUpd, lb, bm.nBlocks);
 }
 
 // Internal-face slots of the least-squares gradient sum with compile-time
@@ -507,7 +832,13 @@ __device__ __forceinline__ void gradInternalW(const DevMesh& m, int P, int e0, i
 // update: k_grad_bnd_pre is not launched, k_grad_bnd_post leaves g).
 // The face kernels run one workgroup row (blockIdx.y) per instance over that
 // instance's boundary faces; empty faces carry no value and are skipped.
+// Merged launch sequences run the three as one kernel (k_grad_m).
 // ---------------------------------------------------------------------------
+// boundary fields of the fused gradient step
+struct BndBufs {
+    double *g, *snb, *Gb, *sigb;
+};
+
 __device__ __forceinline__ int faceInst(const BlockMap& bm) {
     return bm.finInst ? bm.finInst[blockIdx.y] : (int)blockIdx.y;
 }
@@ -540,9 +871,10 @@ __global__ __launch_bounds__(kBlock) void k_aitken(const DevMesh m, const BlockM
                                                    double* __restrict__ alpha, double* __restrict__ res,
                                                    const Ctl* __restrict__ ctlAll) {
     const int lb = logicalBlock(bm.nBlocks);
-    const int inst = bm.inst[lb];
+    const Tile tl = bm.at(lb);
+    const int inst = tl.inst;
     const Ctl* ctl = ctlAll + inst;
-    if (ctl->outerDone) return;
+    if (ctl->pending != kPendGrad) return;
     if (ctl->firstInner) x = nullptr;
     const double* D = ctl->dpar ? D1 : D0;
     double* Dn = ctl->dpar ? D0 : D1;
@@ -550,11 +882,9 @@ __global__ __launch_bounds__(kBlock) void k_aitken(const DevMesh m, const BlockM
     const double a0 = ctl->relaxD;
     const int C = m.nCells;
     const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
-    const int s1 = bm.s1[lb];
-    const int cEnd = bm.iCell0[inst] + bm.iNCell[inst];
-    for (int s = bm.s0[lb] + wave; s < s1; s += kBlock / 64) {
+    for (int s = tl.s0 + wave; s < tl.s1; s += kBlock / 64) {
         const int P = s * kSlice + lane;
-        if (P >= cEnd) continue;
+        if (P >= tl.cEnd) continue;
         double Ds[3], r[3];
 #pragma unroll
         for (int k = 0; k < 3; ++k) {
@@ -568,6 +898,149 @@ __global__ __launch_bounds__(kBlock) void k_aitken(const DevMesh m, const BlockM
     }
 }
 
+// Settings of an instance's boundary update, the same for all of its faces.
+struct BndStep {
+    int mode;
+    bool aitken, relax, first;
+    double ra, a0;
+};
+__device__ __forceinline__ BndStep bndStep(const Ctl* ctl, int mode) {
+    BndStep u;
+    u.mode = mode;
+    u.aitken = mode == 0 && ctl->relaxAitken;
+    u.relax = mode == 0 && !u.aitken && ctl->relaxD != 1.0;
+    u.ra = u.relax ? ctl->relaxD : 1.0;
+    u.first = ctl->iCorr == 0;
+    u.a0 = ctl->relaxD;
+    return u;
+}
+
+// Boundary value Dbv and snGrad sn of face b (type != empty) of a cell with
+// updated displacement DuP (the solve's D + x), relaxed displacement DnP and
+// previous gradient Gold
+__device__ __forceinline__ void bndPreFace(const DevMesh& m, const BndStep& u, int b, int type, const double* DuP,
+                                           const double* DnP, const double* Gold, const double* Db, const double* g,
+                                           double* alphaB, double* resB, double* Dbv, double* sn) {
+    const int mode = u.mode, B = m.nBoundary;
+    const bool aitken = u.aitken, relax = u.relax, first = u.first;
+    const double ra = u.ra;
+    const double k0 = m.bKv[b], k1 = m.bKv[(size_t)B + b], k2 = m.bKv[2 * (size_t)B + b];
+    const double dl = m.bDelta[b];
+    const bool trac = type == 1;
+    const bool sym = type == 3;
+    const bool zs = type == 4;
+    // solidSymmetry (first order, normal patch delta so no k correction):
+    // value D_P - n (n.D_P) after the solve (relaxed like every boundary
+    // value), snGrad -n (n.D_P) deltaCoeffs from the relaxed cell value
+    const double nb0 = m.bN[b], nb1 = m.bN[(size_t)B + b], nb2 = m.bN[2 * (size_t)B + b];
+    const double nDu = nb0 * DuP[0] + nb1 * DuP[1] + nb2 * DuP[2];
+    const double nDn = nb0 * DnP[0] + nb1 * DnP[1] + nb2 * DnP[2];
+    const double nbv[3] = {nb0, nb1, nb2};
+    double kGv[3], gvv[3];
+#pragma unroll
+    for (int j = 0; j < 3; ++j) {
+        kGv[j] = k0 * Gold[j] + k1 * Gold[3 + j] + k2 * Gold[6 + j];
+        gvv[j] = (mode == 1 || !(trac || zs)) ? 0.0 : g[(size_t)j * B + b];
+    }
+    // fixedDisplacementZeroShear (direction-mixed, valueFraction nn, first
+    // order): n (n.Dbar) + (I - nn).(D_P + k.G_P + g/deltaCoeffs), the value
+    // from the solved cell value, the snGrad from the relaxed one
+    double zu[3] = {0, 0, 0}, zn[3] = {0, 0, 0};
+    if (zs) {
+        double gu[3], gn[3];
+#pragma unroll
+        for (int j = 0; j < 3; ++j) {
+            gu[j] = DuP[j] + kGv[j] + gvv[j] / dl;
+            gn[j] = DnP[j] + kGv[j] + gvv[j] / dl;
+        }
+        const double nD = nb0 * m.bVal[b] + nb1 * m.bVal[(size_t)B + b] + nb2 * m.bVal[2 * (size_t)B + b];
+        const double ngu = nb0 * gu[0] + nb1 * gu[1] + nb2 * gu[2];
+        const double ngn = nb0 * gn[0] + nb1 * gn[1] + nb2 * gn[2];
+#pragma unroll
+        for (int j = 0; j < 3; ++j) {
+            zu[j] = nbv[j] * nD + (gu[j] - nbv[j] * ngu);
+            zn[j] = nbv[j] * nD + (gn[j] - nbv[j] * ngn);
+        }
+    }
+    // correctBoundaryConditions after the solve, then relaxField on the
+    // patch values (fixed values stay); the snGrads follow the relaxed cell
+#pragma unroll
+    for (int j = 0; j < 3; ++j) {
+        const double kG = kGv[j];
+        if (zs) {
+            Dbv[j] = zu[j];
+            sn[j] = (zn[j] - (DnP[j] + kG)) * dl;
+        } else if (sym) {
+            Dbv[j] = DuP[j] - nbv[j] * nDu;
+            sn[j] = -nbv[j] * nDn * dl;
+        } else if (trac) {
+            Dbv[j] = DuP[j] + kG + gvv[j] / dl;
+            sn[j] = gvv[j];
+        } else {
+            Dbv[j] = m.bVal[(size_t)j * B + b];
+            sn[j] = (Dbv[j] - (DnP[j] + kG)) * dl;
+        }
+    }
+    if (type != 0 && (relax || aitken)) {
+        double Dbp[3];
+#pragma unroll
+        for (int j = 0; j < 3; ++j) Dbp[j] = Db[(size_t)j * B + b];
+        if (aitken) {
+            const double r[3] = {Dbp[0] - Dbv[0], Dbp[1] - Dbv[1], Dbp[2] - Dbv[2]};
+            const double al = aitkenFactor(r, alphaB, resB, b, B, first, u.a0);
+#pragma unroll
+            for (int j = 0; j < 3; ++j) Dbv[j] -= al * r[j];
+        } else {
+#pragma unroll
+            for (int j = 0; j < 3; ++j) Dbv[j] = Dbp[j] + ra * (Dbv[j] - Dbp[j]);
+        }
+    }
+}
+
+// Boundary gradient and stress of face b from the cell gradient Gn and the
+// face's snGrad, and the next traction snGrad
+__device__ __forceinline__ void bndPostFace(const DevMesh& m, int mode, bool zeroStress, int b, int type, int P,
+                                            const double* Gn, const double* __restrict__ snb, double* __restrict__ Gb,
+                                            double* __restrict__ sigb, double* __restrict__ g) {
+    const int B = m.nBoundary;
+    const double nv[3] = {m.bN[b], m.bN[(size_t)B + b], m.bN[2 * (size_t)B + b]};
+    double Gbv[9], sb[6];
+#pragma unroll
+    for (int j = 0; j < 3; ++j) {
+        const double nG = nv[0] * Gn[j] + nv[1] * Gn[3 + j] + nv[2] * Gn[6 + j];
+        const double sn = snb[(size_t)j * B + b];
+#pragma unroll
+        for (int i = 0; i < 3; ++i) Gbv[3 * i + j] = Gn[3 * i + j] + nv[i] * (sn - nG);
+    }
+    hooke(Gbv, cellMu(m, P), cellK(m, P), sb);
+    if (zeroStress) {  // cold start: the stress field is still zero
+#pragma unroll
+        for (int q = 0; q < 6; ++q) sb[q] = 0.0;
+    }
+    if (Gb) {
+#pragma unroll
+        for (int q = 0; q < 9; ++q) Gb[(size_t)q * B + b] = Gbv[q];
+    }
+#pragma unroll
+    for (int q = 0; q < 6; ++q) sigb[(size_t)q * B + b] = sb[q];
+    if (mode != 2 && (type == 1 || type == 4)) {
+        // fixedDisplacementZeroShear: the traction snGrad for zero
+        // traction and pressure (its shear-free refGrad)
+        const bool zs = type == 4;
+        const double ik = cellImpK(m, P);
+        const double Tt[9] = {sb[0] - ik * Gbv[0], sb[1] - ik * Gbv[1], sb[2] - ik * Gbv[2],
+                              sb[1] - ik * Gbv[3], sb[3] - ik * Gbv[4], sb[4] - ik * Gbv[5],
+                              sb[2] - ik * Gbv[6], sb[4] - ik * Gbv[7], sb[5] - ik * Gbv[8]};
+        const double rik = 1.0 / ik;
+        const double pr = zs ? 0.0 : m.bPres[b];
+#pragma unroll
+        for (int j = 0; j < 3; ++j) {
+            const double nT = nv[0] * Tt[j] + nv[1] * Tt[3 + j] + nv[2] * Tt[6 + j];
+            g[(size_t)j * B + b] = (zs ? -nT : (m.bVal[(size_t)j * B + b] - nv[j] * pr) - nT) * rik;
+        }
+    }
+}
+
 template <typename T>
 __global__ __launch_bounds__(kBlock) void k_grad_bnd_pre(const DevMesh m, const BlockMap bm,
                                                          const double* __restrict__ D0, const T* __restrict__ x,
@@ -578,15 +1051,12 @@ __global__ __launch_bounds__(kBlock) void k_grad_bnd_pre(const DevMesh m, const 
                                                          int mode) {
     const int inst = faceInst(bm);
     const Ctl* ctl = ctlAll + inst;
-    if (mode == 0 && ctl->outerDone) return;
+    if (mode == 0 && ctl->pending != kPendGrad) return;
     if (mode == 0 && ctl->firstInner) x = nullptr;  // no PCG iteration ran: the update is zero
     const double* __restrict__ D = ctl->dpar ? D1 : D0;
     // Aitken: the relaxed cell values are in the buffer receiving D' (k_aitken)
-    const bool aitken = mode == 0 && ctl->relaxAitken;
+    const BndStep u = bndStep(ctl, mode);
     const double* __restrict__ Dr = ctl->dpar ? D0 : D1;
-    const bool relax = mode == 0 && !aitken && ctl->relaxD != 1.0;
-    const double ra = relax ? ctl->relaxD : 1.0;
-    const bool first = ctl->iCorr == 0;
     const int C = m.nCells, B = m.nBoundary;
     const int b0 = bm.iB0[inst], b1 = b0 + bm.iNB[inst];
     for (int b = b0 + blockIdx.x * kBlock + threadIdx.x; b < b1; b += gridDim.x * kBlock) {
@@ -601,82 +1071,12 @@ __global__ __launch_bounds__(kBlock) void k_grad_bnd_pre(const DevMesh m, const 
             const double DP = D[(size_t)k * C + P];
             const double xv = x ? (double)x[(size_t)k * C + P] : 0.0;
             DuP[k] = DP + xv;
-            DnP[k] = aitken ? Dr[(size_t)k * C + P] : DP + ra * xv;
+            DnP[k] = u.aitken ? Dr[(size_t)k * C + P] : DP + u.ra * xv;
         }
 #pragma unroll
         for (int q = 0; q < 9; ++q) Gold[q] = (mode == 1) ? 0.0 : G[(size_t)q * C + P];
-        const double k0 = m.bKv[b], k1 = m.bKv[(size_t)B + b], k2 = m.bKv[2 * (size_t)B + b];
-        const double dl = m.bDelta[b];
-        const bool trac = type == 1;
-        const bool sym = type == 3;
-        const bool zs = type == 4;
-        // solidSymmetry (first order, normal patch delta so no k correction):
-        // value D_P - n (n.D_P) after the solve (relaxed like every boundary
-        // value), snGrad -n (n.D_P) deltaCoeffs from the relaxed cell value
-        const double nb0 = m.bN[b], nb1 = m.bN[(size_t)B + b], nb2 = m.bN[2 * (size_t)B + b];
-        const double nDu = nb0 * DuP[0] + nb1 * DuP[1] + nb2 * DuP[2];
-        const double nDn = nb0 * DnP[0] + nb1 * DnP[1] + nb2 * DnP[2];
-        const double nbv[3] = {nb0, nb1, nb2};
-        double kGv[3], gvv[3];
-#pragma unroll
-        for (int j = 0; j < 3; ++j) {
-            kGv[j] = k0 * Gold[j] + k1 * Gold[3 + j] + k2 * Gold[6 + j];
-            gvv[j] = (mode == 1 || !(trac || zs)) ? 0.0 : g[(size_t)j * B + b];
-        }
-        // fixedDisplacementZeroShear (direction-mixed, valueFraction nn, first
-        // order): n (n.Dbar) + (I - nn).(D_P + k.G_P + g/deltaCoeffs), the value
-        // from the solved cell value, the snGrad from the relaxed one
-        double zu[3] = {0, 0, 0}, zn[3] = {0, 0, 0};
-        if (zs) {
-            double gu[3], gn[3];
-#pragma unroll
-            for (int j = 0; j < 3; ++j) {
-                gu[j] = DuP[j] + kGv[j] + gvv[j] / dl;
-                gn[j] = DnP[j] + kGv[j] + gvv[j] / dl;
-            }
-            const double nD = nb0 * m.bVal[b] + nb1 * m.bVal[(size_t)B + b] + nb2 * m.bVal[2 * (size_t)B + b];
-            const double ngu = nb0 * gu[0] + nb1 * gu[1] + nb2 * gu[2];
-            const double ngn = nb0 * gn[0] + nb1 * gn[1] + nb2 * gn[2];
-#pragma unroll
-            for (int j = 0; j < 3; ++j) {
-                zu[j] = nbv[j] * nD + (gu[j] - nbv[j] * ngu);
-                zn[j] = nbv[j] * nD + (gn[j] - nbv[j] * ngn);
-            }
-        }
-        // correctBoundaryConditions after the solve, then relaxField on the
-        // patch values (fixed values stay); the snGrads follow the relaxed cell
         double Dbv[3], sn[3];
-#pragma unroll
-        for (int j = 0; j < 3; ++j) {
-            const double kG = kGv[j];
-            if (zs) {
-                Dbv[j] = zu[j];
-                sn[j] = (zn[j] - (DnP[j] + kG)) * dl;
-            } else if (sym) {
-                Dbv[j] = DuP[j] - nbv[j] * nDu;
-                sn[j] = -nbv[j] * nDn * dl;
-            } else if (trac) {
-                Dbv[j] = DuP[j] + kG + gvv[j] / dl;
-                sn[j] = gvv[j];
-            } else {
-                Dbv[j] = m.bVal[(size_t)j * B + b];
-                sn[j] = (Dbv[j] - (DnP[j] + kG)) * dl;
-            }
-        }
-        if (type != 0 && (relax || aitken)) {
-            double Dbp[3];
-#pragma unroll
-            for (int j = 0; j < 3; ++j) Dbp[j] = Db[(size_t)j * B + b];
-            if (aitken) {
-                const double r[3] = {Dbp[0] - Dbv[0], Dbp[1] - Dbv[1], Dbp[2] - Dbv[2]};
-                const double al = aitkenFactor(r, alphaB, resB, b, B, first, ctl->relaxD);
-#pragma unroll
-                for (int j = 0; j < 3; ++j) Dbv[j] -= al * r[j];
-            } else {
-#pragma unroll
-                for (int j = 0; j < 3; ++j) Dbv[j] = Dbp[j] + ra * (Dbv[j] - Dbp[j]);
-            }
-        }
+        bndPreFace(m, u, b, type, DuP, DnP, Gold, Db, g, alphaB, resB, Dbv, sn);
 #pragma unroll
         for (int j = 0; j < 3; ++j) {
             Db[(size_t)j * B + b] = Dbv[j];
@@ -690,11 +1090,12 @@ __global__ __launch_bounds__(kBlock) void k_grad(const DevMesh m, const BlockMap
                                                  const T* __restrict__ x, double* __restrict__ D1,
                                                  double* __restrict__ G, const double* __restrict__ Db,
                                                  const double* __restrict__ DI, const double* __restrict__ Dold,
-                                                 Ctl* __restrict__ ctlAll, double* __restrict__ part, int mode) {
+                                                 const Ctl* __restrict__ ctlAll, double* __restrict__ part, int mode) {
     const int lb = logicalBlock(bm.nBlocks);
-    const int inst = bm.inst[lb];
-    Ctl* ctl = ctlAll + inst;
-    if (mode == 0 && ctl->outerDone) return;
+    const Tile tl = bm.at(lb);
+    const int inst = tl.inst;
+    const Ctl* ctl = ctlAll + inst;
+    if (mode == 0 && ctl->pending != kPendGrad) return;
     if (mode == 0 && ctl->firstInner) x = nullptr;  // no PCG iteration ran: the update is zero
     // current field and the buffer receiving D' (per-instance ping-pong)
     const double* __restrict__ D = ctl->dpar ? D1 : D0;
@@ -707,15 +1108,13 @@ __global__ __launch_bounds__(kBlock) void k_grad(const DevMesh m, const BlockMap
     const double* Dg = aitken ? Dn : D;
     const T* xg = aitken ? nullptr : x;
     const int C = m.nCells, B = m.nBoundary;
-    double acc[6] = {0, 0, 0, 0, 0, 0};  // max|D'-D|, max|D'-Dold|, max|D'|, sum D'
+    double acc[6] = {0, 0, 0, 0, 0, 0};  // max|D'-D|^2, max|D'-Dold|^2, max|D'|^2, sum D'
     const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
-    const int s1 = bm.s1[lb];
-    const int cEnd = bm.iCell0[inst] + bm.iNCell[inst];
-    for (int s = bm.s0[lb] + wave; s < s1; s += kBlock / 64) {
+    for (int s = tl.s0 + wave; s < tl.s1; s += kBlock / 64) {
         const int P = s * kSlice + lane;
-        const int e0 = m.sliceStart[s];
-        const int width = m.sliceWidth[s];
-        if (P >= cEnd) continue;
+        const int width = m.width(s);
+        const int e0 = m.entry0(s);
+        if (P >= tl.cEnd) continue;
         double DP[3], DnP[3], CP[3];
 #pragma unroll
         for (int k = 0; k < 3; ++k) {
@@ -792,12 +1191,15 @@ __global__ __launch_bounds__(kBlock) void k_grad(const DevMesh m, const BlockMap
         }
         const double M0 = m.minv[P], M1 = m.minv[(size_t)C + P], M2 = m.minv[2 * (size_t)C + P];
         const double M3 = m.minv[3 * (size_t)C + P], M4 = m.minv[4 * (size_t)C + P], M5 = m.minv[5 * (size_t)C + P];
+        double Gn[9];
 #pragma unroll
         for (int j = 0; j < 3; ++j) {
-            stS(G + (size_t)j * C + P, M0 * A[j] + M1 * A[3 + j] + M2 * A[6 + j]);
-            stS(G + (size_t)(3 + j) * C + P, M1 * A[j] + M3 * A[3 + j] + M4 * A[6 + j]);
-            stS(G + (size_t)(6 + j) * C + P, M2 * A[j] + M4 * A[3 + j] + M5 * A[6 + j]);
+            Gn[j] = M0 * A[j] + M1 * A[3 + j] + M2 * A[6 + j];
+            Gn[3 + j] = M1 * A[j] + M3 * A[3 + j] + M4 * A[6 + j];
+            Gn[6 + j] = M2 * A[j] + M4 * A[3 + j] + M5 * A[6 + j];
         }
+#pragma unroll
+        for (int q = 0; q < 9; ++q) stS(G + (size_t)q * C + P, Gn[q]);
         if (Dn && !aitken) {
 #pragma unroll
             for (int q = 0; q < 3; ++q) stS(Dn + (size_t)q * C + P, DnP[q]);
@@ -813,13 +1215,13 @@ __global__ __launch_bounds__(kBlock) void k_grad(const DevMesh m, const BlockMap
                 dn2 += DnP[q] * DnP[q];
                 acc[3 + q] += DnP[q];
             }
-            acc[0] = nanMax(acc[0], sqrt(dx2));
-            acc[1] = nanMax(acc[1], sqrt(dold2));
-            acc[2] = nanMax(acc[2], sqrt(dn2));
+            acc[0] = nanMax(acc[0], dx2);
+            acc[1] = nanMax(acc[1], dold2);
+            acc[2] = nanMax(acc[2], dn2);
         }
     }
     if (mode == 2) return;
-    storeBlockPartials<6>(acc, 7u, part, lb, bm.nBlocks);
+    storeBlockPartials<6, 3>(acc, part, kOffGrad, lb, bm.nBlocks);
 }
 
 // ---------------------------------------------------------------------------
@@ -854,7 +1256,7 @@ __global__ __launch_bounds__(kBlock) void k_iface_pre(const DevMesh m, const dou
                                                       const T* __restrict__ x, const double* __restrict__ D1,
                                                       double* __restrict__ DI, const double* __restrict__ sigI,
                                                       const Ctl* __restrict__ ctl, int mode) {
-    if (mode == 0 && ctl->outerDone) return;
+    if (mode == 0 && ctl->pending != kPendGrad) return;
     if (mode != 0 || ctl->firstInner) x = nullptr;
     const bool post = mode == 3;
     const double* __restrict__ Dcur = ctl->dpar ? D1 : D0;
@@ -905,7 +1307,7 @@ __global__ __launch_bounds__(kBlock) void k_iface_post(const DevMesh m, const do
                                                        const double* __restrict__ D1, const double* __restrict__ G,
                                                        const double* __restrict__ DI, double* __restrict__ sigI,
                                                        const Ctl* __restrict__ ctl, int mode) {
-    if (mode == 0 && ctl->outerDone) return;
+    if (mode == 0 && ctl->pending != kPendGrad) return;
     // the gradient's cell values: k_grad left D' in the buffer the flip at
     // the end of the step makes current (mode 0), else the current field
     const double* __restrict__ D = (mode == 0) == (ctl->dpar != 0) ? D0 : D1;
@@ -946,8 +1348,8 @@ __global__ __launch_bounds__(kBlock) void k_grad_bnd_post(const DevMesh m, const
                                                           const Ctl* __restrict__ ctlAll, int mode) {
     const int inst = faceInst(bm);
     const Ctl* ctl = ctlAll + inst;
-    if (mode == 0 && ctl->outerDone) return;
-    const int C = m.nCells, B = m.nBoundary;
+    if (mode == 0 && ctl->pending != kPendGrad) return;
+    const int C = m.nCells;
     const int b0 = bm.iB0[inst], b1 = b0 + bm.iNB[inst];
     for (int b = b0 + blockIdx.x * kBlock + threadIdx.x; b < b1; b += gridDim.x * kBlock) {
         const int type = m.bType[b];
@@ -956,42 +1358,7 @@ __global__ __launch_bounds__(kBlock) void k_grad_bnd_post(const DevMesh m, const
         double Gn[9];
 #pragma unroll
         for (int q = 0; q < 9; ++q) Gn[q] = G[(size_t)q * C + P];
-        const double nv[3] = {m.bN[b], m.bN[(size_t)B + b], m.bN[2 * (size_t)B + b]};
-        double Gbv[9], sb[6];
-#pragma unroll
-        for (int j = 0; j < 3; ++j) {
-            const double nG = nv[0] * Gn[j] + nv[1] * Gn[3 + j] + nv[2] * Gn[6 + j];
-            const double sn = snb[(size_t)j * B + b];
-#pragma unroll
-            for (int i = 0; i < 3; ++i) Gbv[3 * i + j] = Gn[3 * i + j] + nv[i] * (sn - nG);
-        }
-        hooke(Gbv, cellMu(m, P), cellK(m, P), sb);
-        if (mode == 1 && ctl->sigma0) {  // cold start: the stress field is still zero
-#pragma unroll
-            for (int q = 0; q < 6; ++q) sb[q] = 0.0;
-        }
-        if (Gb) {
-#pragma unroll
-            for (int q = 0; q < 9; ++q) Gb[(size_t)q * B + b] = Gbv[q];
-        }
-#pragma unroll
-        for (int q = 0; q < 6; ++q) sigb[(size_t)q * B + b] = sb[q];
-        if (mode != 2 && (type == 1 || type == 4)) {
-            // fixedDisplacementZeroShear: the traction snGrad for zero
-            // traction and pressure (its shear-free refGrad)
-            const bool zs = type == 4;
-            const double ik = cellImpK(m, P);
-            const double Tt[9] = {sb[0] - ik * Gbv[0], sb[1] - ik * Gbv[1], sb[2] - ik * Gbv[2],
-                                  sb[1] - ik * Gbv[3], sb[3] - ik * Gbv[4], sb[4] - ik * Gbv[5],
-                                  sb[2] - ik * Gbv[6], sb[4] - ik * Gbv[7], sb[5] - ik * Gbv[8]};
-            const double rik = 1.0 / ik;
-            const double pr = zs ? 0.0 : m.bPres[b];
-#pragma unroll
-            for (int j = 0; j < 3; ++j) {
-                const double nT = nv[0] * Tt[j] + nv[1] * Tt[3 + j] + nv[2] * Tt[6 + j];
-                g[(size_t)j * B + b] = (zs ? -nT : (m.bVal[(size_t)j * B + b] - nv[j] * pr) - nT) * rik;
-            }
-        }
+        bndPostFace(m, mode, mode == 1 && ctl->sigma0, b, type, P, Gn, snb, Gb, sigb, g);
     }
 }
 
@@ -1144,16 +1511,14 @@ __global__ __launch_bounds__(kBlock) void k_pcg_start(const DevMesh m, const Blo
                                                       T* __restrict__ r, T* __restrict__ p, Ctl* __restrict__ ctlAll,
                                                       double* __restrict__ part) {
     const int lb = logicalBlock(bm.nBlocks);
-    const int inst = bm.inst[lb];
+    const Tile tl = bm.at(lb);
     const int C = m.nCells;
     const T* __restrict__ invD = MatSel<T>::invDiag(m);
     double acc[6] = {0, 0, 0, 0, 0, 0};
     const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
-    const int s1 = bm.s1[lb];
-    const int cEnd = bm.iCell0[inst] + bm.iNCell[inst];
-    for (int s = bm.s0[lb] + wave; s < s1; s += kBlock / 64) {
+    for (int s = tl.s0 + wave; s < tl.s1; s += kBlock / 64) {
         const int P = s * kSlice + lane;
-        if (P >= cEnd) continue;
+        if (P >= tl.cEnd) continue;
 #pragma unroll
         for (int j = 0; j < 3; ++j) {
             const size_t i = (size_t)j * C + P;
@@ -1165,32 +1530,30 @@ __global__ __launch_bounds__(kBlock) void k_pcg_start(const DevMesh m, const Blo
             acc[3 + j] += (double)z * (double)rT;
         }
     }
-    storeBlockPartials<6>(acc, 0u, part, lb, bm.nBlocks);
+    storeBlockPartials<6, 0>(acc, part, kOffRho, lb, bm.nBlocks);
 }
 
 // lduMatrix::solver start for one component (component 0) of a caller's LDU
 // matrix: r = source - A psi, and the partials of sum|r| and of OpenFOAM's
 // normFactor, sum |A psi - rowSum avg(psi)| + |source - rowSum avg(psi)|,
-// laid out as k_fin_residual reads them (components 1 and 2 zero)
+// laid out as finResidual reads them (components 1 and 2 zero)
 template <typename T>
 __global__ __launch_bounds__(kBlock) void k_ldu_start(const DevMesh m, const BlockMap bm, const double* __restrict__ psi,
                                                       const double* __restrict__ src, double avg, T* __restrict__ r,
                                                       double* __restrict__ part) {
     const int lb = logicalBlock(bm.nBlocks);
-    const int inst = bm.inst[lb];
+    const Tile tl = bm.at(lb);
     const int C = m.nCells;
     const T* __restrict__ invD = MatSel<T>::invDiag(m);
     double acc[12];
 #pragma unroll
     for (int i = 0; i < 12; ++i) acc[i] = 0.0;
     const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
-    const int s1 = bm.s1[lb];
-    const int cEnd = bm.iCell0[inst] + bm.iNCell[inst];
-    for (int s = bm.s0[lb] + wave; s < s1; s += kBlock / 64) {
+    for (int s = tl.s0 + wave; s < tl.s1; s += kBlock / 64) {
         const int P = s * kSlice + lane;
-        const int e0 = m.sliceStart[s];
-        const int width = m.sliceWidth[s];
-        if (P >= cEnd) continue;
+        const int width = m.width(s);
+        const int e0 = m.entry0(s);
+        if (P >= tl.cEnd) continue;
         const double dg = m.diag[P];
         double Ap = dg * psi[P], asum = 0.0;
         for (int k = 0; k < width; ++k) {
@@ -1213,44 +1576,44 @@ __global__ __launch_bounds__(kBlock) void k_ldu_start(const DevMesh m, const Blo
         acc[6] += fabs(src[P] - t);
         acc[9] += (double)(invD[P] * rT) * (double)rT;
     }
-    storeBlockPartials<12>(acc, 0u, part, lb, bm.nBlocks);
+    storeBlockPartials<12, 0>(acc, part, kOffRes, lb, bm.nBlocks);
 }
 
 // ===========================================================================
 // finalize kernels: one workgroup per instance (grid = number of instances)
 // ===========================================================================
 
-// PCG::solve start: normFactor (lduMatrix::solver::normFactor), normalised
-// initial residual, convergence check before the first iteration, z.r
-__global__ __launch_bounds__(kFinBlock) void k_fin_residual(const BlockMap bm, Ctl* __restrict__ ctlAll,
-                                                            const double* __restrict__ part) {
+// the scalar step of one point of the launch sequence, from st.in to st.out
+// (the same array when the launch sequence is not merged)
+template <int POINT>
+__global__ __launch_bounds__(kFinBlock) void k_fin(const BlockMap bm, const Stage st, const double* __restrict__ part) {
     const int inst = bm.finInst ? bm.finInst[blockIdx.x] : (int)blockIdx.x;
-    Ctl* ctl = ctlAll + inst;
-    if (ctl->outerDone) return;
-    __shared__ double tot[12];
-    finReduce<12>(part, bm.nBlocks, bm.iBlk0[inst], bm.iNBlk[inst], 0u, tot);
-    if (threadIdx.x == 0) {
-        double mag2 = 0.0;
-        int any = 0;
-        for (int j = 0; j < 3; ++j) {
-            const double nf = tot[3 + j] + tot[6 + j] + 1e-20;
-            const bool solved = (ctl->solveMask >> j) & 1;  // fvMatrix::solveSegregated valid components
-            ctl->normFactor[j] = nf;
-            ctl->initRes[j] = solved ? tot[j] / nf : 0.0;
-            ctl->finalRes[j] = ctl->initRes[j];
-            mag2 += ctl->initRes[j] * ctl->initRes[j];
-            ctl->rho[j] = tot[9 + j];
-            ctl->nIter[j] = 0;
-            ctl->alpha[j] = 0.0;
-            ctl->beta[j] = 0.0;
-            // iterate unless already converged (finalRes = initRes < tolerance)
-            const int act = solved && (ctl->pcgMaxIter > 0) && !(ctl->initRes[j] < ctl->pcgTol);
-            ctl->active[j] = act;
-            any |= act;
-        }
-        ctl->initResMag = sqrt(mag2);
-        ctl->innerDone = !any;
-        ctl->firstInner = 1;
+    __shared__ Ctl sh;
+    __shared__ double tot[4 * PointOf<POINT>::nv];
+    const Tile tl{inst, 0, 0, 0, bm.iBlk0[inst], bm.iNBlk[inst], bm.iNCell[inst], 0};
+    StageRun<POINT> run;
+    run.load(st.in + inst, part, bm.nBlocks, tl.blk0, tl.nBlk);
+    run.reduce(&sh, tot, part, bm.nBlocks, tl.blk0, tl.nBlk);
+    run.finish(&sh, tot, tl, st.hist, true, st.out + inst);
+}
+
+// mean field of the initial gradient step (the first normFactor's xbar)
+__global__ __launch_bounds__(kFinBlock) void k_fin_init(const BlockMap bm, Ctl* __restrict__ ctlAll,
+                                                        const double* __restrict__ part) {
+    const int inst = bm.finInst ? bm.finInst[blockIdx.x] : (int)blockIdx.x;
+    __shared__ double tot[6];
+    finReduce<6, 3>(part + (size_t)kOffGrad * bm.nBlocks, bm.nBlocks, bm.iBlk0[inst], bm.iNBlk[inst], tot);
+    if (threadIdx.x == 0)
+        for (int j = 0; j < 3; ++j) ctlAll[inst].xbar[j] = tot[3 + j] / (double)bm.iNCell[inst];
+}
+
+// stops the instances at the end of their current PCG solve (mixed
+// precision's fallback)
+__global__ void k_ctl_hold(Ctl* __restrict__ c, int n, int hold) {
+    for (int i = threadIdx.x; i < n; i += blockDim.x) {
+        c[i].hold = hold;
+        c[i].stallWindow = 0;
+        c[i].stalled = 0;
     }
 }
 
@@ -1260,7 +1623,7 @@ __global__ __launch_bounds__(kFinBlock) void k_fin_pcg_start(const BlockMap bm, 
     const int inst = bm.finInst ? bm.finInst[blockIdx.x] : (int)blockIdx.x;
     Ctl* ctl = ctlAll + inst;
     __shared__ double tot[6];
-    finReduce<6>(part, bm.nBlocks, bm.iBlk0[inst], bm.iNBlk[inst], 0u, tot);
+    finReduce<6, 0>(part + (size_t)kOffRho * bm.nBlocks, bm.nBlocks, bm.iBlk0[inst], bm.iNBlk[inst], tot);
     if (threadIdx.x == 0) {
         int any = 0;
         for (int j = 0; j < 3; ++j) {
@@ -1275,104 +1638,6 @@ __global__ __launch_bounds__(kFinBlock) void k_fin_pcg_start(const BlockMap bm, 
         }
         ctl->innerDone = !any;
         ctl->firstInner = 1;
-    }
-}
-
-// alpha = rho / p.q, with PCG's singularity test |p.q|/normFactor < VSMALL
-__global__ __launch_bounds__(kFinBlock) void k_fin_spmv(const BlockMap bm, Ctl* __restrict__ ctlAll,
-                                                        const double* __restrict__ part) {
-    const int inst = bm.finInst ? bm.finInst[blockIdx.x] : (int)blockIdx.x;
-    Ctl* ctl = ctlAll + inst;
-    if (ctl->outerDone || ctl->innerDone) return;
-    __shared__ double tot[3];
-    finReduce<3>(part, bm.nBlocks, bm.iBlk0[inst], bm.iNBlk[inst], 0u, tot);
-    if (threadIdx.x == 0) {
-        int any = 0;
-        for (int j = 0; j < 3; ++j) {
-            if (!ctl->active[j]) { ctl->alpha[j] = 0.0; continue; }
-            if (fabs(tot[j]) / ctl->normFactor[j] < kVSmall) {
-                ctl->active[j] = 0;
-                ctl->alpha[j] = 0.0;
-                continue;
-            }
-            ctl->alpha[j] = ctl->rho[j] / tot[j];
-            any = 1;
-        }
-        if (!any) ctl->innerDone = 1;
-    }
-}
-
-// PCG convergence per component (tolerance, relTol, maxIter) and beta
-__global__ __launch_bounds__(kFinBlock) void k_fin_update(const BlockMap bm, Ctl* __restrict__ ctlAll,
-                                                          const double* __restrict__ part) {
-    const int inst = bm.finInst ? bm.finInst[blockIdx.x] : (int)blockIdx.x;
-    Ctl* ctl = ctlAll + inst;
-    if (ctl->outerDone || ctl->innerDone) return;
-    __shared__ double tot[6];
-    finReduce<6>(part, bm.nBlocks, bm.iBlk0[inst], bm.iNBlk[inst], 0u, tot);
-    if (threadIdx.x == 0) {
-        int any = 0;
-        for (int j = 0; j < 3; ++j) {
-            if (!ctl->active[j]) continue;
-            ctl->nIter[j] += 1;
-            ctl->innerTotal += 1;
-            const double fr = tot[3 + j] / ctl->normFactor[j];
-            ctl->finalRes[j] = fr;
-            const bool conv = fr < ctl->pcgTol || (ctl->pcgRelTol > 1e-20 && fr < ctl->pcgRelTol * ctl->initRes[j]);
-            const int act = !conv && ctl->nIter[j] < ctl->pcgMaxIter;
-            if (ctl->pcMode == 0) {  // diagonal preconditioner: z.r came with the update
-                ctl->beta[j] = tot[j] / ctl->rho[j];
-                ctl->rho[j] = tot[j];
-            }
-            ctl->active[j] = act;
-            any |= act;
-        }
-        ctl->innerDone = !any;
-        ctl->firstInner = 0;
-    }
-}
-
-// solidModel::converged (total-displacement form) and the mean field for the
-// next normFactor; mode 1 (initialisation) only sets the mean
-__global__ __launch_bounds__(kFinBlock) void k_fin_grad(const BlockMap bm, Ctl* __restrict__ ctlAll,
-                                                        const double* __restrict__ part, double* __restrict__ hist,
-                                                        int mode) {
-    const int inst = bm.finInst ? bm.finInst[blockIdx.x] : (int)blockIdx.x;
-    Ctl* ctl = ctlAll + inst;
-    if (mode == 0 && ctl->outerDone) return;
-    __shared__ double tot[6];
-    finReduce<6>(part, bm.nBlocks, bm.iBlk0[inst], bm.iNBlk[inst], 7u, tot);
-    if (threadIdx.x != 0) return;
-    const double nc = (double)bm.iNCell[inst];
-    for (int j = 0; j < 3; ++j) ctl->xbar[j] = tot[3 + j] / nc;
-    if (mode != 0) return;
-    ctl->dpar ^= 1;  // k_grad wrote D' into the other buffer
-    double denom = tot[1];
-    if (denom < kSmall) denom = tot[2] < kSmall ? kSmall : tot[2];
-    const double rvf = tot[0] / denom;
-    const double ir = ctl->initResMag;
-    const int i = ctl->iCorr;
-    ctl->rvf = rvf;
-    const bool conv = i > 1 && ((ir < ctl->solTol && rvf < ctl->solTol) || rvf < ctl->altTol || ir < ctl->altTol);
-    if (hist && i < ctl->histCap) {
-        double* h = hist + (size_t)inst * 3 * ctl->histCap;
-        h[i] = ir;
-        h[ctl->histCap + i] = rvf;
-        h[2 * ctl->histCap + i] = (double)(ctl->nIter[0] + ctl->nIter[1] + ctl->nIter[2]);
-    }
-    if (!isfinite(ir) || !isfinite(rvf)) {
-        ctl->diverged = 1;
-        ctl->outerDone = 1;
-        ctl->nOuter = i + 1;
-    } else if (conv) {
-        ctl->converged = 1;
-        ctl->outerDone = 1;
-        ctl->nOuter = i + 1;
-    } else if (i + 1 >= ctl->nCorr) {
-        ctl->outerDone = 1;
-        ctl->nOuter = i + 1;
-    } else {
-        ctl->iCorr = i + 1;
     }
 }
 

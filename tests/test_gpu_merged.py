@@ -1,0 +1,97 @@
+"""Merged launch sequences (one slot count, few tiles: kernels that reduce their
+predecessor's partials themselves) against the general ones (finalize kernels,
+any tiles).  A batch of hexahedra and tetrahedra has no single slot count and
+takes the general sequence; each member alone takes the merged one.  Both round
+alike, so the results are equal to the last bit, at the edges of the tiles: one
+cell, one slice less, exactly and more, a tile's remainder, several tiles."""
+import numpy as np
+import pytest
+
+from tests._cases import E_STEEL, NU_STEEL
+
+pytestmark = pytest.mark.gpu
+
+# outer iterations capped: every kernel of the sequence runs, nothing converges
+CAPPED = dict(solutionTolerance=1e-14, alternativeTolerance=1e-14, pcgTolerance=1e-16, pcgRelTol=0.1)
+
+
+@pytest.fixture(scope="module")
+def ctx():
+    from solids4foam_amd import Context
+    c = Context(0)
+    yield c
+    c.close()
+
+
+def _box(ctx, n, seed, law="uniform", tiles=None):
+    from solids4foam_amd import PolyMesh, SolverMesh, cases
+    pm = PolyMesh.box(*n, L=tuple(0.1 * v for v in n), jitter=0.1 if min(n) > 1 else 0.0, seed=seed)
+    types = [cases.TRAC] * 6
+    types[0] = cases.FIX
+    m = SolverMesh(ctx, pm, types)
+    rng = np.random.default_rng(seed)
+    if law == "uniform":
+        m.set_material(E_STEEL, NU_STEEL)
+    else:
+        m.set_material(E_STEEL * rng.uniform(0.5, 2.0, pm.nCells), np.full(pm.nCells, NU_STEEL))
+    for p in range(6):
+        m.set_bc(p, (0.0, 0.0, 0.0))
+    m.set_bc(1, (1e6, -2e6, 5e5))
+    if tiles:
+        m.set_tiles(*tiles)
+    return m
+
+
+def _tets(ctx):
+    from solids4foam_amd import cases
+    return cases.tet_inclusions(ctx, n=4, seed=3)[1]
+
+
+def _same(a, b):
+    return all(np.array_equal(a[k], b[k]) for k in ("D", "sigma")) and \
+        all(a[k] == b[k] for k in ("nOuter", "pcgIterations", "initialResidual", "residualvf"))
+
+
+@pytest.mark.parametrize("precision", [0, 1])
+@pytest.mark.parametrize("precond", [0, 2])
+@pytest.mark.parametrize("law", ["uniform", "cells"])
+def test_merged_equals_general(ctx, precision, precond, law):
+    from solids4foam_amd.batch import Batch
+    print(f"[merged] precision={precision} precond={precond} {law}", flush=True)
+    sizes = [((1, 1, 1), None), ((7, 3, 3), None), ((4, 4, 4), None), ((5, 13, 1), None), ((16, 16, 1), None),
+             ((17, 16, 1), None), ((11, 10, 9), (65536, 1)), ((23, 9, 8), None)]
+    members = [_box(ctx, n, 5 + i, law, tiles=t) for i, (n, t) in enumerate(sizes)] + [_tets(ctx)]
+    for outer, inner in ((1, 0), (2, 1), (6, 100)):
+        opts = dict(CAPPED, precision=precision, preconditioner=precond, nCorrectors=outer, pcgMaxIter=inner)
+        alone = [m.solve(**opts) for m in members]
+        b = Batch(ctx)
+        for m in members:
+            b.add(m)
+        for i, (r, a) in enumerate(zip(b.solve(**opts), alone)):
+            assert _same(r, a), (outer, inner, i, np.abs(r["D"] - a["D"]).max() / max(np.abs(a["D"]).max(), 1e-300))
+        b.close()
+
+
+@pytest.mark.parametrize("relax", [0.0, 0.8])
+def test_line_between_the_two(ctx, relax):
+    # one tile per slice: 1,024 tiles are merged, 1,025 are not; the batch of both is not
+    from solids4foam_amd.batch import Batch
+    print(f"[merged] line relax={relax}", flush=True)
+    members = [_box(ctx, n, 2, tiles=(65536, 1)) for n in ((64, 32, 32), (64, 41, 25))]
+    opts = dict(CAPPED, precision=1, preconditioner=0, nCorrectors=4, pcgMaxIter=30, relaxD=relax)
+    alone = [m.solve(**opts) for m in members]
+    b = Batch(ctx)
+    for m in members:
+        b.add(m)
+    for r, a in zip(b.solve(**opts), alone):
+        assert _same(r, a)
+
+
+def test_batch_of_one(ctx):
+    # merged like the member alone, but on a padded structure
+    from solids4foam_amd.batch import Batch
+    m = _box(ctx, (6, 5, 5), 3)
+    opts = dict(CAPPED, precision=0, preconditioner=0, nCorrectors=12, pcgMaxIter=50)
+    b = Batch(ctx)
+    b.add(m)
+    assert _same(b.solve(**opts)[0], m.solve(**opts))
