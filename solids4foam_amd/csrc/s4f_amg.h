@@ -100,7 +100,8 @@ __device__ __forceinline__ bool mgSkip(const Ctl* c) { return c->outerDone || c-
 
 // Coarse-level vectors are rows of four (three components and a zero pad):
 // one 16-byte (FP32) or 32-byte (FP64) load per neighbour instead of three
-// component gathers.  The fine level keeps the PCG's component-major layout.
+// component gathers; so is the fine level's residual r0, which the restriction
+// gathers.  The PCG's vectors stay component-major.
 template <typename T> struct Row4Sel;
 template <> struct Row4Sel<float> { typedef float type __attribute__((ext_vector_type(4))); };
 template <> struct Row4Sel<double> { typedef double type __attribute__((ext_vector_type(4))); };
@@ -122,7 +123,7 @@ __device__ __forceinline__ Row4<T> row4(T a, T b, T c) {
 // row's own cell with a zero coefficient) so a wave's gathers overlap.
 template <typename T, int W>
 __device__ __forceinline__ void mg0DownRowAll(const DevMesh& m, int P, int e0, int lane, int C, const T* __restrict__ b,
-                                              T* __restrict__ r, T w) {
+                                              Row4<T>* __restrict__ r, T w) {
     const T* __restrict__ A = MatSel<T>::a(m);
     const T* __restrict__ invD = MatSel<T>::invDiag(m);
     int nb[W];
@@ -150,8 +151,7 @@ __device__ __forceinline__ void mg0DownRowAll(const DevMesh& m, int P, int e0, i
 #pragma unroll
         for (int j = 0; j < 3; ++j) y[j] -= av * (wi * b[(size_t)j * C + c]);
     }
-#pragma unroll
-    for (int j = 0; j < 3; ++j) stS(r + (size_t)j * C + P, bP[j] - y[j]);
+    stS(r + P, row4(bP[0] - y[0], bP[1] - y[1], bP[2] - y[2]));
 }
 
 // level-0 prolongation + post-smoothing of one row (all three components,
@@ -160,7 +160,7 @@ __device__ __forceinline__ void mg0DownRowAll(const DevMesh& m, int P, int e0, i
 template <typename T, int W>
 __device__ __forceinline__ void mg0UpRowAll(const DevMesh& m, const int* __restrict__ qCol, const T* __restrict__ q,
                                             int P, int e0, int lane, int C, const T* __restrict__ b,
-                                            const T* __restrict__ r0, const int* __restrict__ agg,
+                                            const Row4<T>* __restrict__ r0, const int* __restrict__ agg,
                                             const Row4<T>* __restrict__ e, T* __restrict__ z, T w, T w1, T al,
                                             double* acc) {
     const T* __restrict__ invD = MatSel<T>::invDiag(m);
@@ -183,12 +183,12 @@ __device__ __forceinline__ void mg0UpRowAll(const DevMesh& m, const int* __restr
 #pragma unroll
         for (int j = 0; j < 3; ++j) s[j] += c * ek[j];
     }
-    const Row4<T> eP = e[IP];
+    const Row4<T> eP = e[IP], rP = r0[P];
 #pragma unroll
     for (int j = 0; j < 3; ++j) {
         const size_t i = (size_t)j * C + P;
         const T bv = b[i];
-        const T zv = wi * (bv + r0[i]) + al * (w1 * eP[j] + wi * s[j]);
+        const T zv = wi * (bv + rP[j]) + al * (w1 * eP[j] + wi * s[j]);
         stS(z + i, zv);
         acc[j] += (double)zv * (double)bv;
     }
@@ -198,7 +198,7 @@ __device__ __forceinline__ void mg0UpRowAll(const DevMesh& m, const int* __restr
 // x = w D^-1 b (not stored: k_mg0_up works from b and r), r = b - A x
 template <typename T>
 __global__ __launch_bounds__(kBlock) void k_mg0_down(const DevMesh m, const BlockMap bm, const T* __restrict__ b,
-                                                     T* __restrict__ r, double omega,
+                                                     Row4<T>* __restrict__ r, double omega,
                                                      const Ctl* __restrict__ ctl) {
     const int lb = logicalBlock(bm.nBlocks);
     const Tile tl = bm.at(lb);
@@ -244,12 +244,10 @@ __global__ __launch_bounds__(kBlock) void k_mg0_down(const DevMesh m, const Bloc
                     if (act[j]) y[j] -= a * (w * iDn * b[(size_t)j * C + n]);
             }
         }
+        T rP[3];  // a converged component's residual is not read
 #pragma unroll
-        for (int j = 0; j < 3; ++j) {
-            if (!act[j]) continue;
-            const size_t i = (size_t)j * C + P;
-            r[i] = b[i] - y[j];
-        }
+        for (int j = 0; j < 3; ++j) rP[j] = act[j] ? b[(size_t)j * C + P] - y[j] : (T)0;
+        r[P] = row4(rP[0], rP[1], rP[2]);
     }
 }
 
@@ -263,7 +261,7 @@ __global__ __launch_bounds__(kBlock) void k_mg0_down(const DevMesh m, const Bloc
 // the PCG residual: z.b = rho of the preconditioned residual).
 template <typename T>
 __global__ __launch_bounds__(kBlock) void k_mg0_up(const DevMesh m, const BlockMap bm, const T* __restrict__ b,
-                                                   const T* __restrict__ r0, const int* __restrict__ agg,
+                                                   const Row4<T>* __restrict__ r0, const int* __restrict__ agg,
                                                    const int* __restrict__ qCol, const T* __restrict__ q,
                                                    const Row4<T>* __restrict__ e, T* __restrict__ z, double omega,
                                                    double alpha, const Ctl* __restrict__ ctl,
@@ -309,12 +307,13 @@ __global__ __launch_bounds__(kBlock) void k_mg0_up(const DevMesh m, const BlockM
                 }
             }
         }
+        const Row4<T> rP = r0[P];
 #pragma unroll
         for (int j = 0; j < 3; ++j) {
             if (!act[j]) continue;
             const size_t i = (size_t)j * C + P;
             const T bv = b[i];
-            const T zv = e ? wi * (bv + r0[i]) + al * (w1 * eP[j] + wi * s3[j]) : wi * (bv + r0[i]);
+            const T zv = e ? wi * (bv + rP[j]) + al * (w1 * eP[j] + wi * s3[j]) : wi * (bv + rP[j]);
             z[i] = zv;
             acc[j] += (double)zv * (double)bv;
         }
@@ -331,7 +330,7 @@ __global__ __launch_bounds__(kBlock) void k_mg0_up(const DevMesh m, const BlockM
 // unconditional and in bounds).  Partial z.b per block.
 template <typename T>
 __global__ __launch_bounds__(kBlock) void k_mg0_up_g(const DevMesh m, const BlockMap bm, const T* __restrict__ b,
-                                                     const T* __restrict__ r0, const int* __restrict__ gStart,
+                                                     const Row4<T>* __restrict__ r0, const int* __restrict__ gStart,
                                                      const int* __restrict__ gWidth, const int* __restrict__ gCol,
                                                      const T* __restrict__ g, const Row4<T>* __restrict__ e,
                                                      T* __restrict__ z, double omega, double alpha,
@@ -371,12 +370,13 @@ __global__ __launch_bounds__(kBlock) void k_mg0_up_g(const DevMesh m, const Bloc
             }
         }
         const T wi = w * invD[P];
+        const Row4<T> rP = r0[P];
 #pragma unroll
         for (int j = 0; j < 3; ++j) {
             if (!act[j]) continue;
             const size_t i = (size_t)j * C + P;
             const T bv = b[i];
-            const T zv = wi * (bv + r0[i]) + al * (wi * sum[j]);
+            const T zv = wi * (bv + rP[j]) + al * (wi * sum[j]);
             stS(z + i, zv);
             acc[j] += (double)zv * (double)bv;
         }
@@ -385,112 +385,169 @@ __global__ __launch_bounds__(kBlock) void k_mg0_up_g(const DevMesh m, const Bloc
 }
 
 // ---------------------------------------------------------------------------
-// coarse levels (grid-stride over the slices of one level)
+// coarse levels (grid-stride over the slices of one level, in the XCD-aware
+// order of the level-0 kernels: each XCD a contiguous range of rows, so gathers
+// of neighbouring rows and of a restriction's fine members stay in its L2)
+//
+// A coarse level has few rows of many slots (Galerkin stencils; 27 to 60), so
+// a wavefront per slice left most of the chip idle while each walked its slots
+// in dependent groups of loads.  A slice's slots are dealt over the workgroup's
+// four wavefronts (slot k to wavefront k mod 4, whatever the slice's width:
+// the order of a row's sum depends on the row alone) and the four sums added in
+// wavefront order.
+// Measured, one wavefront per slice -> four: weighted restriction 18.3 -> 6.6 us
+// (262,144 fine cells, FP32), 42 -> 24 us (566,475, FP64), 54 -> 45 us (2.1
+// million, FP32: bound by its gathers); down sweep 8 -> 4.6 us (262,144).  List
+// restriction with one lane per row -> eight: 13.8 -> 4.6 us (262,144), 19.6 ->
+// 5.2 us (566,475, FP64), 5.8 -> 3.2 us (20,250 tetrahedra).
 // ---------------------------------------------------------------------------
 
-// restriction: bc[I] = sum over members i of I of r[i] (r of the finer
-// level: component-major on level 0 when FINE, rows of four otherwise; each
-// member weighted when the prolongation into I is smoothed), and
-// the coarse pre-smoothed value xc[I] = w D^-1 bc[I] (the coarse level's
-// smoothing from zero, formed once here instead of at every use)
-template <typename T, bool FINE>
-__global__ __launch_bounds__(kBlock) void k_mg_restrict(const MgLevel Lc, const T* __restrict__ r0,
-                                                        const Row4<T>* __restrict__ r4, int nFine,
-                                                        Row4<T>* __restrict__ bc, Row4<T>* __restrict__ xc,
-                                                        double omega, const Ctl* __restrict__ ctl) {
-    const T* __restrict__ iDg = MgSel<T>::iD(Lc);
-    const T* __restrict__ mw = MgSel<T>::memW(Lc);
-    const T w = (T)omega;
-    for (int I = logicalBlock(gridDim.x) * kBlock + threadIdx.x; I < Lc.n; I += gridDim.x * kBlock) {
-        if (Lc.rowInst[I] < 0) continue;  // padding row
-        if (mgSkip(ctl + Lc.rowInst[I])) continue;
-        T s[3] = {(T)0, (T)0, (T)0};
-        const int k1 = Lc.memOff[I + 1];
-        // members 8 at a time, loads unconditional (past the end: the last
-        // member again, weight zero), in member order
-        for (int k0 = Lc.memOff[I]; k0 < k1; k0 += 8) {
-            int mi[8];
-            T wv[8];
+// the instance's PCG runs (rowInst: nullptr where all rows are instance 0's;
+// -1: padding row)
+__device__ __forceinline__ bool mgLive(const MgLevel& L, int row, bool on, const Ctl* ctl, int& inst) {
+    inst = L.rowInst ? (on ? L.rowInst[row] : -1) : 0;
+    return on && inst >= 0 && !mgSkip(ctl + inst);
+}
+
+// sum += sum over slots k = wave, wave + 4, ... of coef_k x[idx_k], kMgChunk
+// slots' loads in flight at a time, all unconditional (a slot past the width
+// or empty reads an in-bounds slot and row `own` with a zero coefficient)
+template <typename T>
+__device__ __forceinline__ void slotSum(const int* __restrict__ idx, const T* __restrict__ coef, int width, int wave,
+                                        int lane, int own, const Row4<T>* __restrict__ x, T* sum) {
+    constexpr int kWaves = kBlock / 64;
+    for (int k0 = wave; k0 < width; k0 += kWaves * kMgChunk) {
+        int J[kMgChunk];
+        T c[kMgChunk];
 #pragma unroll
-            for (int u = 0; u < 8; ++u) {
-                const int k = k0 + u < k1 ? k0 + u : k1 - 1;
-                mi[u] = Lc.mem[k];
-                wv[u] = mw ? mw[k] : (T)1;
-            }
-            T rv[8][3];
-#pragma unroll
-            for (int u = 0; u < 8; ++u) {
-                if (FINE) {
-#pragma unroll
-                    for (int j = 0; j < 3; ++j) rv[u][j] = r0[(size_t)j * nFine + mi[u]];
-                } else {
-                    const Row4<T> v = r4[mi[u]];
-#pragma unroll
-                    for (int j = 0; j < 3; ++j) rv[u][j] = v[j];
-                }
-            }
-#pragma unroll
-            for (int u = 0; u < 8; ++u)
-#pragma unroll
-                for (int j = 0; j < 3; ++j)
-                    if (k0 + u < k1) s[j] += wv[u] * rv[u][j];
+        for (int u = 0; u < kMgChunk; ++u) {
+            const int k = k0 + kWaves * u;
+            const int o = (k < width ? k : k0) * kSlice;
+            J[u] = at32(idx + o, lane * 4u);
+            c[u] = at32(coef + o, lane * (unsigned)sizeof(T));
+            if (k >= width) J[u] = -1;
         }
-        // all three components stored: a converged component's coarse
-        // values are never read for an active one
-        const T wi = w * iDg[I];
-        bc[I] = row4(s[0], s[1], s[2]);
-        xc[I] = row4(wi * s[0], wi * s[1], wi * s[2]);
+#pragma unroll
+        for (int u = 0; u < kMgChunk; ++u) {
+            const bool v = J[u] >= 0;
+            const Row4<T> xv = x[v ? J[u] : own];
+            const T cv = v ? c[u] : (T)0;
+#pragma unroll
+            for (int j = 0; j < 3; ++j) sum[j] += cv * xv[j];
+        }
     }
 }
 
-// Coarse-level kernels take their rows in the XCD-aware order of the level-0
-// kernels (logicalBlock: each XCD a contiguous range of rows, so gathers of
-// neighbouring rows and of a restriction's fine members stay in its L2).
-// Coarse-level rows are wider (Galerkin stencils) and of varying width:
-// slots are processed kMgChunk at a time with every load unconditional (slots
-// past the row's width or empty read an in-bounds slot and the row's own
-// value with a zero coefficient).
-
-// restriction into the first coarse level of a smoothed hierarchy: bc = P^T r0
-// with the weighted member lists in the coarse level's sliced-ELL slots (one
-// wave per 64 coarse rows, each slot one coalesced load of members and
-// weights; members in ascending fine-row order), and xc = w D^-1 bc
+// the four wavefronts' sums of a slice, in wavefront 0 (a barrier: all threads)
 template <typename T>
-__global__ __launch_bounds__(kBlock) void k_mg_restrict_w(const MgLevel Lc, const T* __restrict__ r0, int nFine,
-                                                          Row4<T>* __restrict__ bc, Row4<T>* __restrict__ xc,
-                                                          double omega, const Ctl* __restrict__ ctl) {
-    const T* __restrict__ iDg = MgSel<T>::iD(Lc);
-    const T* __restrict__ rw = MgSel<T>::rW(Lc);
-    const T w = (T)omega;
-    const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
-    const int wavesTotal = gridDim.x * (kBlock / 64);
-    for (int s = logicalBlock(gridDim.x) * (kBlock / 64) + wave; s < Lc.nSlices; s += wavesTotal) {
-        const int I = s * kSlice + lane;
-        if (I >= Lc.n) continue;
-        const int inst = Lc.rowInst[I];
-        if (inst < 0) continue;  // padding row
-        if (mgSkip(ctl + inst)) continue;
-        const int e0 = Lc.rStart[s];
-        const int width = Lc.rWidth[s];
-        T sum[3] = {(T)0, (T)0, (T)0};
-        for (int k0 = 0; k0 < width; k0 += kMgChunk) {
-            int mi[kMgChunk];
-            T wv[kMgChunk];
+__device__ __forceinline__ void sumWaves(T (*sh)[3][kSlice], int wave, int lane, T* sum) {
+    if (wave > 0) {
 #pragma unroll
-            for (int u = 0; u < kMgChunk; ++u) {
-                const int k = k0 + u < width ? k0 + u : width - 1;
-                const int en = e0 + k * kSlice + lane;
-                mi[u] = ldS(Lc.rMem + en);
-                wv[u] = k0 + u < width ? ldS(rw + en) : (T)0;
+        for (int j = 0; j < 3; ++j) sh[wave - 1][j][lane] = sum[j];
+    }
+    __syncthreads();
+    if (wave == 0) {
+#pragma unroll
+        for (int q = 0; q < kBlock / 64 - 1; ++q)
+#pragma unroll
+            for (int j = 0; j < 3; ++j) sum[j] += sh[q][j][lane];
+    }
+}
+
+// value of the lane at distance 1, 2 (within a quad) and 4 (once a quad's
+// lanes hold equal values) of a group of eight
+template <int CTRL>
+__device__ __forceinline__ float dppOf(float v) {
+    return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), CTRL, 0xf, 0xf, false));
+}
+template <int CTRL>
+__device__ __forceinline__ double dppOf(double v) {
+    const int lo = __builtin_amdgcn_update_dpp(0, __double2loint(v), CTRL, 0xf, 0xf, false);
+    const int hi = __builtin_amdgcn_update_dpp(0, __double2hiint(v), CTRL, 0xf, 0xf, false);
+    return __hiloint2double(hi, lo);
+}
+template <typename T>
+__device__ __forceinline__ T sumOf8(T v) {
+    v += dppOf<0xB1>(v);   // quad_perm 1 0 3 2
+    v += dppOf<0x4E>(v);   // quad_perm 2 3 0 1
+    return v + dppOf<0x141>(v);  // row_half_mirror
+}
+
+// restriction: bc[I] = sum over members i of I of r[i] (r of the finer level;
+// each member weighted when the prolongation into I is smoothed), and the
+// coarse pre-smoothed value xc[I] = w D^-1 bc[I] (the coarse level's smoothing
+// from zero, formed once here instead of at every use).  Eight lanes per row:
+// a row's member list is read in one coalesced load, and levels of a few
+// thousand rows still fill the chip.
+template <typename T>
+__global__ __launch_bounds__(kBlock) void k_mg_restrict(const MgLevel Lc, const Row4<T>* __restrict__ r,
+                                                        Row4<T>* __restrict__ bc, Row4<T>* __restrict__ xc,
+                                                        double omega, const Ctl* __restrict__ ctl) {
+    constexpr int kRows = kBlock / 8;
+    const T* __restrict__ iDg = MgSel<T>::iD(Lc);
+    const T* __restrict__ mw = MgSel<T>::memW(Lc);
+    const T w = (T)omega;
+    const int sub = threadIdx.x & 7;
+    for (int I = logicalBlock(gridDim.x) * kRows + (threadIdx.x >> 3); I < Lc.n; I += gridDim.x * kRows) {
+        const int k0 = Lc.memOff[I], k1 = Lc.memOff[I + 1];
+        const T wi = w * iDg[I];
+        int inst;
+        if (!mgLive(Lc, I, true, ctl, inst)) continue;  // the eight lanes alike
+        T s[3] = {(T)0, (T)0, (T)0};
+        // loads unconditional (past the end: the last member again, weight zero)
+        for (int kb = k0; kb < k1; kb += 32) {
+            int mi[4];
+            T wv[4];
+#pragma unroll
+            for (int u = 0; u < 4; ++u) {
+                const int k = kb + 8 * u + sub;
+                const int kc = k < k1 ? k : k1 - 1;
+                mi[u] = Lc.mem[kc];
+                wv[u] = k < k1 ? (mw ? mw[kc] : (T)1) : (T)0;
             }
 #pragma unroll
-            for (int u = 0; u < kMgChunk; ++u)
+            for (int u = 0; u < 4; ++u) {
+                const Row4<T> v = r[mi[u]];
 #pragma unroll
-                for (int j = 0; j < 3; ++j) sum[j] += wv[u] * r0[(size_t)j * nFine + mi[u]];
+                for (int j = 0; j < 3; ++j) s[j] += wv[u] * v[j];
+            }
         }
-        const T wi = w * iDg[I];
-        bc[I] = row4(sum[0], sum[1], sum[2]);
-        xc[I] = row4(wi * sum[0], wi * sum[1], wi * sum[2]);
+#pragma unroll
+        for (int j = 0; j < 3; ++j) s[j] = sumOf8(s[j]);
+        // all three components stored: a converged component's coarse
+        // values are never read for an active one
+        if (sub == 0) bc[I] = row4(s[0], s[1], s[2]);
+        if (sub == 1) xc[I] = row4(wi * s[0], wi * s[1], wi * s[2]);
+    }
+}
+
+// restriction into the first coarse level of a smoothed hierarchy: bc = P^T r0
+// with the weighted member lists in the coarse level's sliced-ELL slots (each
+// slot one coalesced load of members and weights; members in ascending
+// fine-row order), and xc = w D^-1 bc
+template <typename T>
+__global__ __launch_bounds__(kBlock) void k_mg_restrict_w(const MgLevel Lc, const Row4<T>* __restrict__ r0,
+                                                          Row4<T>* __restrict__ bc, Row4<T>* __restrict__ xc,
+                                                          double omega, const Ctl* __restrict__ ctl) {
+    __shared__ T sh[kBlock / 64 - 1][3][kSlice];
+    const T* __restrict__ iDg = MgSel<T>::iD(Lc);
+    const T w = (T)omega;
+    const int wave = waveOf(), lane = threadIdx.x & 63;
+    for (int s = logicalBlock(gridDim.x); s < Lc.nSlices; s += gridDim.x) {
+        const int I = s * kSlice + lane;
+        const int e0 = Lc.rStart[s];
+        const int width = Lc.rWidth[s];
+        int inst;
+        const bool live = mgLive(Lc, I, I < Lc.n, ctl, inst);
+        T sum[3] = {(T)0, (T)0, (T)0};
+        if (live) slotSum<T>(Lc.rMem + e0, MgSel<T>::rW(Lc) + e0, width, wave, lane, 0, r0, sum);
+        sumWaves<T>(sh, wave, lane, sum);
+        if (live && wave == 0) {
+            const T wi = w * iDg[I];
+            bc[I] = row4(sum[0], sum[1], sum[2]);
+            xc[I] = row4(wi * sum[0], wi * sum[1], wi * sum[2]);
+        }
+        __syncthreads();  // the next slice's sums take the same LDS
     }
 }
 
@@ -499,49 +556,31 @@ template <typename T>
 __global__ __launch_bounds__(kBlock) void k_mg_down(const MgLevel L, const Row4<T>* __restrict__ b,
                                                     const Row4<T>* __restrict__ x, Row4<T>* __restrict__ r,
                                                     const Ctl* __restrict__ ctl) {
-    const T* __restrict__ A = MgSel<T>::a(L);
+    __shared__ T sh[kBlock / 64 - 1][3][kSlice];
     const T* __restrict__ dg = MgSel<T>::d(L);
-    const int n = L.n;
-    const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
-    const int wavesTotal = gridDim.x * (kBlock / 64);
-    for (int s = logicalBlock(gridDim.x) * (kBlock / 64) + wave; s < L.nSlices; s += wavesTotal) {
+    const int wave = waveOf(), lane = threadIdx.x & 63;
+    for (int s = logicalBlock(gridDim.x); s < L.nSlices; s += gridDim.x) {
         const int P = s * kSlice + lane;
-        if (P >= n) continue;
-        const int inst = L.rowInst[P];
-        if (inst < 0) continue;  // padding row
-        if (mgSkip(ctl + inst)) continue;
-        const Row4<T> bP = b[P];
-        if (L.pass[inst]) {  // already coarsest for this instance: hand b down unchanged
-            r[P] = bP;
-            continue;
-        }
         const int e0 = L.sliceStart[s];
         const int width = L.sliceWidth[s];
-        const Row4<T> xP = x[P];
-        const T d = dg[P];
-        T y[3];
-#pragma unroll
-        for (int j = 0; j < 3; ++j) y[j] = d * xP[j];
-        for (int k0 = 0; k0 < width; k0 += kMgChunk) {
-            int nb[kMgChunk];
-            T a[kMgChunk];
-#pragma unroll
-            for (int u = 0; u < kMgChunk; ++u) {
-                const int k = k0 + u < width ? k0 + u : width - 1;
-                const int e = e0 + k * kSlice + lane;
-                nb[u] = k0 + u < width ? ldS(L.col + e) : -1;
-                a[u] = ldS(A + e);
-            }
-#pragma unroll
-            for (int u = 0; u < kMgChunk; ++u) {
-                const bool v = nb[u] >= 0;
-                const Row4<T> xc = x[v ? nb[u] : P];
-                const T av = v ? a[u] : (T)0;
-#pragma unroll
-                for (int j = 0; j < 3; ++j) y[j] -= av * xc[j];
-            }
+        int inst;
+        const bool live = mgLive(L, P, P < L.n, ctl, inst);
+        const bool pass = live && L.pass[inst];  // already coarsest for this instance: hand b down unchanged
+        const bool last = live && wave == 0;
+        Row4<T> bP = {}, xP = {};
+        T d = (T)0;
+        if (last) {
+            bP = b[P];
+            xP = x[P];
+            d = dg[P];
         }
-        r[P] = row4(bP[0] - y[0], bP[1] - y[1], bP[2] - y[2]);
+        T sum[3] = {(T)0, (T)0, (T)0};
+        if (live && !pass) slotSum<T>(L.col + e0, MgSel<T>::a(L) + e0, width, wave, lane, P, x, sum);
+        sumWaves<T>(sh, wave, lane, sum);
+        if (last)
+            r[P] = pass ? bP
+                        : row4(bP[0] - (d * xP[0] - sum[0]), bP[1] - (d * xP[1] - sum[1]), bP[2] - (d * xP[2] - sum[2]));
+        __syncthreads();
     }
 }
 
@@ -554,52 +593,37 @@ __global__ __launch_bounds__(kBlock) void k_mg_up(const MgLevel L, const Row4<T>
                                                   const Row4<T>* __restrict__ r, const Row4<T>* __restrict__ e,
                                                   Row4<T>* __restrict__ out, double omega, double alpha,
                                                   const Ctl* __restrict__ ctl) {
-    const T* __restrict__ q = MgSel<T>::q(L);
+    __shared__ T sh[kBlock / 64 - 1][3][kSlice];
     const T* __restrict__ iDg = MgSel<T>::iD(L);
     const T w = (T)omega, w1 = (T)(1.0 - omega), al = (T)alpha;
-    const int n = L.n;
-    const int* __restrict__ agg = L.agg;
-    const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
-    const int wavesTotal = gridDim.x * (kBlock / 64);
-    for (int s = logicalBlock(gridDim.x) * (kBlock / 64) + wave; s < L.nSlices; s += wavesTotal) {
+    const int wave = waveOf(), lane = threadIdx.x & 63;
+    for (int s = logicalBlock(gridDim.x); s < L.nSlices; s += gridDim.x) {
         const int P = s * kSlice + lane;
-        if (P >= n) continue;
-        const int inst = L.rowInst[P];
-        if (inst < 0) continue;  // padding row
-        if (mgSkip(ctl + inst)) continue;
-        const int IP = agg[P];
-        const Row4<T> eP = e[IP];
-        if (L.pass[inst]) {  // already coarsest for this instance: the coarser solution unchanged
-            out[P] = eP;
-            continue;
-        }
         const int e0 = L.sliceStart[s];
         const int width = L.qWidth[s];
-        T sum[3] = {(T)0, (T)0, (T)0};
-        for (int k0 = 0; k0 < width; k0 += kMgChunk) {
-            int J[kMgChunk];
-            T c[kMgChunk];
-#pragma unroll
-            for (int u = 0; u < kMgChunk; ++u) {
-                const int k = k0 + u < width ? k0 + u : width - 1;
-                const int en = e0 + k * kSlice + lane;
-                J[u] = k0 + u < width ? ldS(L.qCol + en) : -1;
-                c[u] = ldS(q + en);
-            }
-#pragma unroll
-            for (int u = 0; u < kMgChunk; ++u) {
-                const bool v = J[u] >= 0;
-                const Row4<T> ev = e[v ? J[u] : IP];
-                const T cv = v ? c[u] : (T)0;
-#pragma unroll
-                for (int j = 0; j < 3; ++j) sum[j] += cv * ev[j];
-            }
+        int inst;
+        const bool live = mgLive(L, P, P < L.n, ctl, inst);
+        const bool pass = live && L.pass[inst];  // already coarsest: the coarser solution unchanged
+        const bool last = live && wave == 0;
+        Row4<T> xv = {}, rv = {}, eP = {};
+        T iD = (T)0;
+        if (last) {
+            eP = e[L.agg[P]];
+            xv = x[P];
+            rv = r[P];
+            iD = iDg[P];
         }
-        const Row4<T> xv = x[P], rv = r[P];
-        const T wi = w * iDg[P];
-        out[P] = row4(xv[0] + wi * rv[0] + al * (w1 * eP[0] + wi * sum[0]),
-                      xv[1] + wi * rv[1] + al * (w1 * eP[1] + wi * sum[1]),
-                      xv[2] + wi * rv[2] + al * (w1 * eP[2] + wi * sum[2]));
+        T sum[3] = {(T)0, (T)0, (T)0};
+        if (live && !pass) slotSum<T>(L.qCol + e0, MgSel<T>::q(L) + e0, width, wave, lane, 0, e, sum);
+        sumWaves<T>(sh, wave, lane, sum);
+        if (last) {
+            const T wi = w * iD;
+            out[P] = pass ? eP
+                          : row4(xv[0] + wi * rv[0] + al * (w1 * eP[0] + wi * sum[0]),
+                                 xv[1] + wi * rv[1] + al * (w1 * eP[1] + wi * sum[1]),
+                                 xv[2] + wi * rv[2] + al * (w1 * eP[2] + wi * sum[2]));
+        }
+        __syncthreads();
     }
 }
 
@@ -612,10 +636,8 @@ __global__ __launch_bounds__(kBlock) void k_mg_dense(const MgLevel L, const T* _
                                                      const Ctl* __restrict__ ctl) {
     const int row = blockIdx.x * (kBlock / 64) + (threadIdx.x >> 6);
     const int lane = threadIdx.x & 63;
-    if (row >= L.n) return;
-    const int inst = L.rowInst[row];
-    if (inst < 0) return;  // padding row
-    if (mgSkip(ctl + inst)) return;
+    int inst;
+    if (!mgLive(L, row, row < L.n, ctl, inst)) return;
     const int r0 = L.blkRow0[inst], nb = L.blkN[inst];
     double acc[3] = {0, 0, 0};
     const T* __restrict__ a = Ainv + (size_t)L.invOff[inst] + (size_t)(row - r0) * nb;

@@ -273,7 +273,7 @@ __global__ __launch_bounds__(kBlock) void k_spmvp_m(const DevMesh m, const Block
 // k_mg0_down: r = b - A x with x = w D^-1 b; no load depends on the scalars
 template <typename T, bool AGAIN, int W>
 __global__ __launch_bounds__(kBlock) void k_mg0_down_m(const DevMesh m, const BlockMap bm, const T* __restrict__ b,
-                                                       T* __restrict__ r, double omega, const Stage st,
+                                                       Row4<T>* __restrict__ r, double omega, const Stage st,
                                                        const double* __restrict__ part) {
     constexpr int kPt = AGAIN ? kPtAgain : kPtInner;
     const int lb = logicalBlock(bm.nBlocks);
@@ -328,9 +328,7 @@ __global__ __launch_bounds__(kBlock) void k_mg0_down_m(const DevMesh m, const Bl
             for (int k = 0; k < W; ++k) xn[k] = w * iDN[k] * bN[k][j];
             y[j] = rowProduct<T, W>(all, dP, w * iDP * bP[j], row.a, xn);
         }
-#pragma unroll
-        for (int j = 0; j < 3; ++j)
-            if (act[j]) put32(r + (size_t)j * C, P * kT, (T)(bP[j] - y[j]));
+        r[P] = row4<T>(bP[0] - y[0], bP[1] - y[1], bP[2] - y[2]);  // a converged component's is not read
     }
 }
 // k_residual, the slots in a loop: with the row unrolled the kernel was 20 KB

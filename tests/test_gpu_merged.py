@@ -95,3 +95,20 @@ def test_batch_of_one(ctx):
     b = Batch(ctx)
     b.add(m)
     assert _same(b.solve(**opts)[0], m.solve(**opts))
+
+
+@pytest.mark.parametrize("n,counts", [((1, 1, 1), (3, 3)), ((5, 3, 2), (30, 30)), ((8, 8, 8), (36, 36)),
+                                      ((9, 8, 8), (36, 36)), ((13, 11, 10), (66, 66)), ((20, 20, 20), (90, 66)),
+                                      ((33, 32, 31), (96, 72)), ("tets", (39, 39))])
+def test_vcycle_iteration_counts(ctx, n, counts):
+    # PCG iterations of one tight momentum solve, plain and smoothed multigrid:
+    # a V-cycle that lost a slot or a member converges more slowly.  Counts of
+    # the coarse kernels with one lane per row; a different summation order
+    # moves an iteration's norm by 1e-15, so one iteration per component of slack
+    m = _tets(ctx) if n == "tets" else _box(ctx, n, 3)
+    opts = dict(nCorrectors=2, precision=0, pcgRelTol=0.0, pcgTolerance=1e-10, solutionTolerance=1e-14,
+                alternativeTolerance=1e-14)
+    for precond, want in zip((2, 3), counts):
+        got = m.solve(preconditioner=precond, **opts)["innerTotal"]
+        print(f"[vcycle] {n} precond={precond}: {got}", flush=True)
+        assert abs(got - want) <= 3
