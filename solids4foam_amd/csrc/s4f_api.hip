@@ -950,10 +950,9 @@ struct Chain {
 // With the diagonal preconditioner the lines cross at the same size (64: mixed
 // 889 -> 838, FP64 1130 -> 1174).
 constexpr int kMergeTiles = 1024;
-// the merged kernels read every slot of a row at once, for these slot counts
-inline bool canMerge(const DevMesh& dm, int maxTiles) {
-    return maxTiles <= kMergeTiles && (dm.uniW == 6 || dm.uniW == 4);
-}
+// the slot counts that the kernels of s4f_merged.h are compiled for
+inline bool uniformSlots(const DevMesh& dm) { return dm.uniW == 6 || dm.uniW == 4; }
+inline bool canMerge(const DevMesh& dm, int maxTiles) { return maxTiles <= kMergeTiles && uniformSlots(dm); }
 
 template <int POINT>
 void launchFin(const BlockMap& bm, int nFin, const Chain& c, const Ctl* in, Ctl* out, const double* part, hipStream_t s) {
@@ -2046,18 +2045,18 @@ void launchGradStep(const DevMesh& dm, const BlockMap& bm, int nInst, int maxNB,
                        f.Gb, f.sigb, f.g, ctl, mode);
 }
 
-// the merged residual for a launch's slot count and moduli
-template <typename T>
-auto residualMerged(const DevMesh& dm, const BlockMap& bm) {
-    if (dm.uniW == 6) return dm.mu ? k_residual_m<T, 6, true> : k_residual_m<T, 6, false>;
-    return dm.mu ? k_residual_m<T, 4, true> : k_residual_m<T, 4, false>;
+// the residual for a launch's slot count and moduli (uniform slot counts only)
+template <typename T, bool MERGED>
+auto residualUniform(const DevMesh& dm) {
+    if (dm.uniW == 6) return dm.mu ? k_residual_u<T, 6, true, MERGED> : k_residual_u<T, 6, false, MERGED>;
+    return dm.mu ? k_residual_u<T, 4, true, MERGED> : k_residual_u<T, 4, false, MERGED>;
 }
-
 // The outer step of the momentum loop for the instances whose PCG has
 // finished: gradient step, convergence test, residual (the others skip it).
 template <typename T>
 void launchOuter(const DevMesh& dm, const BlockMap& bm, int nFin, int maxNB, const GradBufs& f, const PcgVecs<T>& v,
                  const double* Dold, const Chain& c, double* part, hipStream_t s) {
+    const bool uni = uniformSlots(dm);
     if (c.merged && !f.aAlpha && dm.nIf == 0) {
         hipLaunchKernelGGL((dm.uniW == 6 ? k_grad_m<T, 6> : k_grad_m<T, 4>), dim3(bm.nBlocks), dim3(kBlock), 0, s, dm,
                            bm, f.D0, (const T*)v.x, f.D1, f.G, f.Db, Dold, c.at(c.x, c.y), part,
@@ -2066,14 +2065,14 @@ void launchOuter(const DevMesh& dm, const BlockMap& bm, int nFin, int maxNB, con
         launchFin<kPtGrad>(bm, nFin, c, c.x, c.y, part, s);
         launchGradStep<T>(dm, bm, nFin, maxNB, f, (const T*)v.x, Dold, c.y, part, 0, s);
     }
-    if (c.merged) {
-        hipLaunchKernelGGL(residualMerged<T>(dm, bm), dim3(bm.nBlocks), dim3(kBlock), 0, s, dm, bm, (const double*)f.D0,
-                           (const double*)f.D1, (const double*)f.G, (const double*)f.sigb, v.r, c.at(c.y, c.z), part);
-    } else {
-        launchFin<kPtRes>(bm, nFin, c, c.x, c.x, part, s);
+    if (!c.merged) launchFin<kPtRes>(bm, nFin, c, c.x, c.x, part, s);
+    if (uni)
+        hipLaunchKernelGGL((c.merged ? residualUniform<T, true>(dm) : residualUniform<T, false>(dm)), dim3(bm.nBlocks),
+                           dim3(kBlock), 0, s, dm, bm, (const double*)f.D0, (const double*)f.D1, (const double*)f.G,
+                           (const double*)f.sigb, v.r, c.at(c.y, c.z), part);
+    else
         hipLaunchKernelGGL((k_residual<T>), dim3(bm.nBlocks), dim3(kBlock), 0, s, dm, bm, (const double*)f.D0,
                            (const double*)f.D1, (const double*)f.G, (const double*)f.sigb, v.r, (const Ctl*)c.x, part);
-    }
 }
 
 // One pass of the momentum loop's launch sequence: the outer step of every

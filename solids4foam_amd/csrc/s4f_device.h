@@ -41,11 +41,19 @@ template <typename T> __device__ __forceinline__ T at32(const T* base, unsigned 
     asm("" : "+s"(b));
     return *(const S4F_GLOBAL T*)(b + off);
 }
+template <typename T> __device__ __forceinline__ T at32s(const T* base, unsigned off) {
+    const S4F_GLOBAL char* b = (const S4F_GLOBAL char*)base;
+    asm("" : "+s"(b));
+    return __builtin_nontemporal_load((const S4F_GLOBAL T*)(b + off));
+}
 template <typename T> __device__ __forceinline__ void put32(T* base, unsigned off, T v) {
     S4F_GLOBAL char* b = (S4F_GLOBAL char*)base;
     asm("" : "+s"(b));
     *(S4F_GLOBAL T*)(b + off) = v;
 }
+// Loads above stay above: the scheduler would otherwise put each next to its
+// first use to save registers, and a slot's loads would wait for one another.
+__device__ __forceinline__ void loadsAbove() { asm volatile("" ::: "memory"); }
 // wavefront of the workgroup, known uniform
 __device__ __forceinline__ int waveOf() { return __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6); }
 
@@ -108,7 +116,10 @@ struct DevMesh {
     const unsigned char* sliceIf; // per slice: 1 if it holds interface entries
     const int* zone;              // material zone of each cell (nullptr: one material)
     __device__ __forceinline__ int width(int s) const { return uniW ? uniW : sliceWidth[s]; }
-    __device__ __forceinline__ int entry0(int s) const { return contig ? s * uniW * kSlice : sliceStart[s]; }
+    // s uniform over the wavefront, and so is the result (a scalar base for at32)
+    __device__ __forceinline__ int entry0(int s) const {
+        return __builtin_amdgcn_readfirstlane(contig ? s * uniW * kSlice : sliceStart[s]);
+    }
 };
 
 // Reduced scalars an instance still owes its control block: the block partials

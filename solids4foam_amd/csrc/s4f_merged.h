@@ -17,15 +17,6 @@
 
 namespace s4f {
 
-__device__ __forceinline__ double fmaT(double a, double b, double c) { return __builtin_fma(a, b, c); }
-__device__ __forceinline__ float fmaT(float a, float b, float c) { return __builtin_fmaf(a, b, c); }
-// v, rounded here: no later addition contracts with the product that formed it
-template <typename T>
-__device__ __forceinline__ T rounded(T v) {
-    asm("" : "+v"(v));
-    return v;
-}
-
 // y = d x - sum_k a_k x_k in slot order, rounded as the kernels for tiles of
 // any kind round it: their unrolled rows (all three components active)
 // contract d x with the first term's subtraction, their loops over the slots
@@ -37,11 +28,6 @@ __device__ __forceinline__ T rowProduct(bool all, T d, T x, const T* a, const T*
 #pragma unroll
     for (int k = 1; k < W; ++k) y = fmaT(-a[k], xn[k], y);
     return y;
-}
-
-// a.b, rounded as the compiler contracts a0 b0 + a1 b1 + a2 b2
-__device__ __forceinline__ double dot3(double a0, double b0, double a1, double b1, double a2, double b2) {
-    return fmaT(a2, b2, fmaT(a0, b0, a1 * b1));
 }
 
 // hooke() with its contractions spelled out (mu2 = 2 mu)
@@ -331,150 +317,183 @@ __global__ __launch_bounds__(kBlock) void k_mg0_down_m(const DevMesh m, const Bl
         r[P] = row4<T>(bP[0] - y[0], bP[1] - y[1], bP[2] - y[2]);  // a converged component's is not read
     }
 }
-// k_residual, the slots in a loop: with the row unrolled the kernel was 20 KB
-// of code and the two workgroups of 512 cells waited 16.1 us, mostly for their
-// instructions; 11.2 us as a loop.  Half a row's loads in flight at a time (168
-// registers) measured the same as one slot's (160) from 512 to 64,000 cells and
-// 2 % worse from 262,144 on, so it is one slot.  MU: moduli per cell (a branch
-// in the row would let the loads of all slots drift together).
-template <typename T, int W, bool MU>
-__global__ __launch_bounds__(kBlock, 3) void k_residual_m(
+// The residual of meshes of one slot count, in merged launch sequences
+// (MERGED) and with finalize kernels: one slice per wavefront,
+// the slots in a loop.  A wavefront's time is its instructions (one about every
+// 2.5 ns) plus a load latency per slot, so
+//   * the slots are not unrolled (unrolled, 512 cells took 16.1 us, as a loop 11.2),
+//   * the loop's registers are kept to what one slot needs: the sums over the
+//     workgroup's cells (SliceAcc) are no part of it,
+//   * boundary slots are visited only where the wavefront has any (a bit per slot).
+
+// A thread's sums over its cells: its first (mostly only) slice's live in
+// registers from that slice's end on, earlier slices' of larger tiles in LDS.
+template <int N>
+struct SliceAcc {
+    double (*lds)[kBlock];
+    bool first = true;
+    __device__ __forceinline__ void get(double* v) const {
+#pragma unroll
+        for (int i = 0; i < N; ++i) v[i] = first ? 0.0 : lds[i][threadIdx.x];
+    }
+    __device__ __forceinline__ void put(const double* v) {
+#pragma unroll
+        for (int i = 0; i < N; ++i) lds[i][threadIdx.x] = v[i];
+        first = false;
+    }
+};
+
+// k_residual.  MU: moduli per cell (a branch in the row would let the loads of
+// all slots drift together).  Not MERGED (more cells than the L2s hold): a
+// slot's loads are issued together and the face data streams past the L2;
+// 128^3 cells (FP32 PCG): 277 us before (k_residual), 335 with the loads as the
+// compiler schedules them, 270 now, against 169 for each array read once: the
+// neighbour planes' gradients are fetched again from beyond the 4 MB L2s.  Two
+// slots at a time: 287.  MERGED the compiler's schedule is better (512 cells:
+// 10.4 us, 12.4 with the loads together; before 11.2).
+template <typename T, int W, bool MU, bool MERGED>
+__global__ __launch_bounds__(kBlock, 3) void k_residual_u(
     const DevMesh m, const BlockMap bm, const double* __restrict__ D0, const double* __restrict__ D1,
     const double* __restrict__ G, const double* __restrict__ sigb, T* __restrict__ r, const Stage st,
     double* __restrict__ part) {
-    constexpr int U = 1;  // slots whose loads are in flight at a time
     constexpr int kPt = kPtRes;
     const int lb = logicalBlock(bm.nBlocks);
     const Tile tl = bm.at(lb);
     __shared__ Ctl sh;
     __shared__ double tot[4 * PointOf<kPt>::nv];
-    StageRun<kPt> run;
-    run.load(st.in + tl.inst, part, bm.nBlocks, tl.blk0, tl.nBlk);
+    __shared__ double accL[12][kBlock];
     const int C = m.nCells, B = m.nBoundary;
     const size_t E = m.nEntries;
     const T* __restrict__ invD = MatSel<T>::invDiag(m);
     const int wave = waveOf(), lane = threadIdx.x & 63;
     int s = tl.s0 + wave;
-    int nb[U] = {};  // columns of the group of slots at hand
-    auto cols = [&](int s, int k0, int* n) {
-        const int* __restrict__ col = m.col + m.entry0(s) + k0 * kSlice;
-#pragma unroll
-        for (int u = 0; u < U; ++u) n[u] = at32(col + u * kSlice, lane * 4u);
+    int e0 = s < tl.s1 ? m.entry0(s) : 0;
+    int nb = kPad;  // column of the slot at hand
+    // face data read once: past the gathered rows in the L2 where those do not fit
+    auto stream = [&](const double* p) { return MERGED ? at32(p, lane * 8u) : at32s(p, lane * 8u); };
+    auto col = [&](int e0, int k) {
+        const int* p = m.col + e0 + k * kSlice;
+        return MERGED ? at32(p, lane * 4u) : at32s(p, lane * 4u);
     };
-    bool have = s < tl.s1 && s * kSlice + lane < tl.cEnd;
-    if (have) cols(s, 0, nb);
-    run.reduce(&sh, tot, part, bm.nBlocks, tl.blk0, tl.nBlk);
-    run.finish(&sh, tot, tl, st.hist, lb == tl.blk0, st.out + tl.inst);
-    if (pendingOf(&sh) != kPendRes) return;
-    const double* __restrict__ D = __builtin_amdgcn_readfirstlane(sh.dpar) ? D1 : D0;
-    const double xb[3] = {sh.xbar[0], sh.xbar[1], sh.xbar[2]};
-    const double sf = (sh.sigma0 && sh.iCorr == 0) ? 0.0 : 1.0;
+    const Ctl* c;
+    if constexpr (MERGED) {
+        StageRun<kPt> run;
+        run.load(st.in + tl.inst, part, bm.nBlocks, tl.blk0, tl.nBlk);
+        if (s < tl.s1) nb = col(e0, 0);
+        run.reduce(&sh, tot, part, bm.nBlocks, tl.blk0, tl.nBlk);
+        run.finish(&sh, tot, tl, st.hist, lb == tl.blk0, st.out + tl.inst);
+        c = &sh;
+    } else {
+        c = st.in + tl.inst;
+        if (s < tl.s1) nb = col(e0, 0);
+    }
+    if (pendingOf(c) != kPendRes) return;
+    const double* __restrict__ D = __builtin_amdgcn_readfirstlane(c->dpar) ? D1 : D0;
+    const double xb[3] = {c->xbar[0], c->xbar[1], c->xbar[2]};
+    // a cold start's first residual sees the zero initial stress field
+    const double sf = (c->sigma0 && c->iCorr == 0) ? 0.0 : 1.0;
+    SliceAcc<12> sa{accL};
     double acc[12];
-#pragma unroll
-    for (int i = 0; i < 12; ++i) acc[i] = 0.0;
-    for (; s < tl.s1; s += kBlock / 64) {
+    sa.get(acc);
+    while (s < tl.s1) {
         const int P = s * kSlice + lane;
-        if (P >= tl.cEnd) continue;
-        const int e0 = m.entry0(s);
-        const unsigned l8 = lane * 8u, p8 = P * 8u;
-        if (!have) cols(s, 0, nb);
-        have = false;
+        const bool on = P < tl.cEnd;
+        const unsigned l8 = lane * 8u, p8 = (on ? P : tl.cEnd - 1) * 8u;  // no cell: any row, its sums dropped
         double DP[3], GP[9], CP[3], sP[6];
 #pragma unroll
         for (int k = 0; k < 3; ++k) { DP[k] = at32(D + (size_t)k * C, p8); CP[k] = at32(m.cC + (size_t)k * C, p8); }
 #pragma unroll
         for (int k = 0; k < 9; ++k) GP[k] = at32(G + (size_t)k * C, p8);
+        loadsAbove();
         hookeF(GP, 2.0 * ((MU ? at32(m.mu, p8) : m.mu0) * sf), (MU ? at32(m.K, p8) : m.K0) * sf, sP);
         double sum[10] = {};  // div sigma, Rhie-Chow, off-diagonal product, coefficient sum
-        bool hasB = false;
+        unsigned bs = 0;      // slots in which the wavefront has boundary faces
 #pragma unroll 1
-        for (int k0 = 0; k0 < W; k0 += U) {
-            int nx[U] = {};
-            if (k0 + U < W) cols(s, k0 + U, nx);
+        for (int k = 0; k < W; ++k) {
+            const int nx = k + 1 < W ? col(e0, k + 1) : kPad;
+            const size_t e = (size_t)e0 + k * kSlice;
+            const bool v = nb >= 0;
+            bs |= __any(!v && nb != kPad) ? 1u << k : 0u;
+            const unsigned c8 = v ? nb * 8u : p8;
+            double S0r = stream(m.eS + e), S1r = stream(m.eS + E + e), S2r = stream(m.eS + 2 * E + e);
+            double w = stream(m.eW + e), cfr = stream(m.eC + e), ar = stream(m.eA + e);
+            double GN[9], DN[3], CN[3];
 #pragma unroll
-            for (int u = 0; u < U; ++u) {
-                const size_t e = (size_t)e0 + (k0 + u) * kSlice;
-                const bool v = nb[u] >= 0;
-                hasB |= !v && nb[u] != kPad;
-                const int c = v ? nb[u] : P;
-                const unsigned c8 = c * 8u;
-                const double S0r = at32(m.eS + e, l8), S1r = at32(m.eS + E + e, l8), S2r = at32(m.eS + 2 * E + e, l8);
-                const double w = at32(m.eW + e, l8), cfr = at32(m.eC + e, l8), ar = at32(m.eA + e, l8);
-                const double S0 = v ? S0r : 0.0, S1 = v ? S1r : 0.0, S2 = v ? S2r : 0.0;
-                const double cf = v ? cfr : 0.0, a = v ? ar : 0.0;
-                double GN[9], DN[3], CN[3];
+            for (int q = 0; q < 9; ++q) GN[q] = at32(G + (size_t)q * C, c8);
 #pragma unroll
-                for (int q = 0; q < 9; ++q) GN[q] = at32(G + (size_t)q * C, c8);
-#pragma unroll
-                for (int q = 0; q < 3; ++q) {
-                    DN[q] = at32(D + (size_t)q * C, c8);
-                    CN[q] = at32(m.cC + (size_t)q * C, c8);
-                }
-                const double mu2 = 2.0 * ((MU ? at32(m.mu, c8) : m.mu0) * sf);
-                const double KN = (MU ? at32(m.K, c8) : m.K0) * sf;
-                faceTerms(w, S0, S1, S2, cf, a, mu2, KN, sP, GP, DP, CP, GN, DN, CN, sum);
+            for (int q = 0; q < 3; ++q) {
+                DN[q] = at32(D + (size_t)q * C, c8);
+                CN[q] = at32(m.cC + (size_t)q * C, c8);
             }
-#pragma unroll
-            for (int u = 0; u < U; ++u) nb[u] = nx[u];
+            const double muN = MU ? at32(m.mu, c8) : m.mu0, KNr = MU ? at32(m.K, c8) : m.K0;
+            if (!MERGED) loadedHere(S0r, S1r, S2r, w, cfr, ar, GN, DN, CN);
+            const double S0 = v ? S0r : 0.0, S1 = v ? S1r : 0.0, S2 = v ? S2r : 0.0;
+            const double cf = v ? cfr : 0.0, a = v ? ar : 0.0;
+            const double mu2 = 2.0 * (muN * sf), KN = KNr * sf;
+            faceTerms(w, S0, S1, S2, cf, a, mu2, KN, sP, GP, DP, CP, GN, DN, CN, sum);
+            nb = nx;
         }
-        if (__any(hasB)) {  // boundary slots: the loads of a wavefront with any at once, zero area elsewhere
-#pragma unroll 1
-            for (int k0 = 0; k0 < W; k0 += W / 2) {
-                int n[W / 2];
-                double Sb[W / 2][3], sb[W / 2][6];
+        for (; bs; bs &= bs - 1) {
+            const int k = __builtin_ctz(bs);
+            const size_t e = (size_t)e0 + k * kSlice;
+            const int n = col(e0, k);
+            if (n >= 0 || n == kPad) continue;
+            const unsigned b8 = (-1 - n) * 8u;
+            double S[3], sb[6];
 #pragma unroll
-                for (int u = 0; u < W / 2; ++u) {
-                    const size_t e = (size_t)e0 + (k0 + u) * kSlice;
-                    n[u] = at32(m.col + e, lane * 4u);
-                    const bool v = n[u] < 0 && n[u] != kPad;
-                    const unsigned b8 = v ? (-1 - n[u]) * 8u : 0u;
+            for (int q = 0; q < 3; ++q) S[q] = at32(m.eS + (size_t)q * E + e, l8);
 #pragma unroll
-                    for (int q = 0; q < 3; ++q) Sb[u][q] = at32(m.eS + (size_t)q * E + e, l8);
-#pragma unroll
-                    for (int q = 0; q < 6; ++q) sb[u][q] = at32(sigb + (size_t)q * B, b8);
-                }
-#pragma unroll
-                for (int u = 0; u < W / 2; ++u) {
-                    if (n[u] >= 0 || n[u] == kPad) continue;
-                    sum[0] += dot3(Sb[u][0], sb[u][0], Sb[u][1], sb[u][1], Sb[u][2], sb[u][2]);
-                    sum[1] += dot3(Sb[u][0], sb[u][1], Sb[u][1], sb[u][3], Sb[u][2], sb[u][4]);
-                    sum[2] += dot3(Sb[u][0], sb[u][2], Sb[u][1], sb[u][4], Sb[u][2], sb[u][5]);
-                }
-            }
+            for (int q = 0; q < 6; ++q) sb[q] = at32(sigb + (size_t)q * B, b8);
+            sum[0] += dot3(S[0], sb[0], S[1], sb[1], S[2], sb[2]);
+            sum[1] += dot3(S[0], sb[1], S[1], sb[3], S[2], sb[4]);
+            sum[2] += dot3(S[0], sb[2], S[1], sb[4], S[2], sb[5]);
         }
         const double dg = at32(m.diag, p8);
-        const T iDP = at32(invD, P * (unsigned)sizeof(T));
+        const T iDP = at32(invD, p8 / (unsigned)(8 / sizeof(T)));
         const double rowsum = dg - sum[9];
         double src[3] = {0.0, 0.0, 0.0};
-        if (m.fext) {
+        if (m.fext && on) {
 #pragma unroll
             for (int j = 0; j < 3; ++j) src[j] = m.fext[(size_t)j * C + P] - (m.iner ? m.iner[P] * DP[j] : 0.0);
         }
+        sa.get(acc);
+        if (on) {
 #pragma unroll
-        for (int j = 0; j < 3; ++j) {
-            const double R = (sum[j] + sum[3 + j]) + src[j];
-            const double MD = fmaT(dg, DP[j], -sum[6 + j]);
-            acc[j] += fabs(R);
-            acc[3 + j] += fabs(fmaT(-rowsum, xb[j], MD));
-            acc[6 + j] += fabs(fmaT(-rowsum, xb[j], MD + R));
-            const T rT = (T)R;
-            put32(r + (size_t)j * C, P * (unsigned)sizeof(T), rT);
-            const T z = iDP * rT;
-            acc[9 + j] += (double)z * (double)rT;
+            for (int j = 0; j < 3; ++j) {
+                const double R = (sum[j] + sum[3 + j]) + src[j];
+                const double MD = fmaT(dg, DP[j], -sum[6 + j]);
+                acc[j] += fabs(R);
+                acc[3 + j] += fabs(fmaT(-rowsum, xb[j], MD));
+                acc[6 + j] += fabs(fmaT(-rowsum, xb[j], MD + R));
+                const T rT = (T)R;
+                put32(r + (size_t)j * C, P * (unsigned)sizeof(T), rT);
+                const T z = iDP * rT;
+                acc[9 + j] += (double)z * (double)rT;
+            }
         }
+        s += kBlock / 64;
+        if (s >= tl.s1) break;
+        sa.put(acc);
+        e0 = m.entry0(s);
+        nb = col(e0, 0);
     }
     storeBlockPartials<12, 0>(acc, part, kOffRes, lb, bm.nBlocks);
 }
+
 // The gradient step in one launch (no Aitken relaxation, no sub-meshes): the
 // tile's boundary faces go into a queue in LDS, its threads update them one
 // face each (k_grad_bnd_pre), the cells form their gradients (k_grad), and the
 // threads return to the faces (k_grad_bnd_post).  Workgroup barriers order the
 // three through the workgroup's own global stores.  Two slots' gathers in
 // flight at a time (three, with the cell's own values loaded over the first
-// face update, measured the same up to 64,000 cells and worse above).  512
-// cells: 16 us, and 10 + 6 + 4 us in three launches.
+// face update, measured the same up to 64,000 cells and worse above; face
+// loads issued before the scalars are known slowed the launches that find
+// nothing to do).  Of 16 us at 512 cells the faces took 5.6 (queue, update,
+// return); with a ballot per slot for the queue and a face's loads at once it
+// is 14.7, and 10 + 6 + 4 us in three launches.  24 boxes: 41 -> 38 us.  The
+// update in the cells' own lanes, without queue or barriers, took 19.4 and 45.
 template <typename T, int W>
-__global__ __launch_bounds__(kBlock, 3) void k_grad_m(
+__global__ __launch_bounds__(kBlock, 4) void k_grad_m(
     const DevMesh m, const BlockMap bm, double* __restrict__ D0, const T* __restrict__ x, double* __restrict__ D1,
     double* G, double* Db, const double* __restrict__ Dold, const Stage st, double* __restrict__ part,
     const BndBufs bb) {
@@ -485,21 +504,22 @@ __global__ __launch_bounds__(kBlock, 3) void k_grad_m(
     const Tile tl = bm.at(lb);
     __shared__ Ctl sh;
     __shared__ double tot[4 * PointOf<kPt>::nv];
-    __shared__ int qn, qFace[kBlock * W], qCell[kBlock * W];
+    __shared__ int qCount[kWaves], qFace[kBlock * W], qCell[kBlock * W];
     StageRun<kPt> run;
     run.load(st.in + tl.inst, part, bm.nBlocks, tl.blk0, tl.nBlk);
     const int C = m.nCells, B = m.nBoundary;
     const int wave = waveOf(), lane = threadIdx.x & 63;
-    int nb[W] = {};
+    int nb[W];
     auto cols = [&](int s) {
-        const int* __restrict__ col = m.col + m.entry0(s);
 #pragma unroll
-        for (int k = 0; k < W; ++k) nb[k] = at32(col + k * kSlice, lane * 4u);
+        for (int k = 0; k < W; ++k) nb[k] = kPad;
+        if (s < tl.s1 && s * kSlice + lane < tl.cEnd) {
+            const int* __restrict__ col = m.col + m.entry0(s);
+#pragma unroll
+            for (int k = 0; k < W; ++k) nb[k] = at32(col + k * kSlice, lane * 4u);
+        }
     };
-    {
-        const int s = tl.s0 + wave;
-        if (s < tl.s1 && s * kSlice + lane < tl.cEnd) cols(s);
-    }
+    cols(tl.s0 + wave);
     run.reduce(&sh, tot, part, bm.nBlocks, tl.blk0, tl.nBlk);
     run.finish(&sh, tot, tl, st.hist, lb == tl.blk0, st.out + tl.inst);
     if (pendingOf(&sh) != kPendGrad) return;
@@ -515,24 +535,40 @@ __global__ __launch_bounds__(kBlock, 3) void k_grad_m(
         const int P = s * kSlice + lane;
         const bool on = s < tl.s1 && P < tl.cEnd;
         const unsigned p8 = P * 8u, pT = P * (unsigned)sizeof(T);
-        if (threadIdx.x == 0) qn = 0;
-        __syncthreads();
-        if (on) {
-            if (sb != tl.s0) cols(s);
-#pragma unroll
-            for (int k = 0; k < W; ++k)
-                if (nb[k] < 0 && nb[k] != kPad) {
-                    const int at = atomicAdd(&qn, 1);
-                    qFace[at] = -1 - nb[k];
-                    qCell[at] = P;
-                }
+        if (sb != tl.s0) {
+            __syncthreads();  // the queue is reused
+            cols(s);
         }
-        double DP[3], DnP[3], CP[3], Mi[6];
+        // a wavefront's boundary faces, in its own part of the queue
+        int n = 0;
+#pragma unroll
+        for (int k = 0; k < W; ++k) {
+            const bool isB = nb[k] < 0 && nb[k] != kPad;
+            const unsigned long long mask = __ballot(isB);
+            if (isB) {
+                const int at = wave * (kSlice * W) + n + __popcll(mask & ((1ull << lane) - 1));
+                qFace[at] = -1 - nb[k];
+                qCell[at] = P;
+            }
+            n += __popcll(mask);
+        }
+        if (lane == 0) qCount[wave] = n;
         __syncthreads();
-        const int nq = qn;
+        // its parts end to end
+        const int q0 = qCount[0], q1 = q0 + qCount[1], q2 = q1 + qCount[2], nq = q2 + qCount[3];
+        auto place = [&](int i) {
+            const int w = (i >= q0) + (i >= q1) + (i >= q2);
+            return w * (kSlice * W) + i - (w == 0 ? 0 : w == 1 ? q0 : w == 2 ? q1 : q2);
+        };
+        double DP[3], DnP[3], CP[3], Mi[6];
         for (int i = threadIdx.x; i < nq; i += kBlock) {
-            const int b = qFace[i], Pf = qCell[i];
+            const int at = place(i), b = qFace[at], Pf = qCell[at];
+            FaceIn f;
+            f.fixed(m, b);
+            f.fields(m, b, bb.g, Db);
             double Du[3], Dr[3], Gold[9], Dbn[3], sn[3];
+#pragma unroll
+            for (int q = 0; q < 9; ++q) Gold[q] = at32(G + (size_t)q * C, Pf * 8u);
 #pragma unroll
             for (int k = 0; k < 3; ++k) {
                 const double d0 = at32(D + (size_t)k * C, Pf * 8u);
@@ -540,13 +576,11 @@ __global__ __launch_bounds__(kBlock, 3) void k_grad_m(
                 Du[k] = d0 + xv;
                 Dr[k] = fmaT(ra, xv, d0);
             }
-#pragma unroll
-            for (int q = 0; q < 9; ++q) Gold[q] = at32(G + (size_t)q * C, Pf * 8u);
-            bndPreFace(m, u, b, m.bType[b], Du, Dr, Gold, Db, bb.g, nullptr, nullptr, Dbn, sn);
+            bndPreFace(m, u, b, f, Du, Dr, Gold, nullptr, nullptr, Dbn, sn);
 #pragma unroll
             for (int q = 0; q < 3; ++q) {
-                Db[(size_t)q * B + b] = Dbn[q];
-                bb.snb[(size_t)q * B + b] = sn[q];
+                put32(Db + (size_t)q * B, b * 8u, Dbn[q]);
+                put32(bb.snb + (size_t)q * B, b * 8u, sn[q]);
             }
         }
         __syncthreads();
@@ -567,19 +601,32 @@ __global__ __launch_bounds__(kBlock, 3) void k_grad_m(
             const int* __restrict__ colS = m.col + m.entry0(s);
 #pragma unroll 1
             for (int k0 = 0; k0 < W; k0 += U) {
+                int n[U];
+                double cN[U][3], dN[U][3];
+                T xN[U][3];
+#pragma unroll
+                for (int u = 0; u < U; ++u) n[u] = at32(colS + (k0 + u) * kSlice, lane * 4u);
 #pragma unroll
                 for (int u = 0; u < U; ++u) {
-                    const int n = at32(colS + (k0 + u) * kSlice, lane * 4u);
-                    const bool v = n >= 0;
-                    hasB |= !v && n != kPad;
-                    const int c = v ? n : P;
+                    const int c = n[u] >= 0 ? n[u] : P;
                     const unsigned c8 = c * 8u, cT = c * (unsigned)sizeof(T);
+#pragma unroll
+                    for (int q = 0; q < 3; ++q) {
+                        cN[u][q] = at32(m.cC + (size_t)q * C, c8);
+                        xN[u][q] = at32(x + (size_t)q * C, cT);
+                        dN[u][q] = at32(D + (size_t)q * C, c8);
+                    }
+                }
+                loadsAbove();
+#pragma unroll
+                for (int u = 0; u < U; ++u) {
+                    const bool v = n[u] >= 0;
+                    hasB |= !v && n[u] != kPad;
                     double d[3], dv[3];
 #pragma unroll
                     for (int q = 0; q < 3; ++q) {
-                        d[q] = at32(m.cC + (size_t)q * C, c8) - CP[q];
-                        const double xN = hasX ? (double)at32(x + (size_t)q * C, cT) : 0.0;
-                        dv[q] = fmaT(ra, xN, at32(D + (size_t)q * C, c8)) - DnP[q];
+                        d[q] = cN[u][q] - CP[q];
+                        dv[q] = fmaT(ra, hasX ? (double)xN[u][q] : 0.0, dN[u][q]) - DnP[q];
                     }
                     const double dd = dot3(d[0], d[0], d[1], d[1], d[2], d[2]);
                     const double rr = v ? 1.0 / dd : 0.0;
@@ -637,13 +684,19 @@ __global__ __launch_bounds__(kBlock, 3) void k_grad_m(
         }
         __syncthreads();
         for (int i = threadIdx.x; i < nq; i += kBlock) {
-            const int b = qFace[i], Pf = qCell[i];
-            double Gn[9];
+            const int at = place(i), b = qFace[at], Pf = qCell[at];
+            const int type = at32(m.bType, b * 4u);
+            double Gn[9], n[3], val[3], sn[3];
+#pragma unroll
+            for (int q = 0; q < 3; ++q) {
+                n[q] = at32(m.bN + (size_t)q * B, b * 8u);
+                val[q] = at32(m.bVal + (size_t)q * B, b * 8u);
+                sn[q] = at32(bb.snb + (size_t)q * B, b * 8u);
+            }
 #pragma unroll
             for (int q = 0; q < 9; ++q) Gn[q] = at32(G + (size_t)q * C, Pf * 8u);
-            bndPostFace(m, 0, false, b, m.bType[b], Pf, Gn, bb.snb, bb.Gb, bb.sigb, bb.g);
+            bndPostFace(m, 0, false, b, type, Pf, Gn, n, val, sn, bb.Gb, bb.sigb, bb.g);
         }
-        __syncthreads();  // the queue is reused
     }
     storeBlockPartials<6, 3>(acc, part, kOffGrad, lb, bm.nBlocks);
 }

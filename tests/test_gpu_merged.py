@@ -73,12 +73,16 @@ def test_merged_equals_general(ctx, precision, precond, law):
 
 
 @pytest.mark.parametrize("relax", [0.0, 0.8])
-def test_line_between_the_two(ctx, relax):
-    # one tile per slice: 1,024 tiles are merged, 1,025 are not; the batch of both is not
+@pytest.mark.parametrize("law", ["uniform", "cells"])
+@pytest.mark.parametrize("tets", [False, True])
+def test_line_between_the_two(ctx, relax, law, tets):
+    # one tile per slice: 1,024 tiles are merged, 1,025 are not (one slot count
+    # still); the batch of both is not, and with tetrahedra has no single slot count
     from solids4foam_amd.batch import Batch
-    print(f"[merged] line relax={relax}", flush=True)
-    members = [_box(ctx, n, 2, tiles=(65536, 1)) for n in ((64, 32, 32), (64, 41, 25))]
-    opts = dict(CAPPED, precision=1, preconditioner=0, nCorrectors=4, pcgMaxIter=30, relaxD=relax)
+    print(f"[merged] line relax={relax} {law} tets={tets}", flush=True)
+    members = [_box(ctx, n, 2, law, tiles=t) for n, t in (((64, 32, 32), (65536, 1)), ((64, 41, 25), (65536, 1)))]
+    members.append(_tets(ctx) if tets else _box(ctx, (23, 21, 17), 4, law, tiles=(3, 4)))  # many slices a tile
+    opts = dict(CAPPED, precision=0, preconditioner=0, nCorrectors=4, pcgMaxIter=30, relaxD=relax)
     alone = [m.solve(**opts) for m in members]
     b = Batch(ctx)
     for m in members:
