@@ -226,27 +226,42 @@ __global__ __launch_bounds__(kBlock) void k_mg0_down(const DevMesh m, const Bloc
             mg0DownRowAll<T, 4>(m, P, e0, lane, C, b, r, w);
             continue;
         }
-        const T iD = invD[P];
-        T xP[3], y[3];
+        // some components, or another slot count: as in k_spmvp
+        const T iD = invD[P], dP = dg[P];
+        T bP[3] = {}, y[3] = {};
 #pragma unroll
         for (int j = 0; j < 3; ++j) {
-            xP[j] = act[j] ? w * iD * b[(size_t)j * C + P] : (T)0;
-            y[j] = dg[P] * xP[j];
+            if (!act[j]) continue;
+            bP[j] = b[(size_t)j * C + P];
+            y[j] = rounded(dP * (w * iD * bP[j]));
         }
-        for (int k = 0; k < width; ++k) {
-            const int e = e0 + k * kSlice + lane;
-            const int n = m.col[e];
-            if (n >= 0) {
-                const T a = A[e];
-                const T iDn = invD[n];
+        for (int k0 = 0; k0 < width; k0 += kRowChunk) {
+            int n[kRowChunk];
+            T av[kRowChunk], iDn[kRowChunk];
 #pragma unroll
-                for (int j = 0; j < 3; ++j)
-                    if (act[j]) y[j] -= a * (w * iDn * b[(size_t)j * C + n]);
+            for (int u = 0; u < kRowChunk; ++u) {
+                const int e = e0 + (k0 + u < width ? k0 + u : k0) * kSlice + lane;
+                const int ne = ldS(m.col + e);
+                const T ae = ldS(A + e);
+                const bool v = k0 + u < width && ne >= 0;
+                n[u] = v ? ne : P;
+                av[u] = v ? ae : (T)0;
+            }
+#pragma unroll
+            for (int u = 0; u < kRowChunk; ++u) iDn[u] = invD[n[u]];
+#pragma unroll
+            for (int j = 0; j < 3; ++j) {
+                if (!act[j]) continue;
+                T bn[kRowChunk];
+#pragma unroll
+                for (int u = 0; u < kRowChunk; ++u) bn[u] = b[(size_t)j * C + n[u]];
+#pragma unroll
+                for (int u = 0; u < kRowChunk; ++u) y[j] = fmaT(-av[u], w * iDn[u] * bn[u], y[j]);
             }
         }
         T rP[3];  // a converged component's residual is not read
 #pragma unroll
-        for (int j = 0; j < 3; ++j) rP[j] = act[j] ? b[(size_t)j * C + P] - y[j] : (T)0;
+        for (int j = 0; j < 3; ++j) rP[j] = act[j] ? bP[j] - y[j] : (T)0;
         r[P] = row4(rP[0], rP[1], rP[2]);
     }
 }

@@ -956,7 +956,10 @@ inline bool canMerge(const DevMesh& dm, int maxTiles) { return maxTiles <= kMerg
 
 template <int POINT>
 void launchFin(const BlockMap& bm, int nFin, const Chain& c, const Ctl* in, Ctl* out, const double* part, hipStream_t s) {
-    hipLaunchKernelGGL((k_fin<POINT>), dim3(nFin), dim3(kFinBlock), 0, s, bm, c.at(in, out), part);
+    if (bm.nBlocks > kFinWideTiles)
+        hipLaunchKernelGGL((k_fin_wide<POINT>), dim3(nFin), dim3(4 * kFinBlock), 0, s, bm, c.at(in, out), part);
+    else
+        hipLaunchKernelGGL((k_fin<POINT>), dim3(nFin), dim3(kFinBlock), 0, s, bm, c.at(in, out), part);
 }
 
 // search direction + SpMV, alpha, solution / residual update of one PCG
@@ -4672,17 +4675,26 @@ s4f_status s4f_ldu_create(s4f_ctx* ctx, int32_t nCells, int32_t nFaces, const in
         }
         h.nSlices = (nCells + kSlice - 1) / kSlice;
         h.sliceStart.resize((size_t)h.nSlices + 1);
-        h.sliceWidth.resize(h.nSlices);
+        h.sliceWidth.assign(h.nSlices, 0);
+        long long slots = 0;
+        int wmax = 0;
+        for (int sI = 0; sI < h.nSlices; ++sI) {
+            for (int l = 0; l < kSlice; ++l) {
+                const int c = sI * kSlice + l;
+                if (c < nCells) h.sliceWidth[sI] = std::max(h.sliceWidth[sI], cnt[c]);
+            }
+            slots += h.sliceWidth[sI];
+            wmax = std::max(wmax, h.sliceWidth[sI]);
+        }
+        // the slices of a mesh's boundary have a slot or two less: one slot
+        // count for all (empty slots) opens the merged launch sequence, while
+        // it costs at most a quarter more entries
+        const int wUni = wmax <= 4 ? 4 : 6;
+        if (wmax <= 6 && 4LL * wUni * h.nSlices <= 5 * slots) std::fill(h.sliceWidth.begin(), h.sliceWidth.end(), wUni);
         size_t E = 0;
         for (int sI = 0; sI < h.nSlices; ++sI) {
             h.sliceStart[sI] = (int)E;
-            int wmax = 0;
-            for (int l = 0; l < kSlice; ++l) {
-                const int c = sI * kSlice + l;
-                if (c < nCells) wmax = std::max(wmax, cnt[c]);
-            }
-            h.sliceWidth[sI] = wmax;
-            E += (size_t)wmax * kSlice;
+            E += (size_t)h.sliceWidth[sI] * kSlice;
         }
         h.sliceStart[h.nSlices] = (int)E;
         h.col.assign(E, kPad);

@@ -152,6 +152,7 @@ __device__ __forceinline__ double overWaves(const double* out, int i) {
 }
 
 constexpr int kFinBlock = 256;
+constexpr int kFinWideTiles = 4096;
 
 // Block partials are stored value-major: value i of logical block lb sits at
 // part[i * nb + lb] (nb = the launch's logical block count), so a finalize
@@ -525,6 +526,13 @@ __device__ __forceinline__ void loadedHere(double& a, double& b, double& c, doub
                    "+v"(h[2]), "+v"(i[0]), "+v"(i[1]), "+v"(i[2]));
 }
 
+__device__ __forceinline__ void loadedHere(double* x) {
+    asm volatile(""
+                 : "+v"(x[0]), "+v"(x[1]), "+v"(x[2]), "+v"(x[3]), "+v"(x[4]), "+v"(x[5]), "+v"(x[6]), "+v"(x[7]),
+                   "+v"(x[8]), "+v"(x[9]), "+v"(x[10]), "+v"(x[11]), "+v"(x[12]), "+v"(x[13]), "+v"(x[14]),
+                   "+v"(x[15]), "+v"(x[16]), "+v"(x[17]), "+v"(x[18]), "+v"(x[19]), "+v"(x[20]), "+v"(x[21]),
+                   "+v"(x[22]), "+v"(x[23]));
+}
 __device__ __forceinline__ void loadedHere(double (*a)[3], double (*b)[3], double (*c)[3], double* s) {
     asm volatile(""
                  : "+v"(a[0][0]), "+v"(a[0][1]), "+v"(a[0][2]), "+v"(a[1][0]), "+v"(a[1][1]), "+v"(a[1][2]),
@@ -675,6 +683,12 @@ __global__ __launch_bounds__(kBlock) void k_residual(const DevMesh m, const Bloc
     storeBlockPartials<12, 0>(acc, part, kOffRes, lb, bm.nBlocks);
 }
 
+// Slots of a row whose loads are in flight together where the row's slot count
+// is not compiled in.  One component of a 7-point matrix, 272,640 rows, FP64:
+// 13.0 us slot by slot, 10.4 six at a time; two of three components active, FP32,
+// 128^3 cells: 66 -> 51 us (and 53 -> 33 for the V-cycle's first residual).
+constexpr int kRowChunk = 6;
+
 // Row of the fused direction update + SpMV with all three components active
 // and a compile-time slot count W: every load of the row is issued without a
 // branch (invalid slots gather the row's own cell and contribute zero), so
@@ -732,7 +746,7 @@ __device__ __forceinline__ void spmvpRowAll(const DevMesh& m, int P, int e0, int
 // reduce = 0 it is a plain q = M p (s4f_spmv3).
 // ---------------------------------------------------------------------------
 template <typename T, bool MG>
-__global__ __launch_bounds__(kBlock) void k_spmvp(const DevMesh m, const BlockMap bm, const T* __restrict__ r,
+__global__ __launch_bounds__(kBlock, 5) void k_spmvp(const DevMesh m, const BlockMap bm, const T* __restrict__ r,
                                                   T* pA, T* pB, T* __restrict__ q, const Ctl* __restrict__ ctlAll,
                                                   double* __restrict__ part, int reduce,
                                                   const T* __restrict__ zArr) {
@@ -754,13 +768,6 @@ __global__ __launch_bounds__(kBlock) void k_spmvp(const DevMesh m, const BlockMa
                          reduce ? ctl->active[2] != 0 : true};
     const bool all = reduce && act[0] && act[1] && act[2];
     const T be[3] = {reduce ? (T)ctl->beta[0] : (T)0, reduce ? (T)ctl->beta[1] : (T)0, reduce ? (T)ctl->beta[2] : (T)0};
-    // direction component of cell c
-    auto dir = [&](int j, int c) -> T {
-        const size_t i = (size_t)j * C + c;
-        if (!reduce) return pOld[i];
-        const T z = MG ? zArr[i] : invD[c] * r[i];
-        return first ? z : z + be[j] * pOld[i];
-    };
     double acc[3] = {0, 0, 0};
     const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
     for (int s = tl.s0 + wave; s < tl.s1; s += kBlock / 64) {
@@ -776,21 +783,53 @@ __global__ __launch_bounds__(kBlock) void k_spmvp(const DevMesh m, const BlockMa
             spmvpRowAll<T, 4, MG>(m, P, e0, lane, C, r, pOld, zArr, pNew, q, first, be, acc);
             continue;
         }
-        T pP[3], y[3];
-        const T d = dg[P];
+        // some components, or another slot count: kRowChunk slots' loads in
+        // flight at a time (a slot past the row or empty reads the row's own
+        // cell with a zero coefficient), the active components only
+        auto dir = [&](int j, T z0, T iD, T o) -> T {
+            if (!reduce) return o;
+            const T z = MG ? z0 : iD * z0;
+            return first ? z : z + be[j] * o;
+        };
+        const T* __restrict__ src = MG ? zArr : r;
+        const bool diagZ = !MG && reduce;
+        T pP[3] = {}, y[3] = {};
+        const T d = dg[P], iDP = diagZ ? invD[P] : (T)0;
 #pragma unroll
         for (int j = 0; j < 3; ++j) {
-            pP[j] = act[j] ? dir(j, P) : (T)0;
-            y[j] = d * pP[j];
+            if (!act[j]) continue;
+            const size_t i = (size_t)j * C + P;
+            pP[j] = dir(j, reduce ? src[i] : (T)0, iDP, pOld[i]);
+            y[j] = rounded(d * pP[j]);
         }
-        for (int k = 0; k < width; ++k) {
-            const int e = e0 + k * kSlice + lane;
-            const int n = m.col[e];
-            if (n >= 0) {
-                const T a = A[e];
+        for (int k0 = 0; k0 < width; k0 += kRowChunk) {
+            int c[kRowChunk];
+            T av[kRowChunk], iD[kRowChunk];
 #pragma unroll
-                for (int j = 0; j < 3; ++j)
-                    if (act[j]) y[j] -= a * dir(j, n);
+            for (int u = 0; u < kRowChunk; ++u) {
+                const int e = e0 + (k0 + u < width ? k0 + u : k0) * kSlice + lane;
+                const int n = ldS(m.col + e);
+                const T ae = ldS(A + e);
+                const bool v = k0 + u < width && n >= 0;
+                c[u] = v ? n : P;
+                av[u] = v ? ae : (T)0;
+            }
+            if (diagZ) {
+#pragma unroll
+                for (int u = 0; u < kRowChunk; ++u) iD[u] = invD[c[u]];
+            }
+#pragma unroll
+            for (int j = 0; j < 3; ++j) {
+                if (!act[j]) continue;
+                T z[kRowChunk], o[kRowChunk];
+#pragma unroll
+                for (int u = 0; u < kRowChunk; ++u) {
+                    const size_t i = (size_t)j * C + c[u];
+                    z[u] = reduce ? src[i] : (T)0;
+                    o[u] = pOld[i];
+                }
+#pragma unroll
+                for (int u = 0; u < kRowChunk; ++u) y[j] = fmaT(-av[u], dir(j, z[u], iD[u], o[u]), y[j]);
             }
         }
 #pragma unroll
@@ -1713,6 +1752,69 @@ __global__ __launch_bounds__(kFinBlock) void k_fin(const BlockMap bm, const Stag
     StageRun<POINT> run;
     run.load(st.in + inst, part, bm.nBlocks, tl.blk0, tl.nBlk);
     run.reduce(&sh, tot, part, bm.nBlocks, tl.blk0, tl.nBlk);
+    run.finish(&sh, tot, tl, st.hist, true, st.out + inst);
+}
+
+// The same on four times the threads, for launches of more than kFinWideTiles
+// tiles: an instance of more has its rows split into four runs, each reduced as
+// k_fin does and the four added in order (one of fewer keeps k_fin's order, and
+// its bits, in the first).  Measured for 12, 6 and 3 values, k_fin -> wide: 8,192
+// tiles (128^3 cells) 20.6 -> 18.6, 16.0 -> 11.9 (points before the outer step
+// 12.8 -> 8.8), 10.4 -> 5.6 us, then bound by what one CU reads from beyond its
+// L2; 2,213 tiles 6.4 -> 6.9, 5.5 -> 7.5, 4.8 -> 5.4.
+template <int POINT>
+__global__ __launch_bounds__(4 * kFinBlock) void k_fin_wide(const BlockMap bm, const Stage st,
+                                                            const double* __restrict__ part) {
+    typedef PointOf<POINT> Pt;
+    const int inst = bm.finInst ? bm.finInst[blockIdx.x] : (int)blockIdx.x;
+    __shared__ Ctl sh;
+    __shared__ double run4[4][4 * Pt::nv], tot[4 * Pt::nv];
+    const Tile tl{inst, 0, 0, 0, bm.iBlk0[inst], bm.iNBlk[inst], bm.iNCell[inst], 0};
+    constexpr int nw = (int)(sizeof(Ctl) / 8);
+    if ((int)threadIdx.x < nw)
+        reinterpret_cast<long long*>(&sh)[threadIdx.x] = reinterpret_cast<const long long*>(st.in + inst)[threadIdx.x];
+    const int g = threadIdx.x / kFinBlock, t = threadIdx.x % kFinBlock, nb = bm.nBlocks;
+    const int len = tl.nBlk > kFinWideTiles ? (tl.nBlk + 3) / 4 : tl.nBlk;
+    const int b1 = tl.nBlk < (g + 1) * len ? tl.nBlk : (g + 1) * len;
+    const double* col = part + (size_t)Pt::off * nb + tl.blk0;
+    constexpr int kRows = 24 / Pt::nv;  // rows whose loads are in flight together
+    double v[Pt::nv];
+#pragma unroll
+    for (int i = 0; i < Pt::nv; ++i) v[i] = 0.0;
+    for (int b = g * len + t; b < b1; b += kRows * kFinBlock) {
+        double x[24];
+#pragma unroll
+        for (int r = 0; r < kRows; ++r)
+#pragma unroll
+            for (int i = 0; i < Pt::nv; ++i) {
+                const int row = b + r * kFinBlock;
+                x[r * Pt::nv + i] = col[(size_t)i * nb + (row < b1 ? row : b)];
+            }
+        loadedHere(x);
+#pragma unroll
+        for (int r = 0; r < kRows; ++r)
+#pragma unroll
+            for (int i = 0; i < Pt::nv; ++i) {
+                const double xv = b + r * kFinBlock < b1 ? x[r * Pt::nv + i] : 0.0;
+                v[i] = i < Pt::nmax ? nanMax(v[i], xv) : v[i] + xv;
+            }
+    }
+    waveReduceAll<Pt::nv, Pt::nmax>(v, run4[g], (t >> 6));
+    __syncthreads();
+    if (threadIdx.x < Pt::nv) {
+        const int i = threadIdx.x;
+        double s = overWaves<Pt::nmax>(run4[0], i);
+#pragma unroll
+        for (int q = 1; q < 4; ++q) {
+            const double x = overWaves<Pt::nmax>(run4[q], i);
+            s = i < Pt::nmax ? nanMax(s, x) : s + x;
+        }
+        tot[4 * i] = s;
+#pragma unroll
+        for (int q = 1; q < 4; ++q) tot[4 * i + q] = 0.0;
+    }
+    __syncthreads();
+    StageRun<POINT> run;
     run.finish(&sh, tot, tl, st.hist, true, st.out + inst);
 }
 

@@ -116,3 +116,34 @@ def test_vcycle_iteration_counts(ctx, n, counts):
         got = m.solve(preconditioner=precond, **opts)["innerTotal"]
         print(f"[vcycle] {n} precond={precond}: {got}", flush=True)
         assert abs(got - want) <= 3
+
+
+@pytest.mark.parametrize("n", [(1, 1, 1), (2, 1, 1), (40, 1, 1), (9, 8, 1), (7, 6, 5), (16, 16, 17), (33, 32, 32)])
+@pytest.mark.parametrize("wide", [False, True])
+@pytest.mark.parametrize("mixed", [False, True])
+def test_ldu_slot_counts(ctx, n, wide, mixed):
+    # one slot count (padded, merged launches), and rows of up to seven slots (general);
+    # a manufactured solution, diagonally dominant by a tenth: the error is bounded by
+    # the residual's 1e-11 (FP32: 1e-5) of |b| times the condition number of about 20
+    from solids4foam_amd.solid import LduSolver
+    c = np.arange(n[0] * n[1] * n[2]).reshape(n[2], n[1], n[0])
+    lower = np.concatenate([c[:, :, :-1].ravel(), c[:, :-1].ravel(), c[:-1].ravel()])
+    upper = np.concatenate([c[:, :, 1:].ravel(), c[:, 1:].ravel(), c[1:].ravel()])
+    if wide:
+        if c.size < 20:
+            pytest.skip("no room for far neighbours")
+        far = np.arange(0, c.size - 13, 7)
+        far = far[~np.isin(far * c.size + far + 13, lower * c.size + upper)]
+        lower, upper = np.concatenate([lower, far]), np.concatenate([upper, far + 13])
+    order = np.lexsort((upper, lower))
+    lower, upper = lower[order], upper[order]
+    rng = np.random.default_rng(c.size)
+    a = rng.uniform(0.5, 1.5, lower.size)
+    off = np.bincount(lower, a, c.size) + np.bincount(upper, a, c.size)
+    diag = 1.1 * off + 0.1
+    psi = rng.normal(size=c.size)
+    src = diag * psi - np.bincount(lower, a * psi[upper], c.size) - np.bincount(upper, a * psi[lower], c.size)
+    tol = 1e-6 if mixed else 1e-12
+    got, info = LduSolver(ctx, c.size, lower, upper).solve(diag, -a, src, np.zeros(c.size), tolerance=tol, mixed=mixed)
+    print(f"[ldu] {n} wide={wide} mixed={mixed}: {info['nIterations']} iterations", flush=True)
+    assert np.linalg.norm(got - psi) <= (2e-4 if mixed else 2e-10) * max(1.0, np.linalg.norm(psi))
