@@ -1828,6 +1828,39 @@ __global__ __launch_bounds__(kFinBlock) void k_fin_init(const BlockMap bm, Ctl* 
         for (int j = 0; j < 3; ++j) ctlAll[inst].xbar[j] = tot[3 + j] / (double)bm.iNCell[inst];
 }
 
+// n rows of K components from component-major storage (K arrays `stride` apart)
+template <int K>
+__global__ __launch_bounds__(kBlock) void k_to_rows(const double* __restrict__ src, size_t stride, int n,
+                                                    double* __restrict__ out) {
+    for (int i = blockIdx.x * kBlock + threadIdx.x; i < n * K; i += gridDim.x * kBlock)
+        out[i] = src[(size_t)(i % K) * stride + i / K];
+}
+
+// a symmetric LDU matrix into the sliced-ELL entries of its faces (-upper) ...
+__global__ __launch_bounds__(kBlock) void k_ldu_faces(int nFaces, const double* __restrict__ upper,
+                                                      const int* __restrict__ own, const int* __restrict__ nei,
+                                                      double* __restrict__ a64, float* __restrict__ a32) {
+    for (int f = blockIdx.x * kBlock + threadIdx.x; f < nFaces; f += gridDim.x * kBlock) {
+        const double a = -upper[f];
+        a64[own[f]] = a;
+        a64[nei[f]] = a;
+        if (a32) {
+            a32[own[f]] = (float)a;
+            a32[nei[f]] = (float)a;
+        }
+    }
+}
+// ... and its diagonal's inverse and FP32 copies
+__global__ __launch_bounds__(kBlock) void k_ldu_diag(int n, const double* __restrict__ d, double* __restrict__ inv,
+                                                     float* __restrict__ d32, float* __restrict__ inv32) {
+    for (int i = blockIdx.x * kBlock + threadIdx.x; i < n; i += gridDim.x * kBlock) {
+        inv[i] = 1.0 / d[i];
+        const float v = (float)d[i];
+        d32[i] = v;
+        inv32[i] = 1.0f / v;
+    }
+}
+
 // stops the instances at the end of their current PCG solve (mixed
 // precision's fallback)
 __global__ void k_ctl_hold(Ctl* __restrict__ c, int n, int hold) {
