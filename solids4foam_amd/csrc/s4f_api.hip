@@ -97,8 +97,10 @@ struct s4f_ctx {
     int children = 0;
     bool destroyPending = false;
     // two chunks each of device and pinned host memory for fields on their way
-    // to the caller (downloadRows), shared by the context's meshes
+    // to the caller (downloadRows), shared by the context's meshes; as large as
+    // the largest fields so far, up to kStageChunk
     std::mutex stageMutex;
+    size_t stageChunk = 0;
     DArr<double> stageDev;
     double* stageHost = nullptr;
     hipEvent_t stageEv[2] = {nullptr, nullptr};
@@ -1055,6 +1057,21 @@ struct RowField {
 };
 void downloadRows(s4f_ctx* ctx, const std::vector<RowField>& fields, hipStream_t s) {
     std::lock_guard<std::mutex> lock(ctx->stageMutex);
+    size_t need = 0, chunk = (size_t)1 << 14;
+    for (const RowField& f : fields) need += (size_t)f.n * f.k;
+    if (need == 0) return;
+    while (chunk < need && chunk < kStageChunk) chunk *= 2;
+    if (chunk > ctx->stageChunk) {  // no transfer is under way: each call waits for its own
+        ctx->stageChunk = 0;
+        if (ctx->stageHost) (void)hipHostFree(ctx->stageHost);
+        ctx->stageHost = nullptr;
+        ctx->stageDev.alloc(2 * chunk);
+        HIP_CHECK(hipHostMalloc((void**)&ctx->stageHost, 2 * chunk * sizeof(double), hipHostMallocDefault));
+        for (hipEvent_t& e : ctx->stageEv)
+            if (!e) HIP_CHECK(hipEventCreateWithFlags(&e, hipEventDisableTiming));
+        ctx->stageChunk = chunk;
+    }
+    chunk = ctx->stageChunk;
     struct Piece {
         double* out;
         size_t at, count;
@@ -1067,9 +1084,9 @@ void downloadRows(s4f_ctx* ctx, const std::vector<RowField>& fields, hipStream_t
         size_t used = 0;
         for (; iField < fields.size(); ++iField, c = 0) {
             const RowField& f = fields[iField];
-            const int n = (int)std::min<size_t>(f.n - c, (kStageChunk - used) / f.k);
+            const int n = (int)std::min<size_t>(f.n - c, (chunk - used) / f.k);
             if (n > 0) {
-                double* dst = ctx->stageDev.p + b * kStageChunk + used;
+                double* dst = ctx->stageDev.p + b * chunk + used;
                 const dim3 g(std::min(1024, (n * f.k + kBlock - 1) / kBlock));
                 hipLaunchKernelGGL((f.k == 3 ? k_to_rows<3> : f.k == 6 ? k_to_rows<6> : k_to_rows<9>), g, dim3(kBlock), 0,
                                    s, f.src + c, f.stride, n, dst);
@@ -1081,7 +1098,7 @@ void downloadRows(s4f_ctx* ctx, const std::vector<RowField>& fields, hipStream_t
         }
         if (used == 0) return false;
         HIP_CHECK(hipGetLastError());
-        HIP_CHECK(hipMemcpyAsync(ctx->stageHost + b * kStageChunk, ctx->stageDev.p + b * kStageChunk,
+        HIP_CHECK(hipMemcpyAsync(ctx->stageHost + b * chunk, ctx->stageDev.p + b * chunk,
                                  used * sizeof(double), hipMemcpyDeviceToHost, s));
         HIP_CHECK(hipEventRecord(ctx->stageEv[b], s));
         return true;
@@ -1092,7 +1109,7 @@ void downloadRows(s4f_ctx* ctx, const std::vector<RowField>& fields, hipStream_t
         HIP_CHECK(hipEventSynchronize(ctx->stageEv[b]));
         for (const Piece& q : pieces[b])
             parallelFor((int)q.count, 1 << 16, [&](int i0, int i1) {
-                std::memcpy(q.out + i0, ctx->stageHost + b * kStageChunk + q.at + i0, (size_t)(i1 - i0) * sizeof(double));
+                std::memcpy(q.out + i0, ctx->stageHost + b * chunk + q.at + i0, (size_t)(i1 - i0) * sizeof(double));
             });
     }
 }
@@ -2655,9 +2672,6 @@ s4f_status s4f_ctx_create(int device, s4f_ctx** out) {
         HIP_CHECK(hipStreamCreateWithFlags(&c->capture, hipStreamNonBlocking));
         HIP_CHECK(hipEventCreate(&c->ev0));
         HIP_CHECK(hipEventCreate(&c->ev1));
-        c->stageDev.alloc(2 * kStageChunk);
-        HIP_CHECK(hipHostMalloc((void**)&c->stageHost, 2 * kStageChunk * sizeof(double), hipHostMallocDefault));
-        for (hipEvent_t& e : c->stageEv) HIP_CHECK(hipEventCreateWithFlags(&e, hipEventDisableTiming));
         hipDeviceProp_t prop;
         HIP_CHECK(hipGetDeviceProperties(&prop, device));
         c->nCU = prop.multiProcessorCount;
