@@ -100,12 +100,23 @@ __device__ __forceinline__ bool mgSkip(const Ctl* c) { return c->outerDone || c-
 
 // Coarse-level vectors are rows of four (three components and a zero pad):
 // one 16-byte (FP32) or 32-byte (FP64) load per neighbour instead of three
-// component gathers; so is the fine level's residual r0, which the restriction
-// gathers.  The PCG's vectors stay component-major.
+// component gathers; the fine level's residual r0, which the restriction
+// gathers, is rows of three.  The PCG's vectors stay component-major.
 template <typename T> struct Row4Sel;
 template <> struct Row4Sel<float> { typedef float type __attribute__((ext_vector_type(4))); };
 template <> struct Row4Sel<double> { typedef double type __attribute__((ext_vector_type(4))); };
 template <typename T> using Row4 = typename Row4Sel<T>::type;
+
+// The fine level's residual is stored without the pad: it is as large as the
+// PCG's vectors, and written and read once per cell besides the gathers.
+// First weighted restriction with rows of four -> three: 45 -> 37 us (128^3 cells,
+// FP32), 23.0 -> 21.5 (566,475, FP64); V-cycle at 200^3 0.763 -> 0.725 ms
+// (component-major with one wavefront per slice: 0.732).
+template <typename T>
+struct Row3 {
+    T v[3];
+    __device__ __forceinline__ T operator[](int j) const { return v[j]; }
+};
 
 template <typename T>
 __device__ __forceinline__ Row4<T> row4(T a, T b, T c) {
@@ -123,7 +134,7 @@ __device__ __forceinline__ Row4<T> row4(T a, T b, T c) {
 // row's own cell with a zero coefficient) so a wave's gathers overlap.
 template <typename T, int W>
 __device__ __forceinline__ void mg0DownRowAll(const DevMesh& m, int P, int e0, int lane, int C, const T* __restrict__ b,
-                                              Row4<T>* __restrict__ r, T w) {
+                                              Row3<T>* __restrict__ r, T w) {
     const T* __restrict__ A = MatSel<T>::a(m);
     const T* __restrict__ invD = MatSel<T>::invDiag(m);
     int nb[W];
@@ -151,7 +162,7 @@ __device__ __forceinline__ void mg0DownRowAll(const DevMesh& m, int P, int e0, i
 #pragma unroll
         for (int j = 0; j < 3; ++j) y[j] -= av * (wi * b[(size_t)j * C + c]);
     }
-    stS(r + P, row4(bP[0] - y[0], bP[1] - y[1], bP[2] - y[2]));
+    r[P] = Row3<T>{{bP[0] - y[0], bP[1] - y[1], bP[2] - y[2]}};
 }
 
 // level-0 prolongation + post-smoothing of one row (all three components,
@@ -160,7 +171,7 @@ __device__ __forceinline__ void mg0DownRowAll(const DevMesh& m, int P, int e0, i
 template <typename T, int W>
 __device__ __forceinline__ void mg0UpRowAll(const DevMesh& m, const int* __restrict__ qCol, const T* __restrict__ q,
                                             int P, int e0, int lane, int C, const T* __restrict__ b,
-                                            const Row4<T>* __restrict__ r0, const int* __restrict__ agg,
+                                            const Row3<T>* __restrict__ r0, const int* __restrict__ agg,
                                             const Row4<T>* __restrict__ e, T* __restrict__ z, T w, T w1, T al,
                                             double* acc) {
     const T* __restrict__ invD = MatSel<T>::invDiag(m);
@@ -183,7 +194,8 @@ __device__ __forceinline__ void mg0UpRowAll(const DevMesh& m, const int* __restr
 #pragma unroll
         for (int j = 0; j < 3; ++j) s[j] += c * ek[j];
     }
-    const Row4<T> eP = e[IP], rP = r0[P];
+    const Row4<T> eP = e[IP];
+    const Row3<T> rP = r0[P];
 #pragma unroll
     for (int j = 0; j < 3; ++j) {
         const size_t i = (size_t)j * C + P;
@@ -198,7 +210,7 @@ __device__ __forceinline__ void mg0UpRowAll(const DevMesh& m, const int* __restr
 // x = w D^-1 b (not stored: k_mg0_up works from b and r), r = b - A x
 template <typename T>
 __global__ __launch_bounds__(kBlock) void k_mg0_down(const DevMesh m, const BlockMap bm, const T* __restrict__ b,
-                                                     Row4<T>* __restrict__ r, double omega,
+                                                     Row3<T>* __restrict__ r, double omega,
                                                      const Ctl* __restrict__ ctl) {
     const int lb = logicalBlock(bm.nBlocks);
     const Tile tl = bm.at(lb);
@@ -262,7 +274,7 @@ __global__ __launch_bounds__(kBlock) void k_mg0_down(const DevMesh m, const Bloc
         T rP[3];  // a converged component's residual is not read
 #pragma unroll
         for (int j = 0; j < 3; ++j) rP[j] = act[j] ? bP[j] - y[j] : (T)0;
-        r[P] = row4(rP[0], rP[1], rP[2]);
+        r[P] = Row3<T>{{rP[0], rP[1], rP[2]}};
     }
 }
 
@@ -276,7 +288,7 @@ __global__ __launch_bounds__(kBlock) void k_mg0_down(const DevMesh m, const Bloc
 // the PCG residual: z.b = rho of the preconditioned residual).
 template <typename T>
 __global__ __launch_bounds__(kBlock) void k_mg0_up(const DevMesh m, const BlockMap bm, const T* __restrict__ b,
-                                                   const Row4<T>* __restrict__ r0, const int* __restrict__ agg,
+                                                   const Row3<T>* __restrict__ r0, const int* __restrict__ agg,
                                                    const int* __restrict__ qCol, const T* __restrict__ q,
                                                    const Row4<T>* __restrict__ e, T* __restrict__ z, double omega,
                                                    double alpha, const Ctl* __restrict__ ctl,
@@ -322,7 +334,7 @@ __global__ __launch_bounds__(kBlock) void k_mg0_up(const DevMesh m, const BlockM
                 }
             }
         }
-        const Row4<T> rP = r0[P];
+        const Row3<T> rP = r0[P];
 #pragma unroll
         for (int j = 0; j < 3; ++j) {
             if (!act[j]) continue;
@@ -345,7 +357,7 @@ __global__ __launch_bounds__(kBlock) void k_mg0_up(const DevMesh m, const BlockM
 // unconditional and in bounds).  Partial z.b per block.
 template <typename T>
 __global__ __launch_bounds__(kBlock) void k_mg0_up_g(const DevMesh m, const BlockMap bm, const T* __restrict__ b,
-                                                     const Row4<T>* __restrict__ r0, const int* __restrict__ gStart,
+                                                     const Row3<T>* __restrict__ r0, const int* __restrict__ gStart,
                                                      const int* __restrict__ gWidth, const int* __restrict__ gCol,
                                                      const T* __restrict__ g, const Row4<T>* __restrict__ e,
                                                      T* __restrict__ z, double omega, double alpha,
@@ -385,7 +397,7 @@ __global__ __launch_bounds__(kBlock) void k_mg0_up_g(const DevMesh m, const Bloc
             }
         }
         const T wi = w * invD[P];
-        const Row4<T> rP = r0[P];
+        const Row3<T> rP = r0[P];
 #pragma unroll
         for (int j = 0; j < 3; ++j) {
             if (!act[j]) continue;
@@ -427,9 +439,9 @@ __device__ __forceinline__ bool mgLive(const MgLevel& L, int row, bool on, const
 // sum += sum over slots k = wave, wave + 4, ... of coef_k x[idx_k], kMgChunk
 // slots' loads in flight at a time, all unconditional (a slot past the width
 // or empty reads an in-bounds slot and row `own` with a zero coefficient)
-template <typename T>
+template <typename T, typename Row>
 __device__ __forceinline__ void slotSum(const int* __restrict__ idx, const T* __restrict__ coef, int width, int wave,
-                                        int lane, int own, const Row4<T>* __restrict__ x, T* sum) {
+                                        int lane, int own, const Row* __restrict__ x, T* sum) {
     constexpr int kWaves = kBlock / 64;
     for (int k0 = wave; k0 < width; k0 += kWaves * kMgChunk) {
         int J[kMgChunk];
@@ -445,7 +457,7 @@ __device__ __forceinline__ void slotSum(const int* __restrict__ idx, const T* __
 #pragma unroll
         for (int u = 0; u < kMgChunk; ++u) {
             const bool v = J[u] >= 0;
-            const Row4<T> xv = x[v ? J[u] : own];
+            const Row xv = x[v ? J[u] : own];
             const T cv = v ? c[u] : (T)0;
 #pragma unroll
             for (int j = 0; j < 3; ++j) sum[j] += cv * xv[j];
@@ -494,8 +506,8 @@ __device__ __forceinline__ T sumOf8(T v) {
 // from zero, formed once here instead of at every use).  Eight lanes per row:
 // a row's member list is read in one coalesced load, and levels of a few
 // thousand rows still fill the chip.
-template <typename T>
-__global__ __launch_bounds__(kBlock) void k_mg_restrict(const MgLevel Lc, const Row4<T>* __restrict__ r,
+template <typename T, typename Row>
+__global__ __launch_bounds__(kBlock) void k_mg_restrict(const MgLevel Lc, const Row* __restrict__ r,
                                                         Row4<T>* __restrict__ bc, Row4<T>* __restrict__ xc,
                                                         double omega, const Ctl* __restrict__ ctl) {
     constexpr int kRows = kBlock / 8;
@@ -522,7 +534,7 @@ __global__ __launch_bounds__(kBlock) void k_mg_restrict(const MgLevel Lc, const 
             }
 #pragma unroll
             for (int u = 0; u < 4; ++u) {
-                const Row4<T> v = r[mi[u]];
+                const Row v = r[mi[u]];
 #pragma unroll
                 for (int j = 0; j < 3; ++j) s[j] += wv[u] * v[j];
             }
@@ -541,7 +553,7 @@ __global__ __launch_bounds__(kBlock) void k_mg_restrict(const MgLevel Lc, const 
 // slot one coalesced load of members and weights; members in ascending
 // fine-row order), and xc = w D^-1 bc
 template <typename T>
-__global__ __launch_bounds__(kBlock) void k_mg_restrict_w(const MgLevel Lc, const Row4<T>* __restrict__ r0,
+__global__ __launch_bounds__(kBlock) void k_mg_restrict_w(const MgLevel Lc, const Row3<T>* __restrict__ r0,
                                                           Row4<T>* __restrict__ bc, Row4<T>* __restrict__ xc,
                                                           double omega, const Ctl* __restrict__ ctl) {
     __shared__ T sh[kBlock / 64 - 1][3][kSlice];
@@ -555,7 +567,7 @@ __global__ __launch_bounds__(kBlock) void k_mg_restrict_w(const MgLevel Lc, cons
         int inst;
         const bool live = mgLive(Lc, I, I < Lc.n, ctl, inst);
         T sum[3] = {(T)0, (T)0, (T)0};
-        if (live) slotSum<T>(Lc.rMem + e0, MgSel<T>::rW(Lc) + e0, width, wave, lane, 0, r0, sum);
+        if (live) slotSum(Lc.rMem + e0, MgSel<T>::rW(Lc) + e0, width, wave, lane, 0, r0, sum);
         sumWaves<T>(sh, wave, lane, sum);
         if (live && wave == 0) {
             const T wi = w * iDg[I];
@@ -590,7 +602,7 @@ __global__ __launch_bounds__(kBlock) void k_mg_down(const MgLevel L, const Row4<
             d = dg[P];
         }
         T sum[3] = {(T)0, (T)0, (T)0};
-        if (live && !pass) slotSum<T>(L.col + e0, MgSel<T>::a(L) + e0, width, wave, lane, P, x, sum);
+        if (live && !pass) slotSum(L.col + e0, MgSel<T>::a(L) + e0, width, wave, lane, P, x, sum);
         sumWaves<T>(sh, wave, lane, sum);
         if (last)
             r[P] = pass ? bP
@@ -629,7 +641,7 @@ __global__ __launch_bounds__(kBlock) void k_mg_up(const MgLevel L, const Row4<T>
             iD = iDg[P];
         }
         T sum[3] = {(T)0, (T)0, (T)0};
-        if (live && !pass) slotSum<T>(L.qCol + e0, MgSel<T>::q(L) + e0, width, wave, lane, 0, e, sum);
+        if (live && !pass) slotSum(L.qCol + e0, MgSel<T>::q(L) + e0, width, wave, lane, 0, e, sum);
         sumWaves<T>(sh, wave, lane, sum);
         if (last) {
             const T wi = w * iD;

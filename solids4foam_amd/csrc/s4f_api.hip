@@ -1826,11 +1826,12 @@ void buildAmg(s4f_mesh* M, bool smoothed) {
     A.buildSeconds = std::chrono::duration<double>(std::chrono::steady_clock::now() - t0).count();
 }
 
-// V-cycle work vectors, rows of four; level 0 holds only the residual
+// V-cycle work vectors, rows of four; level 0 holds only the residual, rows of three
 template <typename T>
 struct MgVec;
 template <>
 struct MgVec<double> {
+    static Row3<double>* r0(AmgDevLevel& L) { L.r64.alloc(3 * (size_t)L.n); return reinterpret_cast<Row3<double>*>(L.r64.p); }
     static Row4<double>* x(AmgDevLevel& L) { return v4(L.x64, L.n); }
     static Row4<double>* b(AmgDevLevel& L) { return v4(L.b64, L.n); }
     static Row4<double>* r(AmgDevLevel& L) { return v4(L.r64, L.n); }
@@ -1845,6 +1846,7 @@ struct MgVec<double> {
 };
 template <>
 struct MgVec<float> {
+    static Row3<float>* r0(AmgDevLevel& L) { L.r32.alloc(3 * (size_t)L.n); return reinterpret_cast<Row3<float>*>(L.r32.p); }
     static Row4<float>* x(AmgDevLevel& L) { return v4(L.x32, L.n); }
     static Row4<float>* b(AmgDevLevel& L) { return v4(L.b32, L.n); }
     static Row4<float>* r(AmgDevLevel& L) { return v4(L.r32, L.n); }
@@ -1883,11 +1885,11 @@ void launchMg0Up(std::vector<std::unique_ptr<AmgDevLevel>>& d, const DevMesh& dm
     const Row4<T>* e1 = d.size() > 1 ? (const Row4<T>*)MgVec<T>::xs(*d[1]) : nullptr;
     if (D0.gCol.p && e1)
         hipLaunchKernelGGL((k_mg0_up_g<T>), dim3(bm.nBlocks), dim3(kBlock), 0, s, dm, bm, (const T*)v.r,
-                           (const Row4<T>*)MgVec<T>::r(D0), (const int*)D0.gStart.p, (const int*)D0.gWidth.p,
+                           (const Row3<T>*)MgVec<T>::r0(D0), (const int*)D0.gStart.p, (const int*)D0.gWidth.p,
                            (const int*)D0.gCol.p, MgVec<T>::g(D0), e1, v.z, omega, alpha, (const Ctl*)ctl, part);
     else
         hipLaunchKernelGGL((k_mg0_up<T>), dim3(bm.nBlocks), dim3(kBlock), 0, s, dm, bm, (const T*)v.r,
-                           (const Row4<T>*)MgVec<T>::r(D0), (const int*)D0.agg.p, (const int*)D0.qCol.p, MgVec<T>::q(D0),
+                           (const Row3<T>*)MgVec<T>::r0(D0), (const int*)D0.agg.p, (const int*)D0.qCol.p, MgVec<T>::q(D0),
                            e1, v.z, omega, alpha, (const Ctl*)ctl, part);
 }
 
@@ -1904,7 +1906,7 @@ void launchVcycle(const MgRun& R, const DevMesh& dm, const BlockMap& bm, const P
     const int nl = (int)A.d.size();
     const double w = R.omega;
     AmgDevLevel& D0 = *A.d[0];
-    Row4<T>* r0 = MgVec<T>::r(D0);
+    Row3<T>* r0 = MgVec<T>::r0(D0);
     if (ch.merged) {
         hipLaunchKernelGGL((dm.uniW == 6 ? k_mg0_down_m<T, AGAIN, 6> : k_mg0_down_m<T, AGAIN, 4>), dim3(bm.nBlocks), dim3(kBlock), 0, s, dm, bm, (const T*)v.r, r0, w,
                            ch.at(in, ch.w), (const double*)part);
@@ -1921,13 +1923,16 @@ void launchVcycle(const MgRun& R, const DevMesh& dm, const BlockMap& bm, const P
             AmgDevLevel& Lf = *A.d[l - 1];
             Row4<T>* b = MgVec<T>::b(L);
             Row4<T>* x = MgVec<T>::x(L);
-            const Row4<T>* r = MgVec<T>::r(Lf);
+            const dim3 gr(gridRows(8 * (long long)L.n));
             if (l == 1 && L.rMem.p)  // smoothed prolongation: weighted lists in sliced ELL
-                hipLaunchKernelGGL((k_mg_restrict_w<T>), dim3(gridSlices(L.nSlices)), dim3(kBlock), 0, s, L.view(), r, b,
-                                   x, w, (const Ctl*)ctl);
+                hipLaunchKernelGGL((k_mg_restrict_w<T>), dim3(gridSlices(L.nSlices)), dim3(kBlock), 0, s, L.view(),
+                                   (const Row3<T>*)r0, b, x, w, (const Ctl*)ctl);
+            else if (l == 1)
+                hipLaunchKernelGGL((k_mg_restrict<T, Row3<T>>), gr, dim3(kBlock), 0, s, L.view(), (const Row3<T>*)r0, b, x,
+                                   w, (const Ctl*)ctl);
             else
-                hipLaunchKernelGGL((k_mg_restrict<T>), dim3(gridRows(8 * (long long)L.n)), dim3(kBlock), 0, s, L.view(), r,
-                                   b, x, w, (const Ctl*)ctl);
+                hipLaunchKernelGGL((k_mg_restrict<T, Row4<T>>), gr, dim3(kBlock), 0, s, L.view(),
+                                   (const Row4<T>*)MgVec<T>::r(Lf), b, x, w, (const Ctl*)ctl);
             if (l < nl - 1)
                 hipLaunchKernelGGL((k_mg_down<T>), dim3(gridSlices(L.nSlices)), dim3(kBlock), 0, s, L.view(),
                                    (const Row4<T>*)b, (const Row4<T>*)x, MgVec<T>::r(L), (const Ctl*)ctl);
@@ -3503,7 +3508,7 @@ double replayT(s4f_mesh* M, int kernel, int launches) {
             case S4F_KERNEL_MG0_DOWN: {
                 AmgDevLevel& D0 = *AK.d[0];
                 hipLaunchKernelGGL((k_mg0_down<T>), dim3(bm.nBlocks), dim3(kBlock), 0, s, dm, bm, (const T*)v.r,
-                                   MgVec<T>::r(D0), AK.omega, (const Ctl*)rc.p);
+                                   MgVec<T>::r0(D0), AK.omega, (const Ctl*)rc.p);
                 break;
             }
             case S4F_KERNEL_MG0_UP:
@@ -3522,7 +3527,7 @@ double replayT(s4f_mesh* M, int kernel, int launches) {
             AmgDevLevel& L = *AK.d[l];
             const size_t n4 = 4 * (size_t)L.n * sizeof(T);
             if (l == 0) {  // the fine level keeps only the residual
-                HIP_CHECK(hipMemsetAsync(MgVec<T>::r(L), 0, n4, s));
+                HIP_CHECK(hipMemsetAsync(MgVec<T>::r0(L), 0, 3 * (size_t)L.n * sizeof(T), s));
                 continue;
             }
             HIP_CHECK(hipMemsetAsync(MgVec<T>::x(L), 0, n4, s));

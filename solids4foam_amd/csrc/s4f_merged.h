@@ -259,7 +259,7 @@ __global__ __launch_bounds__(kBlock) void k_spmvp_m(const DevMesh m, const Block
 // k_mg0_down: r = b - A x with x = w D^-1 b; no load depends on the scalars
 template <typename T, bool AGAIN, int W>
 __global__ __launch_bounds__(kBlock) void k_mg0_down_m(const DevMesh m, const BlockMap bm, const T* __restrict__ b,
-                                                       Row4<T>* __restrict__ r, double omega, const Stage st,
+                                                       Row3<T>* __restrict__ r, double omega, const Stage st,
                                                        const double* __restrict__ part) {
     constexpr int kPt = AGAIN ? kPtAgain : kPtInner;
     const int lb = logicalBlock(bm.nBlocks);
@@ -314,7 +314,7 @@ __global__ __launch_bounds__(kBlock) void k_mg0_down_m(const DevMesh m, const Bl
             for (int k = 0; k < W; ++k) xn[k] = w * iDN[k] * bN[k][j];
             y[j] = rowProduct<T, W>(all, dP, w * iDP * bP[j], row.a, xn);
         }
-        r[P] = row4<T>(bP[0] - y[0], bP[1] - y[1], bP[2] - y[2]);  // a converged component's is not read
+        r[P] = Row3<T>{{(T)(bP[0] - y[0]), (T)(bP[1] - y[1]), (T)(bP[2] - y[2])}};  // a converged component's is not read
     }
 }
 // The residual of meshes of one slot count, in merged launch sequences
