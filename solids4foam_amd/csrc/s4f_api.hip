@@ -3479,6 +3479,12 @@ double replayT(s4f_mesh* M, int kernel, int launches) {
     auto launch = [&]() {
         switch (kernel) {
             case S4F_KERNEL_RESIDUAL:
+                if (uniformSlots(dm)) {  // as launchOuter without merged points
+                    hipLaunchKernelGGL((residualUniform<T, false>(dm)), dim3(bm.nBlocks), dim3(kBlock), 0, s, dm, bm,
+                                       (const double*)st.D0.p, (const double*)st.D1.p, (const double*)st.G.p,
+                                       (const double*)st.sigb.p, v.r, chain.at(rc.p, rc.p + 1), st.part.p);
+                    break;
+                }
                 hipLaunchKernelGGL((k_residual<T>), dim3(bm.nBlocks), dim3(kBlock), 0, s, dm, bm,
                                    (const double*)st.D0.p, (const double*)st.D1.p, (const double*)st.G.p,
                                    (const double*)st.sigb.p, v.r, (const Ctl*)rc.p, st.part.p);
