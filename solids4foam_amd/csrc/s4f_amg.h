@@ -632,16 +632,17 @@ __global__ __launch_bounds__(kBlock) void k_mg_up(const MgLevel L, const Row4<T>
         const bool live = mgLive(L, P, P < L.n, ctl, inst);
         const bool pass = live && L.pass[inst];  // already coarsest: the coarser solution unchanged
         const bool last = live && wave == 0;
+        const int IP = live ? L.agg[P] : 0;
         Row4<T> xv = {}, rv = {}, eP = {};
         T iD = (T)0;
         if (last) {
-            eP = e[L.agg[P]];
+            eP = e[IP];
             xv = x[P];
             rv = r[P];
             iD = iDg[P];
         }
         T sum[3] = {(T)0, (T)0, (T)0};
-        if (live && !pass) slotSum(L.qCol + e0, MgSel<T>::q(L) + e0, width, wave, lane, 0, e, sum);
+        if (live && !pass) slotSum(L.qCol + e0, MgSel<T>::q(L) + e0, width, wave, lane, IP, e, sum);
         sumWaves<T>(sh, wave, lane, sum);
         if (last) {
             const T wi = w * iD;
