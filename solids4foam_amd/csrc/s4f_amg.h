@@ -437,8 +437,10 @@ __device__ __forceinline__ bool mgLive(const MgLevel& L, int row, bool on, const
 }
 
 // sum += sum over slots k = wave, wave + 4, ... of coef_k x[idx_k], kMgChunk
-// slots' loads in flight at a time, all unconditional (a slot past the width
-// or empty reads an in-bounds slot and row `own` with a zero coefficient)
+// slots' loads in flight at a time, all unconditional with a zero coefficient
+// where there is nothing to add: a slot past the width reads the group's first
+// one again, an empty slot row `own`.  Both are rows of the row's own instance,
+// since zero times another instance's infinity or NaN would be NaN.
 template <typename T, typename Row>
 __device__ __forceinline__ void slotSum(const int* __restrict__ idx, const T* __restrict__ coef, int width, int wave,
                                         int lane, int own, const Row* __restrict__ x, T* sum) {
@@ -451,8 +453,8 @@ __device__ __forceinline__ void slotSum(const int* __restrict__ idx, const T* __
             const int k = k0 + kWaves * u;
             const int o = (k < width ? k : k0) * kSlice;
             J[u] = at32(idx + o, lane * 4u);
-            c[u] = at32(coef + o, lane * (unsigned)sizeof(T));
-            if (k >= width) J[u] = -1;
+            const T ce = at32(coef + o, lane * (unsigned)sizeof(T));
+            c[u] = k < width ? ce : (T)0;
         }
 #pragma unroll
         for (int u = 0; u < kMgChunk; ++u) {
@@ -551,7 +553,8 @@ __global__ __launch_bounds__(kBlock) void k_mg_restrict(const MgLevel Lc, const 
 // restriction into the first coarse level of a smoothed hierarchy: bc = P^T r0
 // with the weighted member lists in the coarse level's sliced-ELL slots (each
 // slot one coalesced load of members and weights; members in ascending
-// fine-row order), and xc = w D^-1 bc
+// fine-row order; a row of fewer repeats its first with a zero weight), and
+// xc = w D^-1 bc
 template <typename T>
 __global__ __launch_bounds__(kBlock) void k_mg_restrict_w(const MgLevel Lc, const Row3<T>* __restrict__ r0,
                                                           Row4<T>* __restrict__ bc, Row4<T>* __restrict__ xc,

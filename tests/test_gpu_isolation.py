@@ -97,3 +97,10 @@ def test_server_multigrid(ctx, precision):
     assert got[ids[0]]["status"] == _abi.S4F_ERR_DIVERGED
     for i, (rid, a) in enumerate(zip(ids[1:], alone)):
         assert _equal(got[rid], a), i
+
+
+@pytest.mark.parametrize("precision", [0, 1])
+def test_batch_smoothed_multigrid(ctx, precision):
+    # weighted restriction of the first level
+    from solids4foam_amd import PRECOND_GAMG_SMOOTHED
+    _check_batch(ctx, PRECOND_GAMG_SMOOTHED, precision)
