@@ -437,13 +437,16 @@ __device__ __forceinline__ bool mgLive(const MgLevel& L, int row, bool on, const
 }
 
 // sum += sum over slots k = wave, wave + 4, ... of coef_k x[idx_k], kMgChunk
-// slots' loads in flight at a time, all unconditional with a zero coefficient
-// where there is nothing to add: a slot past the width reads the group's first
-// one again, an empty slot row `own`.  Both are rows of the row's own instance,
-// since zero times another instance's infinity or NaN would be NaN.
+// slots' loads in flight at a time, all unconditional.  A slot past the width
+// reads the group's first one again, and where there is nothing to add row 0 is
+// read and dropped: that row belongs to the launch's first instance, so its
+// value must not enter even with a zero coefficient (zero times infinity or NaN
+// is NaN).  V-cycle with a row of the instance's own gathered in its place ->
+// row 0 dropped: 194 -> 191 us (128^3 cells, FP32, smoothed), 53.8 -> 53.0
+// (64^3), 120.9 -> 117.7 (83^3, FP64).
 template <typename T, typename Row>
 __device__ __forceinline__ void slotSum(const int* __restrict__ idx, const T* __restrict__ coef, int width, int wave,
-                                        int lane, int own, const Row* __restrict__ x, T* sum) {
+                                        int lane, const Row* __restrict__ x, T* sum) {
     constexpr int kWaves = kBlock / 64;
     for (int k0 = wave; k0 < width; k0 += kWaves * kMgChunk) {
         int J[kMgChunk];
@@ -453,16 +456,14 @@ __device__ __forceinline__ void slotSum(const int* __restrict__ idx, const T* __
             const int k = k0 + kWaves * u;
             const int o = (k < width ? k : k0) * kSlice;
             J[u] = at32(idx + o, lane * 4u);
-            const T ce = at32(coef + o, lane * (unsigned)sizeof(T));
-            c[u] = k < width ? ce : (T)0;
+            c[u] = at32(coef + o, lane * (unsigned)sizeof(T));
         }
 #pragma unroll
         for (int u = 0; u < kMgChunk; ++u) {
-            const bool v = J[u] >= 0;
-            const Row xv = x[v ? J[u] : own];
-            const T cv = v ? c[u] : (T)0;
+            const bool v = k0 + kWaves * u < width && J[u] >= 0;
+            const Row xv = x[v ? J[u] : 0];
 #pragma unroll
-            for (int j = 0; j < 3; ++j) sum[j] += cv * xv[j];
+            for (int j = 0; j < 3; ++j) sum[j] += c[u] * (v ? xv[j] : (T)0);
         }
     }
 }
@@ -553,8 +554,7 @@ __global__ __launch_bounds__(kBlock) void k_mg_restrict(const MgLevel Lc, const 
 // restriction into the first coarse level of a smoothed hierarchy: bc = P^T r0
 // with the weighted member lists in the coarse level's sliced-ELL slots (each
 // slot one coalesced load of members and weights; members in ascending
-// fine-row order; a row of fewer repeats its first with a zero weight), and
-// xc = w D^-1 bc
+// fine-row order), and xc = w D^-1 bc
 template <typename T>
 __global__ __launch_bounds__(kBlock) void k_mg_restrict_w(const MgLevel Lc, const Row3<T>* __restrict__ r0,
                                                           Row4<T>* __restrict__ bc, Row4<T>* __restrict__ xc,
@@ -570,7 +570,7 @@ __global__ __launch_bounds__(kBlock) void k_mg_restrict_w(const MgLevel Lc, cons
         int inst;
         const bool live = mgLive(Lc, I, I < Lc.n, ctl, inst);
         T sum[3] = {(T)0, (T)0, (T)0};
-        if (live) slotSum(Lc.rMem + e0, MgSel<T>::rW(Lc) + e0, width, wave, lane, 0, r0, sum);
+        if (live) slotSum(Lc.rMem + e0, MgSel<T>::rW(Lc) + e0, width, wave, lane, r0, sum);
         sumWaves<T>(sh, wave, lane, sum);
         if (live && wave == 0) {
             const T wi = w * iDg[I];
@@ -605,7 +605,7 @@ __global__ __launch_bounds__(kBlock) void k_mg_down(const MgLevel L, const Row4<
             d = dg[P];
         }
         T sum[3] = {(T)0, (T)0, (T)0};
-        if (live && !pass) slotSum(L.col + e0, MgSel<T>::a(L) + e0, width, wave, lane, P, x, sum);
+        if (live && !pass) slotSum(L.col + e0, MgSel<T>::a(L) + e0, width, wave, lane, x, sum);
         sumWaves<T>(sh, wave, lane, sum);
         if (last)
             r[P] = pass ? bP
@@ -635,17 +635,16 @@ __global__ __launch_bounds__(kBlock) void k_mg_up(const MgLevel L, const Row4<T>
         const bool live = mgLive(L, P, P < L.n, ctl, inst);
         const bool pass = live && L.pass[inst];  // already coarsest: the coarser solution unchanged
         const bool last = live && wave == 0;
-        const int IP = live ? L.agg[P] : 0;
         Row4<T> xv = {}, rv = {}, eP = {};
         T iD = (T)0;
         if (last) {
-            eP = e[IP];
+            eP = e[L.agg[P]];
             xv = x[P];
             rv = r[P];
             iD = iDg[P];
         }
         T sum[3] = {(T)0, (T)0, (T)0};
-        if (live && !pass) slotSum(L.qCol + e0, MgSel<T>::q(L) + e0, width, wave, lane, IP, e, sum);
+        if (live && !pass) slotSum(L.qCol + e0, MgSel<T>::q(L) + e0, width, wave, lane, e, sum);
         sumWaves<T>(sh, wave, lane, sum);
         if (last) {
             const T wi = w * iD;
