@@ -2179,14 +2179,80 @@ void launchPass(bool mg, const MgRun& R, const DevMesh& dm, const BlockMap& bm, 
 
 // PCG iterations per pass.  A pass launches the outer step's kernels also for
 // an instance still in its PCG (they exit at once), and PCG iterations also
-// for one that has just finished; with `used` iterations per outer one the
-// empty launches are fewest near sqrt(ratio used), ratio the outer step's
-// launches over an iteration's times two.  One V-cycle iteration has more
-// launches than the outer step, a diagonal one has two.
-int innerPerPass(bool mg, int used) {
-    const double k = std::sqrt((mg ? 0.5 : 2.0) * used);
-    return k >= 12.0 ? 16 : k >= 6.0 ? 8 : k >= 3.0 ? 4 : k >= 1.5 ? 2 : 1;
-}
+// for one that has just finished.  The count that makes the fewest empty
+// launches follows from how many iterations the live instances take per outer
+// one, which varies little from one to the next: an instance of u needs
+// ceil(u / k) passes, each of k iterations and the outer step's launches (about
+// half of an iteration's with a V-cycle, twice those of a diagonal one).
+// One iteration a pass for up to four per outer one -> this rule, us per outer
+// iteration: 128^3 cells FP32 (3.5 per outer one) 1,610 -> 1,551, 64^3 FP32
+// (2.6) 312 -> 293; 64 served requests of up to 128^3 cells 54.3 -> 44.1 s.
+class PassRule {
+  public:
+    explicit PassRule(size_t n) : seen_(n) {}
+    void reset(int i) { seen_[i] = Seen(); }
+    // what the control block of instance i shows at a look
+    void look(int i, const Ctl& c) {
+        Seen& s = seen_[i];
+        if (c.iCorr > s.iCorr) {
+            const double u = (double)(c.pcgTotal - s.pcg) / (c.iCorr - s.iCorr);
+            s.mean = s.iCorr == 0 ? u : 0.5 * (s.mean + u);
+            s.iCorr = c.iCorr;
+            s.pcg = c.pcgTotal;
+        } else {  // the first outer iteration, or one longer than a look
+            s.mean = std::max({s.mean, (double)c.nIter[0], (double)c.nIter[1], (double)c.nIter[2]});
+        }
+    }
+    int choose(bool mg, const std::vector<int>& live) const {
+        const double outer = mg ? 0.5 : 2.0;
+        int best = 1;
+        double least = HUGE_VAL;
+        for (int k : {1, 2, 3, 4, 5, 6, 8, 12, 16}) {
+            double passes = 0.0;
+            for (int i : live) {
+                const double u = std::max(1.0, seen_[i].mean), n = std::floor(u);
+                // a mean between two counts: so many of each; large counts vary by more than k
+                passes += n > 8.0 ? u / k + 0.5
+                                  : (1.0 - (u - n)) * std::ceil(n / k) + (u - n) * std::ceil((n + 1.0) / k);
+            }
+            const double cost = (outer + k) * passes;
+            if (cost < least) {
+                least = cost;
+                best = k;
+            }
+        }
+        return best;
+    }
+
+  private:
+    struct Seen {
+        int iCorr = 0;
+        long long pcg = 0;
+        double mean = 0.0;
+    };
+    std::vector<Seen> seen_;
+};
+
+// Passes between two looks at the control blocks: at most eight, and no more
+// than about kLookSeconds at the pace of the last ones.  What is queued when an
+// instance finishes runs to its end, empty: eight passes of five iterations at
+// 200^3 cells took 4 ms of a solve of 1.1 s.
+constexpr int kLookPasses = 8;
+constexpr double kLookSeconds = 2e-3;
+class LookPace {
+  public:
+    // a look, `passes` passes after the previous one
+    void seen(int passes) {
+        const auto now = std::chrono::steady_clock::now();
+        perPass_ = std::chrono::duration<double>(now - last_).count() / std::max(1, passes);
+        last_ = now;
+    }
+    int passes() const { return std::max(1, (int)std::min<double>(kLookPasses, kLookSeconds / perPass_)); }
+
+  private:
+    std::chrono::steady_clock::time_point last_ = std::chrono::steady_clock::now();
+    double perPass_ = kLookSeconds;
+};
 
 // An instantiated HIP graph of a captured launch sequence.
 struct GraphExec {
@@ -2390,6 +2456,7 @@ void solveT(s4f_mesh* M, const s4f_solve_opts& o, std::vector<InstanceIO>& io, F
     bool graphs = o.eagerLaunch == 0;
     std::map<int, GraphExec> graph;
     int inner = mg ? 1 : 4;
+    PassRule rule(nInst);
     long long passes = 0;
     auto pass = [&]() {
         auto launch = [&](hipStream_t q) {
@@ -2414,6 +2481,7 @@ void solveT(s4f_mesh* M, const s4f_solve_opts& o, std::vector<InstanceIO>& io, F
     struct Flight {  // a burst of passes and the control blocks after it
         hipEvent_t ev = nullptr;
         Ctl* h = nullptr;
+        int passes = 0;
         ~Flight() { if (ev) (void)hipEventDestroy(ev); }
     } flight[2];
     for (int k = 0; k < 2; ++k) {
@@ -2421,9 +2489,10 @@ void solveT(s4f_mesh* M, const s4f_solve_opts& o, std::vector<InstanceIO>& io, F
         HIP_CHECK(hipEventCreateWithFlags(&flight[k].ev, hipEventDisableTiming));
     }
     // bursts grow with the passes already made: a short solve wastes little at its end
+    LookPace pace;
     auto burst = [&](Flight& f) {
-        const int n = (int)std::min<long long>(8, 1 + passes / 16);
-        for (int k = 0; k < n; ++k) pass();
+        f.passes = (int)std::min<long long>(pace.passes(), 1 + passes / 16);
+        for (int k = 0; k < f.passes; ++k) pass();
         HIP_CHECK(hipMemcpyAsync(f.h, st.ctl.p, nInst * sizeof(Ctl), hipMemcpyDeviceToHost, s));
         HIP_CHECK(hipEventRecord(f.ev, s));
     };
@@ -2434,33 +2503,33 @@ void solveT(s4f_mesh* M, const s4f_solve_opts& o, std::vector<InstanceIO>& io, F
     for (int cur = 0;; cur ^= 1) {
         burst(flight[cur ^ 1]);
         HIP_CHECK(hipEventSynchronize(flight[cur].ev));
+        pace.seen(flight[cur].passes);
         const Ctl* hc = flight[cur].h;
-        int nLive = 0, used = 1;
+        std::vector<int> live;
         bool stalled = false;
         for (int i = 0; i < nInst; ++i) {
             if (hc[i].outerDone) continue;
-            ++nLive;
+            live.push_back(i);
             stalled |= hc[i].stalled != 0;
-            used = std::max({used, hc[i].nIter[0], hc[i].nIter[1], hc[i].nIter[2]});
+            rule.look(i, hc[i]);
         }
-        if (nLive == 0) break;
+        if (live.empty()) break;
         if (o.progressSeconds > 0) {  // the per-iteration log, rate-limited
             const double now = std::chrono::duration<double>(std::chrono::steady_clock::now() - tStart).count();
             if (now - tShown >= o.progressSeconds) {
                 tShown = now;
                 int iMax = 0;
                 double rMax = 0.0;
-                for (int i = 0; i < nInst; ++i) {
-                    if (hc[i].outerDone) continue;
+                for (int i : live) {
                     iMax = std::max(iMax, hc[i].iCorr);
                     rMax = std::max(rMax, hc[i].initResMag);
                 }
                 fprintf(stderr, "[s4f] %.0f s: outer iteration %d, %d of %d instances iterating, |initRes| %.3e, "
-                        "residualvf %.3e\n", now, iMax, nLive, nInst, rMax, hc[0].rvf);
+                        "residualvf %.3e\n", now, iMax, (int)live.size(), nInst, rMax, hc[0].rvf);
                 fflush(stderr);
             }
         }
-        inner = innerPerPass(mg, used);
+        inner = rule.choose(mg, live);
         if (stalled) {
             // every instance finishes its PCG and waits before its gradient step
             hipLaunchKernelGGL(k_ctl_hold, dim3(1), dim3(kBlock), 0, s, st.ctl.p, nInst, 1);
@@ -2484,13 +2553,8 @@ void solveT(s4f_mesh* M, const s4f_solve_opts& o, std::vector<InstanceIO>& io, F
         if (nInst > 1) {
             // finished instances leave the launch once they hold a quarter of its tiles
             // (their workgroups exit at once; a new map costs a capture)
-            std::vector<int> live;
             long long tiles = 0;
-            for (int i = 0; i < nInst; ++i)
-                if (!hc[i].outerDone) {
-                    live.push_back(i);
-                    tiles += M->tNBlk[i];
-                }
+            for (int i : live) tiles += M->tNBlk[i];
             if (4 * tiles <= 3 * liveTiles) {
                 // pending partials are laid out by the present map: resolve them, then
                 // wait: queued kernels still read the current tile arrays
@@ -3881,6 +3945,7 @@ struct s4f_server {
     // passes replayed from HIP graphs (per PCG iterations in a pass) while the
     // packed map they were captured on stands (mapGen counts rebuilds)
     std::map<int, GraphExec> graph;
+    PassRule rule{0};
     unsigned mapGen = 0, ranGen = ~0u;
     Ctl* hctl = nullptr;
     // bookkeeping (server thread only)
@@ -3970,6 +4035,7 @@ void serverAllocate(s4f_server* S) {
     S->iBlk0.alloc(S->maxSlots); S->iNBlk.alloc(S->maxSlots); S->iNCell.alloc(S->maxSlots);
     S->iB0.alloc(S->maxSlots); S->iNB.alloc(S->maxSlots);
     S->slotReq.assign(S->maxSlots, -1);
+    S->rule = PassRule(S->maxSlots);
 }
 
 DevMesh serverDm(const s4f_server* S) {
@@ -4203,6 +4269,7 @@ void serverAdmit(s4f_server* S) {
         c.sigma0 = warm ? 0 : 1;
         HIP_CHECK(hipStreamSynchronize(S->ctx->stream));
         hcopy(S->ctx->stream, S->ctl.p + slot, &c, 1);
+        S->rule.reset(slot);
         const int n = (int)pl.nCells;
         hipLaunchKernelGGL(k_slot_init, dim3(std::max(1, std::min(2048, (n + kBlock - 1) / kBlock))), dim3(kBlock), 0,
                            S->ctx->stream, S->D0.p, S->D1.p, S->Dold.p, S->G.p, S->g.p, (int)S->Ccap, (int)S->Bcap,
@@ -4501,10 +4568,13 @@ void serverStep(s4f_server* S) {
     HIP_CHECK(hipGetLastError());
     HIP_CHECK(hipMemcpyAsync(S->hctl, S->ctl.p, S->maxSlots * sizeof(Ctl), hipMemcpyDeviceToHost, s));
     HIP_CHECK(hipStreamSynchronize(s));
-    int used = 1;
+    std::vector<int> live;
     for (int sl : slots)
-        if (!S->hctl[sl].outerDone) used = std::max({used, S->hctl[sl].nIter[0], S->hctl[sl].nIter[1], S->hctl[sl].nIter[2]});
-    S->inner = innerPerPass(S->mgOn, used);
+        if (!S->hctl[sl].outerDone) {
+            live.push_back(sl);
+            S->rule.look(sl, S->hctl[sl]);
+        }
+    if (!live.empty()) S->inner = S->rule.choose(S->mgOn, live);
     // retire
     bool changed = false;
     for (int sl : slots) {
