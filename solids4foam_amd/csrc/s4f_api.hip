@@ -2241,7 +2241,8 @@ constexpr int kLookPasses = 8;
 constexpr double kLookSeconds = 2e-3;
 class LookPace {
   public:
-    // a look, `passes` passes after the previous one
+    void start() { last_ = std::chrono::steady_clock::now(); }
+    // a look, `passes` passes after the previous one (or the start)
     void seen(int passes) {
         const auto now = std::chrono::steady_clock::now();
         perPass_ = std::chrono::duration<double>(now - last_).count() / std::max(1, passes);
@@ -3946,6 +3947,7 @@ struct s4f_server {
     // packed map they were captured on stands (mapGen counts rebuilds)
     std::map<int, GraphExec> graph;
     PassRule rule{0};
+    LookPace pace;
     unsigned mapGen = 0, ranGen = ~0u;
     Ctl* hctl = nullptr;
     // bookkeeping (server thread only)
@@ -4519,10 +4521,6 @@ void serverRebuildMap(s4f_server* S) {
     }
 }
 
-// passes of the launch sequence over every in-flight solve between two looks
-// at their control blocks (a finished solve waits this long at most)
-constexpr int kServerPasses = 8;
-
 // a few passes over every in-flight solve, then retire the converged
 template <typename T>
 void serverStep(s4f_server* S) {
@@ -4543,7 +4541,10 @@ void serverStep(s4f_server* S) {
         launchPass<T>(S->mgOn, run, dm, bm, serverMaxNB(S), serverGradBufs(S), v, (const double*)S->Dold.p, chain,
                       S->part.p, S->inner, q);
     };
-    for (int k = 0; k < kServerPasses; ++k) {
+    // a finished solve, or an arriving one, waits this long at most
+    const int passes = S->pace.passes();
+    S->pace.start();
+    for (int k = 0; k < passes; ++k) {
         // the first pass on a new map runs eagerly (it allocates the
         // multigrid vectors of the packing); later ones are replayed
         const bool eager = S->opts.eagerLaunch != 0 || S->ranGen != S->mapGen;
@@ -4568,6 +4569,7 @@ void serverStep(s4f_server* S) {
     HIP_CHECK(hipGetLastError());
     HIP_CHECK(hipMemcpyAsync(S->hctl, S->ctl.p, S->maxSlots * sizeof(Ctl), hipMemcpyDeviceToHost, s));
     HIP_CHECK(hipStreamSynchronize(s));
+    S->pace.seen(passes);
     std::vector<int> live;
     for (int sl : slots)
         if (!S->hctl[sl].outerDone) {
