@@ -2447,7 +2447,13 @@ void solveT(s4f_mesh* M, const s4f_solve_opts& o, std::vector<InstanceIO>& io, F
         bm.finInst = M->aFin.p;
         bm.nBlocks = (int)tile.size();
         mgRun.nFin = (int)live.size();
+        const bool wasMerged = chain.merged;
         chain = Chain(st.ctl.p, nInst, canMerge(dm, maxTiles(live)), st.hist.p);
+        // the coarse levels keep the rows of the instances that left, and look
+        // at their control blocks in every array of the chain
+        for (int k = 1; chain.merged && !wasMerged && k < kChain; ++k)
+            HIP_CHECK(hipMemcpyAsync(st.ctl.p + (size_t)k * nInst, st.ctl.p, nInst * sizeof(Ctl),
+                                     hipMemcpyDeviceToDevice, s));
     };
     // A pass advances every instance from where it stands, so the host launches
     // passes without knowing where that is and looks at the control blocks of

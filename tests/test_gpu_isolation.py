@@ -104,3 +104,25 @@ def test_batch_smoothed_multigrid(ctx, precision):
     # weighted restriction of the first level
     from solids4foam_amd import PRECOND_GAMG_SMOOTHED
     _check_batch(ctx, PRECOND_GAMG_SMOOTHED, precision)
+
+
+@pytest.mark.parametrize("precond", [0, 2, 3])
+def test_batch_turns_merged(ctx, precond):
+    # an instance over the line of merged launches leaves first (no load): the
+    # others go on in merged launches, on a hierarchy that still holds its rows
+    from solids4foam_amd.batch import Batch
+    print(f"[isolation] batch turns merged precond={precond}", flush=True)
+    opts = dict(CAPPED, precision=0, preconditioner=precond, pcgMaxIter=40, nCorrectors=40)
+    large, _ = _box(ctx, (64, 41, 25), 1, traction=(0.0, 0.0, 0.0))
+    large.set_tiles(65536, 1)  # a tile per slice: 1,025
+    others = [_box(ctx, n, 2 + i)[0] for i, n in enumerate(SIZES)]
+    alone = [m.solve(**opts) for m in others]
+    b = Batch(ctx)
+    for m in others[:1] + [large] + others[1:]:
+        b.add(m)
+    got = b.solve(**opts)
+    assert got[1]["converged"] and got[1]["nOuter"] < 5
+    del got[1]
+    for i, (r, a) in enumerate(zip(got, alone)):
+        assert r["nOuter"] == 40 and _equal(r, a), i
+    b.close()
