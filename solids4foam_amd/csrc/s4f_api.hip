@@ -14,6 +14,7 @@
 #include <map>
 #include <mutex>
 #include <thread>
+#include <tuple>
 #include <type_traits>
 #include <unordered_map>
 #include <cmath>
@@ -2255,6 +2256,35 @@ class LookPace {
     double perPass_ = kLookSeconds;
 };
 
+// Ends a solve whose launches no longer advance an instance: every pass takes
+// an iterating instance at least one step of its PCG or outer loop on, both of
+// which the device counts up to their limits.
+class ProgressWatch {
+  public:
+    explicit ProgressWatch(size_t n) : last_(n) {}
+    // a look at instance i, at least one pass after the previous one
+    void look(int i, const Ctl& c) {
+        const At now{c.iCorr, c.pIt, c.pending, c.innerDone, c.innerTotal};
+        if (now == last_[i].at) {
+            if (++last_[i].looks >= kLooks)
+                throw HipError("the solve does not advance (instance " + std::to_string(i) + ", outer iteration " +
+                               std::to_string(c.iCorr) + ", step " + std::to_string(c.pending) + ")");
+        } else {
+            last_[i].at = now;
+            last_[i].looks = 0;
+        }
+    }
+
+  private:
+    static constexpr int kLooks = 8;
+    typedef std::tuple<int, int, int, int, long long> At;
+    struct Last {
+        At at{-1, 0, 0, 0, 0};
+        int looks = 0;
+    };
+    std::vector<Last> last_;
+};
+
 // An instantiated HIP graph of a captured launch sequence.
 struct GraphExec {
     hipGraphExec_t e = nullptr;
@@ -2464,6 +2494,7 @@ void solveT(s4f_mesh* M, const s4f_solve_opts& o, std::vector<InstanceIO>& io, F
     std::map<int, GraphExec> graph;
     int inner = mg ? 1 : 4;
     PassRule rule(nInst);
+    ProgressWatch watch(nInst);
     long long passes = 0;
     auto pass = [&]() {
         auto launch = [&](hipStream_t q) {
@@ -2495,6 +2526,10 @@ void solveT(s4f_mesh* M, const s4f_solve_opts& o, std::vector<InstanceIO>& io, F
         flight[k].h = hctl + (size_t)k * nInst;
         HIP_CHECK(hipEventCreateWithFlags(&flight[k].ev, hipEventDisableTiming));
     }
+    struct Quiet {  // what is queued reads the graphs and writes the host copies, also when an error ends the loop
+        hipStream_t s;
+        ~Quiet() { (void)hipStreamSynchronize(s); }
+    } quiet{s};
     // bursts grow with the passes already made: a short solve wastes little at its end
     LookPace pace;
     auto burst = [&](Flight& f) {
@@ -2519,6 +2554,7 @@ void solveT(s4f_mesh* M, const s4f_solve_opts& o, std::vector<InstanceIO>& io, F
             live.push_back(i);
             stalled |= hc[i].stalled != 0;
             rule.look(i, hc[i]);
+            if (!hc[i].hold) watch.look(i, hc[i]);
         }
         if (live.empty()) break;
         if (o.progressSeconds > 0) {  // the per-iteration log, rate-limited
@@ -2549,7 +2585,9 @@ void solveT(s4f_mesh* M, const s4f_solve_opts& o, std::vector<InstanceIO>& io, F
                 waiting = true;
                 for (int i = 0; i < nInst; ++i) {
                     fb->live[i] = hctl[i].outerDone ? 0 : 1;
-                    if (!hctl[i].outerDone && !hctl[i].innerDone) waiting = false;
+                    if (hctl[i].outerDone || hctl[i].innerDone) continue;
+                    waiting = false;
+                    watch.look(i, hctl[i]);
                 }
             }
             // an instance that finished meanwhile leaves nothing to continue when it was the last

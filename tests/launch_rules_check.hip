@@ -53,9 +53,38 @@ static void passRule() {
     CHECK(rule.choose(true, {0}) == 1);
 }
 
+static void progressWatch() {
+    ProgressWatch watch(2);
+    auto looks = [&](int i, Ctl c, int n) {
+        try {
+            for (int k = 0; k < n; ++k) watch.look(i, c);
+        } catch (const HipError&) {
+            return true;
+        }
+        return false;
+    };
+    Ctl c = ctlAt(0, 0);
+    for (int k = 0; k < 200; ++k) {  // steps of a PCG, of an outer loop without one
+        ++c.pIt;
+        CHECK(!looks(0, c, 1));
+    }
+    for (int k = 0; k < 200; ++k) {
+        ++c.iCorr;
+        CHECK(!looks(0, c, 1));
+        CHECK(!looks(1, c, 1));
+    }
+    c.pending = 99;  // a step that no launch takes on; the other instance goes on
+    CHECK(!looks(0, c, 4));
+    ++c.iCorr;
+    CHECK(!looks(1, c, 4));
+    CHECK(!looks(0, c, 4));
+    CHECK(looks(0, c, 100));
+    CHECK(!looks(1, c, 2));
+}
+
 int main(int argc, char** argv) {
     const std::string only = argc > 1 ? argv[1] : "";
-    const std::pair<const char*, void (*)()> checks[] = {{"passRule", passRule}};
+    const std::pair<const char*, void (*)()> checks[] = {{"passRule", passRule}, {"progressWatch", progressWatch}};
     for (const auto& c : checks)
         if (only.empty() || only == c.first) c.second();
     return failures ? 1 : 0;
