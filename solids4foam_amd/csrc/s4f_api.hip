@@ -1045,6 +1045,12 @@ void parallelFor(int n, int grain, F&& f) {
     if (err) std::rethrow_exception(err);
 }
 
+// Waits for a stream when its scope is left, by an error too.
+struct StreamQuiet {
+    hipStream_t s;
+    ~StreamQuiet() { (void)hipStreamSynchronize(s); }
+};
+
 // Fields to the caller's arrays, whose rows hold a cell's k components: the
 // device transposes a chunk, which goes through pinned memory and is copied out
 // by several threads while the next one is on its way.  Downloading the
@@ -1058,6 +1064,8 @@ struct RowField {
 };
 void downloadRows(s4f_ctx* ctx, const std::vector<RowField>& fields, hipStream_t s) {
     std::lock_guard<std::mutex> lock(ctx->stageMutex);
+    // an error leaves no transfer behind that the next call's chunks would meet
+    StreamQuiet quiet{s};
     size_t need = 0, chunk = (size_t)1 << 14;
     for (const RowField& f : fields) need += (size_t)f.n * f.k;
     if (need == 0) return;
@@ -2526,10 +2534,8 @@ void solveT(s4f_mesh* M, const s4f_solve_opts& o, std::vector<InstanceIO>& io, F
         flight[k].h = hctl + (size_t)k * nInst;
         HIP_CHECK(hipEventCreateWithFlags(&flight[k].ev, hipEventDisableTiming));
     }
-    struct Quiet {  // what is queued reads the graphs and writes the host copies, also when an error ends the loop
-        hipStream_t s;
-        ~Quiet() { (void)hipStreamSynchronize(s); }
-    } quiet{s};
+    // what is queued reads the graphs and writes the host copies, also when an error ends the loop
+    StreamQuiet quiet{s};
     // bursts grow with the passes already made: a short solve wastes little at its end
     LookPace pace;
     auto burst = [&](Flight& f) {
