@@ -373,7 +373,9 @@ enum { S4F_KERNEL_RESIDUAL = 0,   /* div(sigma) + Rhie-Chow face loop */
 /* Replays `kernel` back to back `launches` times on the mesh's current state
    (e.g. right after a solve) with all three components active, on the
    context's stream between one pair of hipEvents, and returns the average
-   duration in ms.  Launch-by-launch events would perturb the caches the
+   duration in ms.  Replayed is the form of the kernel that a solve of this
+   mesh launches; S4F_KERNEL_FINALIZE gives 0 for a mesh whose solves launch
+   none (one slot count and few workgroup tiles).  Launch-by-launch events would perturb the caches the
    kernels rely on; this is the steady per-launch time. */
 s4f_status s4f_kernel_time(s4f_mesh *mesh, int32_t kernel, int32_t precision, int32_t launches, double *avgMs);
 /* Runs a plain streaming copy kernel (k_copy) of `bytes` read + `bytes`

@@ -975,26 +975,41 @@ void launchFin(const BlockMap& bm, int nFin, const Chain& c, const Ctl* in, Ctl*
         hipLaunchKernelGGL((k_fin<POINT>), dim3(nFin), dim3(kFinBlock), 0, s, bm, c.at(in, out), part);
 }
 
-// search direction + SpMV, alpha, solution / residual update of one PCG
-// iteration; `in`: the control blocks to start from, `again`: they may hold a
-// previous iteration of the same pass
+// search direction + SpMV; `in`: the control blocks to start from, `again`:
+// they may hold a previous iteration of the same pass
+template <typename T, bool MG, bool AGAIN>
+void launchSpmv(const DevMesh& dm, const BlockMap& bm, const PcgVecs<T>& v, const Chain& c, const Ctl* in, double* part,
+                hipStream_t s) {
+    const dim3 g(bm.nBlocks), b(kBlock);
+    if (c.merged)
+        hipLaunchKernelGGL((dm.uniW == 6 ? k_spmvp_m<T, MG, AGAIN, 6> : k_spmvp_m<T, MG, AGAIN, 4>), g, b, 0, s, dm, bm,
+                           (const T*)v.r, v.p, v.p2, v.q, c.at(in, c.v), part, (const T*)v.z);
+    else
+        hipLaunchKernelGGL((k_spmvp<T, MG>), g, b, 0, s, dm, bm, (const T*)v.r, v.p, v.p2, v.q, (const Ctl*)c.x, part, 1,
+                           (const T*)v.z);
+}
+
+// solution and residual update
+template <typename T>
+void launchUpdate(const DevMesh& dm, const BlockMap& bm, const PcgVecs<T>& v, const Chain& c, double* part,
+                  hipStream_t s) {
+    const dim3 g(bm.nBlocks), b(kBlock);
+    if (c.merged)
+        hipLaunchKernelGGL((k_update_m<T>), g, b, 0, s, dm, bm, v.x, (const T*)v.p, (const T*)v.p2, v.r, (const T*)v.q,
+                           c.at(c.v, c.x), part);
+    else
+        hipLaunchKernelGGL((k_update<T>), g, b, 0, s, dm, bm, v.x, (const T*)v.p, (const T*)v.p2, v.r, (const T*)v.q,
+                           (const Ctl*)c.x, part);
+}
+
+// search direction + SpMV, alpha, solution / residual update of one PCG iteration
 template <typename T, bool MG, bool AGAIN>
 void launchPcgBody(const DevMesh& dm, const BlockMap& bm, int nFin, const PcgVecs<T>& v, const Chain& c, const Ctl* in,
                    double* part, hipStream_t s) {
-    const dim3 g(bm.nBlocks), b(kBlock);
-    if (c.merged) {
-        hipLaunchKernelGGL((dm.uniW == 6 ? k_spmvp_m<T, MG, AGAIN, 6> : k_spmvp_m<T, MG, AGAIN, 4>), g, b, 0, s, dm, bm, (const T*)v.r, v.p, v.p2, v.q, c.at(in, c.v),
-                           part, (const T*)v.z);
-        hipLaunchKernelGGL((k_update_m<T>), g, b, 0, s, dm, bm, v.x, (const T*)v.p, (const T*)v.p2, v.r, (const T*)v.q,
-                           c.at(c.v, c.x), part);
-        return;
-    }
-    launchFin<MG ? kPtSpmv : AGAIN ? kPtAgain : kPtInner>(bm, nFin, c, c.x, c.x, part, s);
-    hipLaunchKernelGGL((k_spmvp<T, MG>), g, b, 0, s, dm, bm, (const T*)v.r, v.p, v.p2, v.q, (const Ctl*)c.x, part, 1,
-                       (const T*)v.z);
-    launchFin<kPtUpdate>(bm, nFin, c, c.x, c.x, part, s);
-    hipLaunchKernelGGL((k_update<T>), g, b, 0, s, dm, bm, v.x, (const T*)v.p, (const T*)v.p2, v.r, (const T*)v.q,
-                       (const Ctl*)c.x, part);
+    if (!c.merged) launchFin<MG ? kPtSpmv : AGAIN ? kPtAgain : kPtInner>(bm, nFin, c, c.x, c.x, part, s);
+    launchSpmv<T, MG, AGAIN>(dm, bm, v, c, in, part, s);
+    if (!c.merged) launchFin<kPtUpdate>(bm, nFin, c, c.x, c.x, part, s);
+    launchUpdate<T>(dm, bm, v, c, part, s);
 }
 
 // `n` diagonal PCG iterations from the state in c.x (a pending start already
@@ -1885,6 +1900,19 @@ MgRun meshRun(s4f_mesh* M, bool smoothed) {
     return MgRun{&A.d, A.omega, A.alpha, (int)M->h.instCell0.size()};
 }
 
+// level-0 smoothing from zero and its residual
+template <typename T, bool AGAIN>
+void launchMg0Down(AmgDevLevel& D0, const DevMesh& dm, const BlockMap& bm, const PcgVecs<T>& v, double omega,
+                   const Chain& c, const Ctl* in, double* part, hipStream_t s) {
+    const dim3 g(bm.nBlocks), b(kBlock);
+    if (c.merged)
+        hipLaunchKernelGGL((dm.uniW == 6 ? k_mg0_down_m<T, AGAIN, 6> : k_mg0_down_m<T, AGAIN, 4>), g, b, 0, s, dm, bm,
+                           (const T*)v.r, MgVec<T>::r0(D0), omega, c.at(in, c.w), (const double*)part);
+    else
+        hipLaunchKernelGGL((k_mg0_down<T>), g, b, 0, s, dm, bm, (const T*)v.r, MgVec<T>::r0(D0), omega,
+                           (const Ctl*)c.x);
+}
+
 // level-0 prolongation + post-smoothing: the aggregation form (q) or, on a
 // smoothed hierarchy, the G form
 template <typename T>
@@ -1915,15 +1943,9 @@ void launchVcycle(const MgRun& R, const DevMesh& dm, const BlockMap& bm, const P
     const int nl = (int)A.d.size();
     const double w = R.omega;
     AmgDevLevel& D0 = *A.d[0];
-    Row3<T>* r0 = MgVec<T>::r0(D0);
-    if (ch.merged) {
-        hipLaunchKernelGGL((dm.uniW == 6 ? k_mg0_down_m<T, AGAIN, 6> : k_mg0_down_m<T, AGAIN, 4>), dim3(bm.nBlocks), dim3(kBlock), 0, s, dm, bm, (const T*)v.r, r0, w,
-                           ch.at(in, ch.w), (const double*)part);
-    } else {
-        launchFin<AGAIN ? kPtAgain : kPtInner>(bm, R.nFin, ch, ch.x, ch.x, part, s);
-        hipLaunchKernelGGL((k_mg0_down<T>), dim3(bm.nBlocks), dim3(kBlock), 0, s, dm, bm, (const T*)v.r, r0, w,
-                           (const Ctl*)ch.x);
-    }
+    const Row3<T>* r0 = MgVec<T>::r0(D0);
+    if (!ch.merged) launchFin<AGAIN ? kPtAgain : kPtInner>(bm, R.nFin, ch, ch.x, ch.x, part, s);
+    launchMg0Down<T, AGAIN>(D0, dm, bm, v, w, ch, in, part, s);
     if (nl > 1) {
         // down: restrict the finer level's residual (with the coarse
         // pre-smoothing), then the coarse residual
@@ -1935,10 +1957,10 @@ void launchVcycle(const MgRun& R, const DevMesh& dm, const BlockMap& bm, const P
             const dim3 gr(gridRows(8 * (long long)L.n));
             if (l == 1 && L.rMem.p)  // smoothed prolongation: weighted lists in sliced ELL
                 hipLaunchKernelGGL((k_mg_restrict_w<T>), dim3(gridSlices(L.nSlices)), dim3(kBlock), 0, s, L.view(),
-                                   (const Row3<T>*)r0, b, x, w, (const Ctl*)ctl);
+                                   r0, b, x, w, (const Ctl*)ctl);
             else if (l == 1)
-                hipLaunchKernelGGL((k_mg_restrict<T, Row3<T>>), gr, dim3(kBlock), 0, s, L.view(), (const Row3<T>*)r0, b, x,
-                                   w, (const Ctl*)ctl);
+                hipLaunchKernelGGL((k_mg_restrict<T, Row3<T>>), gr, dim3(kBlock), 0, s, L.view(), r0, b, x, w,
+                                   (const Ctl*)ctl);
             else
                 hipLaunchKernelGGL((k_mg_restrict<T, Row4<T>>), gr, dim3(kBlock), 0, s, L.view(),
                                    (const Row4<T>*)MgVec<T>::r(Lf), b, x, w, (const Ctl*)ctl);
@@ -2150,28 +2172,45 @@ auto residualUniform(const DevMesh& dm) {
     if (dm.uniW == 6) return dm.mu ? k_residual_u<T, 6, true, MERGED> : k_residual_u<T, 6, false, MERGED>;
     return dm.mu ? k_residual_u<T, 4, true, MERGED> : k_residual_u<T, 4, false, MERGED>;
 }
+// boundary values, gradients and boundary stress of an outer iteration: one
+// launch where the sequence is merged, else launchGradStep's on `c.y`
+inline bool gradMerged(const DevMesh& dm, const GradBufs& f, const Chain& c) {
+    return c.merged && !f.aAlpha && dm.nIf == 0;
+}
+template <typename T>
+void launchGrad(const DevMesh& dm, const BlockMap& bm, int nFin, int maxNB, const GradBufs& f, const PcgVecs<T>& v,
+                const double* Dold, const Chain& c, double* part, hipStream_t s) {
+    if (gradMerged(dm, f, c))
+        hipLaunchKernelGGL((dm.uniW == 6 ? k_grad_m<T, 6> : k_grad_m<T, 4>), dim3(bm.nBlocks), dim3(kBlock), 0, s, dm,
+                           bm, f.D0, (const T*)v.x, f.D1, f.G, f.Db, Dold, c.at(c.x, c.y), part,
+                           BndBufs{f.g, f.snb, f.Gb, f.sigb});
+    else
+        launchGradStep<T>(dm, bm, nFin, maxNB, f, (const T*)v.x, Dold, c.y, part, 0, s);
+}
+
+// the residual of an outer iteration
+template <typename T>
+void launchResidual(const DevMesh& dm, const BlockMap& bm, const GradBufs& f, const PcgVecs<T>& v, const Chain& c,
+                    double* part, hipStream_t s) {
+    const dim3 g(bm.nBlocks), b(kBlock);
+    if (uniformSlots(dm))
+        hipLaunchKernelGGL((c.merged ? residualUniform<T, true>(dm) : residualUniform<T, false>(dm)), g, b, 0, s, dm, bm,
+                           (const double*)f.D0, (const double*)f.D1, (const double*)f.G, (const double*)f.sigb, v.r,
+                           c.at(c.y, c.z), part);
+    else
+        hipLaunchKernelGGL((k_residual<T>), g, b, 0, s, dm, bm, (const double*)f.D0, (const double*)f.D1,
+                           (const double*)f.G, (const double*)f.sigb, v.r, (const Ctl*)c.x, part);
+}
+
 // The outer step of the momentum loop for the instances whose PCG has
 // finished: gradient step, convergence test, residual (the others skip it).
 template <typename T>
 void launchOuter(const DevMesh& dm, const BlockMap& bm, int nFin, int maxNB, const GradBufs& f, const PcgVecs<T>& v,
                  const double* Dold, const Chain& c, double* part, hipStream_t s) {
-    const bool uni = uniformSlots(dm);
-    if (c.merged && !f.aAlpha && dm.nIf == 0) {
-        hipLaunchKernelGGL((dm.uniW == 6 ? k_grad_m<T, 6> : k_grad_m<T, 4>), dim3(bm.nBlocks), dim3(kBlock), 0, s, dm,
-                           bm, f.D0, (const T*)v.x, f.D1, f.G, f.Db, Dold, c.at(c.x, c.y), part,
-                           BndBufs{f.g, f.snb, f.Gb, f.sigb});
-    } else {
-        launchFin<kPtGrad>(bm, nFin, c, c.x, c.y, part, s);
-        launchGradStep<T>(dm, bm, nFin, maxNB, f, (const T*)v.x, Dold, c.y, part, 0, s);
-    }
+    if (!gradMerged(dm, f, c)) launchFin<kPtGrad>(bm, nFin, c, c.x, c.y, part, s);
+    launchGrad<T>(dm, bm, nFin, maxNB, f, v, Dold, c, part, s);
     if (!c.merged) launchFin<kPtRes>(bm, nFin, c, c.x, c.x, part, s);
-    if (uni)
-        hipLaunchKernelGGL((c.merged ? residualUniform<T, true>(dm) : residualUniform<T, false>(dm)), dim3(bm.nBlocks),
-                           dim3(kBlock), 0, s, dm, bm, (const double*)f.D0, (const double*)f.D1, (const double*)f.G,
-                           (const double*)f.sigb, v.r, c.at(c.y, c.z), part);
-    else
-        hipLaunchKernelGGL((k_residual<T>), dim3(bm.nBlocks), dim3(kBlock), 0, s, dm, bm, (const double*)f.D0,
-                           (const double*)f.D1, (const double*)f.G, (const double*)f.sigb, v.r, (const Ctl*)c.x, part);
+    launchResidual<T>(dm, bm, f, v, c, part, s);
 }
 
 // One pass of the momentum loop's launch sequence: the outer step of every
@@ -3353,11 +3392,11 @@ s4f_status s4f_residual(s4f_mesh* M, const double* D, const double* gradD, const
         Ctl c0;
         std::memset(&c0, 0, sizeof(c0));
         c0.pending = kPendRes;
-        HIP_CHECK(hipMemcpyAsync(st.ctl.p, &c0, sizeof(Ctl), hipMemcpyHostToDevice, s));
         const DevMesh dm = M->dm();
         const BlockMap bm = M->bmap();
-        hipLaunchKernelGGL((k_residual<double>), dim3(bm.nBlocks), dim3(kBlock), 0, s, dm, bm, (const double*)st.D0.p,
-                           (const double*)st.D1.p, (const double*)st.G.p, (const double*)st.sigb.p, v.r, (const Ctl*)st.ctl.p, st.part.p);
+        const Chain chain(st.ctl.p, 1, canMerge(dm, bm.nBlocks), nullptr);
+        HIP_CHECK(hipMemcpyAsync(chain.y, &c0, sizeof(Ctl), hipMemcpyHostToDevice, s));
+        launchResidual<double>(dm, bm, meshGradBufs(M), v, chain, st.part.p, s);
         HIP_CHECK(hipGetLastError());
         soaToAos(download(st.r64, 3 * (size_t)C, s), C, 3, R);
         return S4F_OK;
@@ -3579,64 +3618,54 @@ double replayT(s4f_mesh* M, int kernel, int launches) {
     std::memset(&c, 0, sizeof(c));
     for (int j = 0; j < 3; ++j) { c.active[j] = 1; c.alpha[j] = 0.5; c.beta[j] = 0.5; c.rho[j] = 1.0; c.normFactor[j] = 1.0; }
     c.pcgMaxIter = 1;
-    // the point of the solve at which the kernel runs; the kernels leave the
-    // control block as it is, the finalize kernels' results go to a second one
+    // the point of the solve at which the kernel runs, in the form that a solve
+    // takes: the kernels leave the control block as it is (merged ones copy it),
+    // the finalize kernels' results go to the last one
     c.pending = kernel == S4F_KERNEL_RESIDUAL ? kPendRes
                 : kernel == S4F_KERNEL_GRAD ? kPendGrad
                 : kernel == S4F_KERNEL_PCG_UPDATE ? kPendUpd : kPendSpmv;
+    const std::vector<Ctl> cs(kChain, c);
     DArr<Ctl> rc;
-    rc.alloc(2);
-    Chain chain(rc.p, 1, false, nullptr);
-    HIP_CHECK(hipMemcpyAsync(rc.p, &c, sizeof(Ctl), hipMemcpyHostToDevice, s));
+    rc.upload(cs, s);
+    const Chain chain(rc.p, 1, canMerge(dm, bm.nBlocks), nullptr);
+    // a merged sequence has no finalize launch
+    if (kernel == S4F_KERNEL_FINALIZE && chain.merged) {
+        HIP_CHECK(hipStreamSynchronize(s));
+        return 0.0;
+    }
     // the multigrid kernels replay the hierarchy of the mesh's last multigrid solve
     const bool smoothedK = M->amgLast == &M->amgSm;
     Amg& AK = smoothedK ? M->amgSm : M->amg;
     auto launch = [&]() {
         switch (kernel) {
             case S4F_KERNEL_RESIDUAL:
-                if (uniformSlots(dm)) {  // as launchOuter without merged points
-                    hipLaunchKernelGGL((residualUniform<T, false>(dm)), dim3(bm.nBlocks), dim3(kBlock), 0, s, dm, bm,
-                                       (const double*)st.D0.p, (const double*)st.D1.p, (const double*)st.G.p,
-                                       (const double*)st.sigb.p, v.r, chain.at(rc.p, rc.p + 1), st.part.p);
-                    break;
-                }
-                hipLaunchKernelGGL((k_residual<T>), dim3(bm.nBlocks), dim3(kBlock), 0, s, dm, bm,
-                                   (const double*)st.D0.p, (const double*)st.D1.p, (const double*)st.G.p,
-                                   (const double*)st.sigb.p, v.r, (const Ctl*)rc.p, st.part.p);
+                launchResidual<T>(dm, bm, meshGradBufs(M), v, chain, st.part.p, s);
                 break;
             case S4F_KERNEL_SPMV:
-                hipLaunchKernelGGL((k_spmvp<T, false>), dim3(bm.nBlocks), dim3(kBlock), 0, s, dm, bm, (const T*)v.r,
-                                   v.p, v.p2, v.q, (const Ctl*)rc.p, st.part.p, 1, (const T*)nullptr);
+                launchSpmv<T, false, false>(dm, bm, v, chain, chain.z, st.part.p, s);
                 std::swap(v.p, v.p2);
                 break;
             case S4F_KERNEL_SPMV_MG:
-                hipLaunchKernelGGL((k_spmvp<T, true>), dim3(bm.nBlocks), dim3(kBlock), 0, s, dm, bm, (const T*)v.r,
-                                   v.p, v.p2, v.q, (const Ctl*)rc.p, st.part.p, 1, (const T*)v.z);
+                launchSpmv<T, true, false>(dm, bm, v, chain, chain.w, st.part.p, s);
                 std::swap(v.p, v.p2);
                 break;
             case S4F_KERNEL_PCG_UPDATE:
-                hipLaunchKernelGGL((k_update<T>), dim3(bm.nBlocks), dim3(kBlock), 0, s, dm, bm, v.x, (const T*)v.p,
-                                   (const T*)v.p2, v.r, (const T*)v.q, (const Ctl*)rc.p, st.part.p);
+                launchUpdate<T>(dm, bm, v, chain, st.part.p, s);
                 break;
             case S4F_KERNEL_FINALIZE:
-                launchFin<kPtUpdate>(bm, 1, chain, rc.p, rc.p + 1, st.part.p, s);
+                launchFin<kPtUpdate>(bm, 1, chain, rc.p, rc.p + kChain - 1, st.part.p, s);
                 break;
             case S4F_KERNEL_GRAD:
-                launchGradStep<T>(dm, bm, 1, M->maxInstNB,
-                                  meshGradBufs(M),
-                                  (const T*)v.x, nullptr, rc.p, st.part.p, 0, s);
+                launchGrad<T>(dm, bm, 1, M->maxInstNB, meshGradBufs(M), v, nullptr, chain, st.part.p, s);
                 break;
-            case S4F_KERNEL_MG0_DOWN: {
-                AmgDevLevel& D0 = *AK.d[0];
-                hipLaunchKernelGGL((k_mg0_down<T>), dim3(bm.nBlocks), dim3(kBlock), 0, s, dm, bm, (const T*)v.r,
-                                   MgVec<T>::r0(D0), AK.omega, (const Ctl*)rc.p);
+            case S4F_KERNEL_MG0_DOWN:
+                launchMg0Down<T, false>(*AK.d[0], dm, bm, v, AK.omega, chain, chain.z, st.part.p, s);
                 break;
-            }
             case S4F_KERNEL_MG0_UP:
-                launchMg0Up<T>(AK.d, dm, bm, v, AK.omega, AK.alpha, rc.p, st.part.p, s);
+                launchMg0Up<T>(AK.d, dm, bm, v, AK.omega, AK.alpha, chain.w, st.part.p, s);
                 break;
             case S4F_KERNEL_VCYCLE:
-                launchVcycle<T, false>(meshRun(M, smoothedK), dm, bm, v, chain, rc.p, st.part.p, s);
+                launchVcycle<T, false>(meshRun(M, smoothedK), dm, bm, v, chain, chain.z, st.part.p, s);
                 break;
             default:
                 throw InvalidError("unknown kernel id");
