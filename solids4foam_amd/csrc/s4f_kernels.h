@@ -833,6 +833,10 @@ __global__ __launch_bounds__(kBlock, 5) void k_spmvp(const DevMesh m, const Bloc
                     z[u] = reduce ? src[i] : (T)0;
                     o[u] = pOld[i];
                 }
+                if (!reduce) {  // a caller's vector: zero times its own infinity would be NaN
+#pragma unroll
+                    for (int u = 0; u < kRowChunk; ++u) o[u] = c[u] == P ? (T)0 : o[u];
+                }
 #pragma unroll
                 for (int u = 0; u < kRowChunk; ++u) y[j] = fmaT(-av[u], dir(j, z[u], iD[u], o[u]), y[j]);
             }

@@ -67,3 +67,21 @@ def test_kernel_times(ctx, n, tets, tiles, merged, precision):
     assert all(v > 0.0 for v in t.values())
     b = m.solve(**opts)
     assert np.array_equal(a["D"], b["D"]) and np.array_equal(a["sigma"], b["sigma"])
+
+
+@pytest.mark.parametrize("mixed", [False, True])
+@pytest.mark.parametrize("n,tets", [((5, 4, 3), False), ((3, 3, 2), True)])
+def test_product_of_an_infinite_value(ctx, n, tets, mixed):
+    # an infinite entry reaches its own row and its neighbours', as infinity: an
+    # empty or boundary slot adds nothing, also where the row's value is infinite
+    print(f"[forms] infinite value {n} tets={tets} mixed={mixed}", flush=True)
+    m, _, _ = _mesh(ctx, n, tets, None)
+    C = m.nCells
+    for cell in (0, C // 2, C - 1):
+        x = np.zeros((C, 3))
+        x[cell] = 1.0
+        reach = m.spmv3(x, mixed=mixed) != 0.0
+        x[cell] = np.inf
+        y = m.spmv3(x, mixed=mixed)
+        assert reach[cell].all() and not np.isnan(y).any()
+        assert np.array_equal(np.isinf(y), reach) and (y[cell] > 0).all()
