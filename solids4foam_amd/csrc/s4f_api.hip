@@ -4880,6 +4880,16 @@ s4f_status s4f_server_destroy(s4f_server* S) {
 // ===========================================================================
 // lduMatrix::solver entry: PCG on a caller's LDU matrix (OpenFOAM addressing)
 // ===========================================================================
+// One slot count for the slices of an LDU matrix, or 0 for each its own.  The
+// slices of a mesh's boundary have a slot or two less: one count for all (empty
+// slots) opens the merged launch sequence, while it costs at most a quarter more
+// entries and their numbers still fit 32 bits.  wmax: the widest slice; slots: of
+// all slices together.
+int lduSlotCount(int wmax, int nSlices, long long slots) {
+    const long long w = wmax <= 4 ? 4 : 6;
+    return wmax <= w && 4 * w * nSlices <= 5 * slots && w * nSlices * kSlice <= INT32_MAX ? (int)w : 0;
+}
+
 struct s4f_ldu {
     s4f_ctx* ctx = nullptr;
     std::unique_ptr<s4f_mesh> M;   // ELL structure + PCG state (no geometry)
@@ -4922,11 +4932,8 @@ s4f_status s4f_ldu_create(s4f_ctx* ctx, int32_t nCells, int32_t nFaces, const in
             slots += h.sliceWidth[sI];
             wmax = std::max(wmax, h.sliceWidth[sI]);
         }
-        // the slices of a mesh's boundary have a slot or two less: one slot
-        // count for all (empty slots) opens the merged launch sequence, while
-        // it costs at most a quarter more entries
-        const int wUni = wmax <= 4 ? 4 : 6;
-        if (wmax <= 6 && 4LL * wUni * h.nSlices <= 5 * slots) std::fill(h.sliceWidth.begin(), h.sliceWidth.end(), wUni);
+        const int wUni = lduSlotCount(wmax, h.nSlices, slots);
+        if (wUni) std::fill(h.sliceWidth.begin(), h.sliceWidth.end(), wUni);
         size_t E = 0;
         for (int sI = 0; sI < h.nSlices; ++sI) {
             h.sliceStart[sI] = (int)E;

@@ -82,9 +82,24 @@ static void progressWatch() {
     CHECK(!looks(1, c, 2));
 }
 
+static void lduSlots() {
+    CHECK(lduSlotCount(6, 100, 600) == 6);
+    CHECK(lduSlotCount(6, 100, 480) == 6);  // a quarter more entries
+    CHECK(lduSlotCount(6, 100, 479) == 0);
+    CHECK(lduSlotCount(4, 100, 320) == 4);
+    CHECK(lduSlotCount(5, 100, 500) == 6);
+    CHECK(lduSlotCount(7, 100, 700) == 0);
+    CHECK(lduSlotCount(0, 1, 0) == 0);      // a single cell
+    // rows of five: their entries can be numbered, six for each could not
+    const int most = INT32_MAX / (6 * kSlice);
+    CHECK(lduSlotCount(5, most, 5LL * most) == 6);
+    CHECK(lduSlotCount(5, most + 1, 5LL * (most + 1)) == 0);
+}
+
 int main(int argc, char** argv) {
     const std::string only = argc > 1 ? argv[1] : "";
-    const std::pair<const char*, void (*)()> checks[] = {{"passRule", passRule}, {"progressWatch", progressWatch}};
+    const std::pair<const char*, void (*)()> checks[] = {{"passRule", passRule}, {"progressWatch", progressWatch},
+                                                         {"lduSlots", lduSlots}};
     for (const auto& c : checks)
         if (only.empty() || only == c.first) c.second();
     return failures ? 1 : 0;

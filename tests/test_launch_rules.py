@@ -19,7 +19,7 @@ def harness(tmp_path_factory):
     return out
 
 
-@pytest.mark.parametrize("rule", ["passRule", "progressWatch"])
+@pytest.mark.parametrize("rule", ["passRule", "progressWatch", "lduSlots"])
 def test_rule(harness, rule):
     r = subprocess.run([harness, rule], capture_output=True, text=True, timeout=60)
     assert r.returncode == 0, r.stdout + r.stderr
