@@ -2231,10 +2231,15 @@ void launchPass(bool mg, const MgRun& R, const DevMesh& dm, const BlockMap& bm, 
 // launches follows from how many iterations the live instances take per outer
 // one, which varies little from one to the next: an instance of u needs
 // ceil(u / k) passes, each of k iterations and the outer step's launches (about
-// half of an iteration's with a V-cycle, twice those of a diagonal one).
+// half of an iteration's with a V-cycle, twice those of a diagonal one).  The
+// instances count by the square of the outer iterations they have left,
+// estimated from the residual's fall so far: the last to finish sets the time.
 // One iteration a pass for up to four per outer one -> this rule, us per outer
-// iteration: 128^3 cells FP32 (3.5 per outer one) 1,610 -> 1,551, 64^3 FP32
-// (2.6) 312 -> 293; 64 served requests of up to 128^3 cells 54.3 -> 44.1 s.
+// iteration: 128^3 cells FP32 (3.5 per outer one) 1,610 -> 1,545, 64^3 FP32
+// (2.6) 312 -> 290; 24 boxes in a batch 431 -> 347 ms, 64 served requests of up
+// to 128^3 cells 54.3 -> 42.6 s.  Weights 1 / the iterations left / their squares:
+// six boxes of 2 and one of 1.1 with most of the iterations 870 / 861 / 851 ms
+// (one iteration a pass: 848), a served burst of seven 311 / 294 / 290.
 class PassRule {
   public:
     explicit PassRule(size_t n) : seen_(n) {}
@@ -2250,22 +2255,22 @@ class PassRule {
         } else {  // the first outer iteration, or one longer than a look
             s.mean = std::max({s.mean, (double)c.nIter[0], (double)c.nIter[1], (double)c.nIter[2]});
         }
+        const double tol = std::max({c.solTol, c.altTol, 1e-16}), res = std::min(c.initResMag, 0.5);
+        s.left = 1.0;
+        if (c.iCorr > 0 && res > tol)
+            s.left = std::max(1.0, std::min(c.iCorr * std::log(res / tol) / -std::log(res), (double)c.nCorr - c.iCorr));
     }
-    int choose(bool mg, const std::vector<int>& live) const {
-        const double outer = mg ? 0.5 : 2.0;
+    // launched: PCG iterations launched so far.  What is queued at the end of a
+    // solve is for nothing, so long passes wait until it is long itself.
+    int choose(bool mg, const std::vector<int>& live, long long launched) const {
+        const long long most = std::max(mg ? 2LL : 4LL, launched / 8);
         int best = 1;
         double least = HUGE_VAL;
         for (int k : {1, 2, 3, 4, 5, 6, 8, 12, 16}) {
-            double passes = 0.0;
-            for (int i : live) {
-                const double u = std::max(1.0, seen_[i].mean), n = std::floor(u);
-                // a mean between two counts: so many of each; large counts vary by more than k
-                passes += n > 8.0 ? u / k + 0.5
-                                  : (1.0 - (u - n)) * std::ceil(n / k) + (u - n) * std::ceil((n + 1.0) / k);
-            }
-            const double cost = (outer + k) * passes;
-            if (cost < least) {
-                least = cost;
+            if (k > most) break;
+            const double c = cost(mg, live, k);
+            if (c < least) {
+                least = c;
                 best = k;
             }
         }
@@ -2276,8 +2281,19 @@ class PassRule {
     struct Seen {
         int iCorr = 0;
         long long pcg = 0;
-        double mean = 0.0;
+        double mean = 0.0, left = 1.0;
     };
+    double cost(bool mg, const std::vector<int>& live, int k) const {
+        double passes = 0.0;
+        for (int i : live) {
+            const double u = std::max(1.0, seen_[i].mean), n = std::floor(u);
+            // a mean between two counts: so many of each; large counts vary by more than k
+            const double p = n > 8.0 ? u / k + 0.5
+                                     : (1.0 - (u - n)) * std::ceil(n / k) + (u - n) * std::ceil((n + 1.0) / k);
+            passes += seen_[i].left * seen_[i].left * p;
+        }
+        return ((mg ? 0.5 : 2.0) + k) * passes;
+    }
     std::vector<Seen> seen_;
 };
 
@@ -2366,6 +2382,45 @@ struct GraphExec {
         }
     }
     void launch(hipStream_t s) const { HIP_CHECK(hipGraphLaunch(e, s)); }
+};
+
+// Graphs of passes, one per number of PCG iterations.  A capture costs as much
+// as several passes launched one by one (30 to 50 us per iteration on two to
+// four levels), and the number changes while a solve settles: a number is
+// captured once it has been taken a few times.
+class PassGraphs {
+  public:
+    void clear() { entries_.clear(); }
+    // one pass of k iterations on stream s; `graphs` is cleared where the runtime cannot capture
+    template <typename F>
+    void run(int k, hipStream_t capture, hipStream_t s, bool& graphs, F&& launch) {
+        if (graphs) {
+            Entry& e = entries_[k];
+            if (!e.graph.e && e.taken++ >= kEager) {
+                try {
+                    e.graph.capture(capture, launch);
+                } catch (const HipError&) {  // the same launches, one by one
+                    (void)hipGetLastError();
+                    HIP_CHECK(hipStreamSynchronize(s));
+                    entries_.clear();
+                    graphs = false;
+                }
+            }
+            if (graphs && e.graph.e) {
+                e.graph.launch(s);
+                return;
+            }
+        }
+        launch(s);
+    }
+
+  private:
+    static constexpr int kEager = 4;  // the first of them allocates every buffer
+    struct Entry {
+        GraphExec graph;
+        int taken = 0;
+    };
+    std::map<int, Entry> entries_;
 };
 
 struct InstanceIO {
@@ -2534,34 +2589,20 @@ void solveT(s4f_mesh* M, const s4f_solve_opts& o, std::vector<InstanceIO>& io, F
     };
     // A pass advances every instance from where it stands, so the host launches
     // passes without knowing where that is and looks at the control blocks of
-    // an earlier burst while the next one runs.  After the first pass (which
-    // allocates every buffer) passes are replayed from HIP graphs, one per
-    // number of PCG iterations in a pass.
+    // an earlier burst while the next one runs.
     bool graphs = o.eagerLaunch == 0;
-    std::map<int, GraphExec> graph;
+    PassGraphs graph;
     int inner = mg ? 1 : 4;
     PassRule rule(nInst);
     ProgressWatch watch(nInst);
-    long long passes = 0;
+    long long passes = 0, launched = 0;
     auto pass = [&]() {
         auto launch = [&](hipStream_t q) {
             launchPass<T>(mg, mgRun, dm, bm, M->maxInstNB, gbuf, v, Dold, chain, st.part.p, inner, q);
         };
-        if (graphs && passes > 0) {
-            GraphExec& g = graph[inner];
-            if (!g.e) {
-                try {
-                    g.capture(ctx->capture, launch);
-                } catch (const HipError&) {  // a runtime without capture: the same launches, one by one
-                    (void)hipGetLastError();
-                    graph.clear();
-                    graphs = false;
-                }
-            }
-        }
-        if (graphs && passes > 0) graph[inner].launch(s);
-        else launch(s);
+        graph.run(inner, ctx->capture, s, graphs, launch);
         ++passes;
+        launched += inner;
     };
     struct Flight {  // a burst of passes and the control blocks after it
         hipEvent_t ev = nullptr;
@@ -2602,8 +2643,8 @@ void solveT(s4f_mesh* M, const s4f_solve_opts& o, std::vector<InstanceIO>& io, F
             if (!hc[i].hold) watch.look(i, hc[i]);
         }
         if (live.empty()) break;
+        const double now = std::chrono::duration<double>(std::chrono::steady_clock::now() - tStart).count();
         if (o.progressSeconds > 0) {  // the per-iteration log, rate-limited
-            const double now = std::chrono::duration<double>(std::chrono::steady_clock::now() - tStart).count();
             if (now - tShown >= o.progressSeconds) {
                 tShown = now;
                 int iMax = 0;
@@ -2617,7 +2658,7 @@ void solveT(s4f_mesh* M, const s4f_solve_opts& o, std::vector<InstanceIO>& io, F
                 fflush(stderr);
             }
         }
-        inner = rule.choose(mg, live);
+        inner = rule.choose(mg, live, launched);
         if (stalled) {
             // every instance finishes its PCG and waits before its gradient step
             hipLaunchKernelGGL(k_ctl_hold, dim3(1), dim3(kBlock), 0, s, st.ctl.p, nInst, 1);
@@ -4022,12 +4063,10 @@ struct s4f_server {
     int maxTiles = 0;       // most tiles of an instance on the map
     int uniW = 0;           // slot count of all slices on the map, 0 when they differ
     long long liveTiles = 0;  // tiles of the map's unfinished instances
-    // passes replayed from HIP graphs (per PCG iterations in a pass) while the
-    // packed map they were captured on stands (mapGen counts rebuilds)
-    std::map<int, GraphExec> graph;
+    PassGraphs graph;  // of the packed map as it stands
+    long long launched = 0;  // PCG iterations launched on it
     PassRule rule{0};
     LookPace pace;
-    unsigned mapGen = 0, ranGen = ~0u;
     Ctl* hctl = nullptr;
     // bookkeeping (server thread only)
     std::vector<Placement> places;
@@ -4576,8 +4615,8 @@ MgRun serverRun(s4f_server* S) {
 }
 
 void serverRebuildMap(s4f_server* S) {
-    S->mapGen++;  // tiles, multigrid packing and slot set change: captured graphs are stale
-    S->graph.clear();
+    S->graph.clear();  // tiles, multigrid packing and slot set change
+    S->launched = 0;
     std::vector<int> slots;
     for (int i = 0; i < S->maxSlots; ++i)
         if (S->slotReq[i] >= 0) slots.push_back(i);
@@ -4623,26 +4662,9 @@ void serverStep(s4f_server* S) {
     // a finished solve, or an arriving one, waits this long at most
     const int passes = S->pace.passes();
     S->pace.start();
-    for (int k = 0; k < passes; ++k) {
-        // the first pass on a new map runs eagerly (it allocates the
-        // multigrid vectors of the packing); later ones are replayed
-        const bool eager = S->opts.eagerLaunch != 0 || S->ranGen != S->mapGen;
-        if (!eager) {
-            GraphExec& g = S->graph[S->inner];
-            if (!g.e) {
-                try {
-                    g.capture(S->ctx->capture, launch);
-                } catch (const HipError&) {  // a runtime without capture: the same launches, one by one
-                    (void)hipGetLastError();
-                    S->graph.clear();
-                    S->opts.eagerLaunch = 1;
-                }
-            }
-        }
-        if (!eager && S->opts.eagerLaunch == 0) S->graph[S->inner].launch(s);
-        else launch(s);
-        S->ranGen = S->mapGen;
-    }
+    bool graphs = S->opts.eagerLaunch == 0;
+    for (int k = 0; k < passes; ++k) S->graph.run(S->inner, S->ctx->capture, s, graphs, launch);
+    if (!graphs) S->opts.eagerLaunch = 1;
     // pending partials are laid out by this map: nothing stays pending over a change
     launchSettle(bm, S->nActive, chain, S->part.p, s);
     HIP_CHECK(hipGetLastError());
@@ -4655,7 +4677,8 @@ void serverStep(s4f_server* S) {
             live.push_back(sl);
             S->rule.look(sl, S->hctl[sl]);
         }
-    if (!live.empty()) S->inner = S->rule.choose(S->mgOn, live);
+    S->launched += (long long)passes * S->inner;
+    if (!live.empty()) S->inner = S->rule.choose(S->mgOn, live, S->launched);
     // retire
     bool changed = false;
     for (int sl : slots) {

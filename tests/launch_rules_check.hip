@@ -30,7 +30,7 @@ static int passLength(bool mg, const std::vector<double>& perOuter) {
         for (int it = 10; it <= 200; it += 10) rule.look(i, ctlAt(it, (long long)(it * perOuter[i])));
         live.push_back(i);
     }
-    return rule.choose(mg, live);
+    return rule.choose(mg, live, 1000);
 }
 
 static void passRule() {
@@ -48,9 +48,28 @@ static void passRule() {
     // a first outer iteration longer than a look counts as what it has used so far
     PassRule rule(1);
     rule.look(0, ctlAt(0, 0, 40));
-    CHECK(rule.choose(false, {0}) >= 8);
+    CHECK(rule.choose(false, {0}, 1000) >= 8);
     rule.reset(0);
-    CHECK(rule.choose(true, {0}) == 1);
+    CHECK(rule.choose(true, {0}, 1000) == 1);
+    // a short solve takes short passes
+    rule.look(0, ctlAt(4, 24));
+    CHECK(rule.choose(true, {0}, 1) == 2 && rule.choose(true, {0}, 24) == 3 && rule.choose(true, {0}, 48) == 6);
+    // the instance with most of the iterations left decides
+    auto at = [](int iCorr, long long pcg, double res) {
+        Ctl c = ctlAt(iCorr, pcg);
+        c.solTol = c.altTol = 1e-8;
+        c.nCorr = 100000;
+        c.initResMag = res;
+        return c;
+    };
+    PassRule two(3);
+    for (int i = 0; i < 2; ++i) two.look(i, at(100, 200, 1e-7));
+    two.look(2, at(100, 105, 0.4));
+    CHECK(two.choose(true, {0, 1, 2}, 1000) == 1);
+    two.look(2, at(100, 105, 2e-8));
+    CHECK(two.choose(true, {0, 1, 2}, 1000) == 2);
+    two.look(2, at(100, 105, NAN));
+    CHECK(two.choose(true, {0, 1, 2}, 1000) == 2);
 }
 
 static void progressWatch() {
