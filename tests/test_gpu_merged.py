@@ -147,3 +147,38 @@ def test_ldu_slot_counts(ctx, n, wide, mixed):
     got, info = LduSolver(ctx, c.size, lower, upper).solve(diag, -a, src, np.zeros(c.size), tolerance=tol, mixed=mixed)
     print(f"[ldu] {n} wide={wide} mixed={mixed}: {info['nIterations']} iterations", flush=True)
     assert np.linalg.norm(got - psi) <= (2e-4 if mixed else 2e-10) * max(1.0, np.linalg.norm(psi))
+
+
+@pytest.mark.parametrize("precision", [0, 1])
+def test_merged_equals_general_smoothed(ctx, precision):
+    # the smoothed hierarchy's weighted restriction and up sweep, in both sequences
+    from solids4foam_amd.batch import Batch
+    print(f"[merged] smoothed precision={precision}", flush=True)
+    sizes = [(1, 1, 1), (7, 3, 3), (4, 4, 4), (17, 16, 1), (23, 9, 8), (28, 25, 24)]
+    members = [_box(ctx, n, 5 + i) for i, n in enumerate(sizes)] + [_tets(ctx)]
+    opts = dict(CAPPED, precision=precision, preconditioner=3, nCorrectors=6, pcgMaxIter=100)
+    alone = [m.solve(**opts) for m in members]
+    b = Batch(ctx)
+    for m in members:
+        b.add(m)
+    for i, (r, a) in enumerate(zip(b.solve(**opts), alone)):
+        assert _same(r, a), i
+    b.close()
+
+
+@pytest.mark.parametrize("precond", [0, 3])
+def test_wide_finalize(ctx, precond):
+    # more than 4,096 tiles: finalize kernels of four runs, alone and in a batch,
+    # where members of fewer tiles keep the order of the one-run kernels
+    from solids4foam_amd.batch import Batch
+    print(f"[merged] wide finalize precond={precond}", flush=True)
+    members = [_box(ctx, n, 2, tiles=t) for n, t in (((65, 64, 64), (65536, 1)), ((64, 41, 25), (65536, 1)),
+                                                     ((23, 21, 17), (3, 4)))]
+    opts = dict(CAPPED, precision=0, preconditioner=precond, nCorrectors=4, pcgMaxIter=12)
+    alone = [m.solve(**opts) for m in members]
+    b = Batch(ctx)
+    for m in members:
+        b.add(m)
+    for i, (r, a) in enumerate(zip(b.solve(**opts), alone)):
+        assert _same(r, a), i
+    b.close()
