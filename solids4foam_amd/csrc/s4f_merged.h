@@ -1,8 +1,9 @@
-// s4f_merged.h -- kernels of merged launch sequences (Chain): meshes and
-// batch members of few tiles (kMergeTiles) and one slot count (6: hexahedra,
-// 4: tetrahedra, 2-D quadrilaterals).
+// s4f_merged.h -- kernels for one slot count (6: hexahedra, 4: tetrahedra, 2-D
+// quadrilaterals): those of merged launch sequences (Chain; meshes and batch
+// members of up to kMergeTiles tiles), and k_residual_u, which larger meshes run
+// too, between finalize kernels.
 //
-// Such kernels move little data; their time is the launch and the chain of
+// Merged kernels move little data; their time is the launch and the chain of
 // dependent loads behind it (data another XCD has just written comes from
 // beyond the L2, about 0.7 us a step).  So each
 //   * resolves its predecessor's scalars itself (StageRun) instead of waiting
