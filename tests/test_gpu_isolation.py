@@ -44,7 +44,7 @@ def _equal(r, a):
         r["nOuter"] == a["nOuter"]
 
 
-def _check_batch(ctx, precond, precision):
+def _check_batch(ctx, precond, precision, tets=False):
     # the first member's load overflows the sums of its first PCG iteration; then
     # it has none: its PCG never runs, and its vectors keep what the first solve left
     from solids4foam_amd.batch import Batch
@@ -52,6 +52,9 @@ def _check_batch(ctx, precond, precision):
     opts = dict(CAPPED, precision=precision, preconditioner=precond, pcgMaxIter=40)
     first, _ = _box(ctx, (12, 11, 10), 1, traction=(1e250, 1e250, 1e250))
     others = [_box(ctx, n, 2 + i)[0] for i, n in enumerate(SIZES)]
+    if tets:  # no single slot count: the sequences with finalize kernels
+        from solids4foam_amd import cases
+        others.append(cases.tet_inclusions(ctx, n=4, seed=3)[1])
     alone = [m.solve(**opts) for m in others]
     b = Batch(ctx)
     for m in [first] + others:
@@ -126,3 +129,9 @@ def test_batch_turns_merged(ctx, precond):
     for i, (r, a) in enumerate(zip(got, alone)):
         assert r["nOuter"] == 40 and _equal(r, a), i
     b.close()
+
+
+@pytest.mark.parametrize("tets", [False, True])
+@pytest.mark.parametrize("precond", [0, 2, 3])
+def test_batch_sequences(ctx, precond, tets):
+    _check_batch(ctx, precond, 0, tets)
